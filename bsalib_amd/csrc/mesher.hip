@@ -29,8 +29,8 @@
 //
 // Each tile's BFM points are evaluated by k_bfm_batch (FP64 MFMA, S(f1+f2)
 // evaluated exactly, the semantics of getFM_full_tnm_scalar_msh_,
-// functionsImpl.F90:247-465); k_msh_integrate interpolates, applies the FRF
-// and the trapezoid weights and adds into m3mf, m3mr.
+// functionsImpl.F90:247-465); k_msh_quad (k_msh_integrate for ONLY_DIAG) interpolates,
+// applies the FRF and the trapezoid weights and adds into m3mf, m3mr.
 
 // ---------------------------------------------------------------------------
 // V table for point evaluation: V[(u*K + k)*NMP + y] = A(y, k; |f_u|), zero for
@@ -198,8 +198,8 @@ __device__ __forceinline__ void msh_entry(int e, int nm, int diag, int &m, int &
 // ---------------------------------------------------------------------------
 // The post-mesh of many tiles in one launch each (bsahip_mesher_run):
 // k_frf_segs fills the FRF tables of every tile, k_msh_copy_pts places the
-// resident level-0 BFM into the fine grids of refined tiles, k_msh_integrate
-// runs the quadrature over a list of (tile, cell range) items.
+// resident level-0 BFM into the fine grids of refined tiles, k_msh_quad /
+// k_msh_integrate runs the quadrature over a list of (tile, cell range) items.
 // ---------------------------------------------------------------------------
 // FRF segment s: n points f0 + i h, out H[off + i*nm + m]; segment of thread t
 // by binary search over the entry offsets eoff (n*nm per segment).
@@ -249,7 +249,8 @@ struct MshTileRun {
    long ldq;
    long h1, h2, h3;            // FRF table offsets (h3 < 0: f1 + f2 evaluated here)
    int nm, nb1, nb2, s1, s2;
-   double f3a, dh1, dh2, ws;
+   double f1a, f2a, f3a, dh1, dh2, ws;
+   double wf;                  // weight of the force sums
 };
 
 // Tile quadrature: bilinear BFM on the BRM grid, exact FRF, trapezoid
@@ -311,111 +312,247 @@ __global__ __launch_bounds__(256) void k_msh_integrate(
          }
       }
    }
-   atomicAdd(T.m3f + mnp, sf * T.ws);
+   atomicAdd(T.m3f + mnp, sf * T.wf);
    atomicAdd(T.m3r + mnp, sr * T.ws);
 }
 
-// The same quadrature for the full model (nm^3 entries), one thread per
-// (m, p) and MSH_NQ consecutive n: Re[H_m(f1) H_n(f2) H_p*(f1+f2)] is
-// Re[H_n(f2) Q] with Q = H_m(f1) conj H_p(f1+f2) shared by the thread's n, and
-// the sum over a BRM row (fixed b) is taken on Q before the H_n(f2) factor:
-//   sum_a w_a w_b B Re[H_n Q] = w_b Re[H_n sum_a w_a B Q].
-// Along the row B is linear in t = (a - a0) / s1, B = (1 - t) e0 + t e1 with
-// e0, e1 per n, so sum_a w_a B Q = e0 sum_a w_a (1 - t) Q + e1 sum_a w_a t Q:
-// the point loop forms the two n-independent sums, each n uses them once per
-// row.  grid (nitems * bx), bx covering nm^2 ceil(nm / MSH_NQ) threads of the
-// item's structure, block 256.
-#ifndef MSH_NQ
-#define MSH_NQ 8
-#endif
+// The same quadrature for the full model (nm^3 entries) as two chained products
+// on FP64 MFMA (v_mfma_f64_16x16x4f64).  With t, s the position of a BRM point
+// within its BFM cell along f1 and f2, the BFM of a cell is
+// sum_{k,l in {0,1}} B_kl T_k(t) S_l(s), T_0 = 1 - t, T_1 = t, and
+//   sum_points w B Re[H_m(f1) H_n(f2) conj H_p(f1+f2)] = sum_kl B_kl(m,n,p) R_kl(m,n,p),
+//   A_k(m,p; b) = sum_a w_a T_k H_m(f1_a) conj H_p(f1_a + f2_b)          (stage 1)
+//   R_kl(m,n,p) = Re sum_b w_b S_l H_n(f2_b) A_k(m,p; b)                 (stage 2)
+// The BFM itself enters once per cell and corner.  What bounds it: stage 1, 8
+// FP64 multiply-adds per (m, p) and point, on the matrix cores; one wave takes
+// 16 (row b, mode p) columns, so H_p(f1+f2) is evaluated once per column and
+// point in the lane that feeds it to the MFMA (no table, no division per
+// (m, p)), and the 16 rows of an MFMA tile are 4 modes m x {A_0, A_1} x
+// {re, im} with the imaginary operand as the second half of the contraction,
+// so no accumulator needs another lane's.  One thread per (m, p) and eight n
+// (the form this replaces) was bound by its two 16-byte table loads, or the
+// division, per point: 125.4 ms, now 10.7 ms, for the rule-based levels of a
+// 200-node deck (10 modes, 1764 tiles, 1.07e8 BRM points).
+// blockIdx.y: the modes p0 .. p0 + pc - 1, pc at most `pcmax`; item q covers
+// the cells [c0, c1) of tile it[q].tile, cell c = cj + ci * nc2, and of a single
+// cell the owned rows [r0, r1).
+// The p chunks fill the 16 columns: a chunk of pc modes takes 16 / pc rows per wave
+// and pass (10 modes as 8 + 2: 0.625 passes per row against 1 for one chunk of 10).
+struct MshItem {
+   int tile, c0, c1, r0, r1;     // r1 < 0: every owned row of the cells
+};
 
-__global__ __launch_bounds__(256) void k_msh_integrate_full(
-   const MshTileRun *__restrict__ tr, const int *__restrict__ it, const int2 *__restrict__ cr,
-   int bx, const double2 *__restrict__ H)
+// Launch shape (msh_shape): modes p per chunk, rows per wave and pass at most, BRM
+// points per staged chunk of L, LDS row strides (16 doubles mod 32, so that the two
+// contraction rows of a half wave fall on different banks) and sizes in doubles.
+struct MshShape {
+   int pcmax, rcap, ac, ldl, ldv, as, vs;
+};
+
+__host__ __device__ inline int msh_odd16(int n16) { return 16 * (n16 | 1); }
+
+// 1 / (K - w^2 M + i w C)
+__device__ __forceinline__ double2 msh_frf(double w, double M, double K, double C)
 {
-   const long q = blockIdx.x / bx;
-   const MshTileRun T = tr[it[q]];
-   const int nm = T.nm;
-   const int nm2 = nm * nm, nm3 = nm2 * nm;
-   const int nthr = nm2 * ((nm + MSH_NQ - 1) / MSH_NQ);
-   const int th = (int)(blockIdx.x % bx) * blockDim.x + threadIdx.x;
-   if (th >= nthr) return;
-   const int m = th % nm, p = (th / nm) % nm, n0 = (th / nm2) * MSH_NQ;
-   const int nn = min(MSH_NQ, nm - n0);
-   const int c0 = cr[q].x, c1 = cr[q].y;
+   const double r = K - w * w * M, im = w * C;
+   const double inv = 1.0 / (r * r + im * im);
+   return make_double2(r * inv, -im * inv);
+}
+
+template <int RT, int RT2, int CPW, int NW>
+__global__ __launch_bounds__(NW * 64) void k_msh_quad(const MshTileRun *__restrict__ tr,
+                                                      const MshItem *__restrict__ items,
+                                                      MshShape sh)
+{
+   extern __shared__ double smq[];
+   const MshItem q = items[blockIdx.x];
+   const MshTileRun T = tr[q.tile];
+   const int nm = T.nm, nm2 = nm * nm;
+   const int p0 = blockIdx.y * sh.pcmax;
+   if (p0 >= nm) return;                                   // uniform: a structure of fewer modes
+   const int pc = min(sh.pcmax, nm - p0);
+   const int rpw = min(16 / pc, sh.rcap);                  // BRM rows per wave and stage-1 pass
+   const int RB = NW * rpw;
+   const int ncol = 2 * nm * pc, nct = (ncol + 15) / 16, lda = msh_odd16(nct);
+   double *L = smq;                                        // [a][4 m + quantity], see below
+   double *As = L + (size_t)sh.ac * sh.ldl;                // [2 row + re/im][(k nm + m) pc + p]
+   double *Vs = As + sh.as;                                // [2 row + re/im][l nm + n]
+   double *accr = Vs + sh.vs;                              // [p][n][m] response sums
+   double *accf = accr + (size_t)nm2 * sh.pcmax;           // force sums
+   const int tid = threadIdx.x, lane = tid & 63;
+   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int lr = lane & 15, lk = lane >> 4;
+   constexpr int NT = NW * 64;
+   constexpr double TWO_PI = 2.0 * M_PI;
+
+   for (int t = tid; t < nm2 * pc; t += NT) accr[t] = accf[t] = 0.0;
+
+   // stage-1 column of this lane: (row bsub of the wave's rows, mode p0 + pl)
+   const int bsub = min(lr / pc, rpw - 1), pl = lr % pc;
+   const bool colok = lr < rpw * pc;
+   const double Mp = T.Mm[p0 + pl], Kp = T.Km[p0 + pl], Cp = T.Cm[p0 + pl];
+   // stage-1 row of this lane in tile rt: mode 4 rt + lr % 4, quantity lr / 4 of
+   // {A_0 re, A_0 im, A_1 re, A_1 im}; first half of the contraction L * Re H_p
+   // with that quantity of L, second half L * Im H_p with its partner, signed
+   const int qa = lr >> 2, ml = lr & 3;
+   const int o1 = ml * 4 + qa, o2 = ml * 4 + (qa ^ 1);
+   const double sg2 = (qa & 1) ? -1.0 : 1.0;
+
    const int nc1 = T.nb1 - 1, nc2 = T.nb2 - 1;
    const int NA = nc1 * T.s1, NB = nc2 * T.s2;
-   const double Mp = T.Mm[p], Kp = T.Km[p], Cp = T.Cm[p];
    const double inv1 = 1.0 / T.s1, inv2 = 1.0 / T.s2;
-   const double2 *H1 = H + T.h1, *H2 = H + T.h2, *H3 = T.h3 >= 0 ? H + T.h3 : nullptr;
-   int e[MSH_NQ];
+   int lci = -1;                                           // cell column whose L is staged
+
+   d4 acc2[RT2][CPW];
+   for (int c = q.c0; c < q.c1; ++c) {
+      const int ci = c / nc2, cj = c % nc2;
+      const int na = (ci == nc1 - 1) ? T.s1 + 1 : T.s1;    // owned BRM points per axis
+      const int nb = (cj == nc2 - 1) ? T.s2 + 1 : T.s2;
+      const int r0 = q.r1 < 0 ? 0 : q.r0, r1 = q.r1 < 0 ? nb : q.r1;
 #pragma unroll
-   for (int j = 0; j < MSH_NQ; ++j) e[j] = m + min(n0 + j, nm - 1) * nm + p * nm2;
-   double sf[MSH_NQ], sr[MSH_NQ];
+      for (int i = 0; i < RT2; ++i)
 #pragma unroll
-   for (int j = 0; j < MSH_NQ; ++j) sf[j] = sr[j] = 0.0;
-   for (int c = c0; c < c1; ++c) {
-      const int ci = c % nc1, cj = c / nc1;
-      const size_t q00 = (size_t)ci + (size_t)cj * T.ldq;
-      double b00[MSH_NQ], b10[MSH_NQ], b01[MSH_NQ], b11[MSH_NQ];
-#pragma unroll
-      for (int j = 0; j < MSH_NQ; ++j) {
-         b00[j] = T.bf[q00 * nm3 + e[j]];
-         b10[j] = T.bf[(q00 + 1) * nm3 + e[j]];
-         b01[j] = T.bf[(q00 + T.ldq) * nm3 + e[j]];
-         b11[j] = T.bf[(q00 + T.ldq + 1) * nm3 + e[j]];
-      }
-      const int ea = (ci == nc1 - 1) ? T.s1 : T.s1 - 1;   // owned BRM points per axis
-      const int eb = (cj == nc2 - 1) ? T.s2 : T.s2 - 1;
-      for (int bb = 0; bb <= eb; ++bb) {
-         const int b = cj * T.s2 + bb;
-         const double wb = (b == 0 || b == NB) ? 0.5 : 1.0;
-         const double sv = bb * inv2;
-         // along the row the BFM is e0 + t (e1 - e0): the sums over a of
-         // w_a (1 - t) Q and w_a t Q do not depend on n, so they are taken
-         // once per point and combined with each n's e0, e1 once per row
-         double W0 = 0.0, W1 = 0.0, A0r = 0.0, A0i = 0.0, A1r = 0.0, A1i = 0.0;
-         for (int aa = 0; aa <= ea; ++aa) {
-            const int a = ci * T.s1 + aa;
-            const double wa = (a == 0 || a == NA) ? 0.5 : 1.0;
-            const double t = aa * inv1;
-            const double2 h1v = H1[(size_t)a * nm + m];
-            double2 h3v;
-            if (H3) {
-               h3v = H3[(size_t)(a + b) * nm + p];
-            } else {
-               const double w3 = 2.0 * M_PI * (T.f3a + a * T.dh1 + b * T.dh2);
-               const double r = Kp - w3 * w3 * Mp, im = w3 * Cp, d = r * r + im * im;
-               h3v = make_double2(r / d, -im / d);
+         for (int j = 0; j < CPW; ++j) acc2[i][j] = (d4){0.0, 0.0, 0.0, 0.0};
+      for (int rb = r0; rb < r1; rb += RB) {
+         // stage 2's left operand: w_b S_l(b) {Re, -Im} H_n(f2_b), zero beyond the rows
+         for (int t = tid; t < RB * 16 * RT2; t += NT) {
+            const int row = t / (16 * RT2), r2 = t % (16 * RT2);
+            const int bb = rb + row, l = r2 >= nm ? 1 : 0, n = r2 - l * nm;
+            double vr = 0.0, vi = 0.0;
+            if (bb < r1 && n < nm) {
+               const int b = cj * T.s2 + bb;
+               const double s = bb * inv2;
+               const double wt = ((b == 0 || b == NB) ? 0.5 : 1.0) * (l ? s : 1.0 - s);
+               const double2 h = msh_frf(TWO_PI * (T.f2a + (double)b * T.dh2), T.Mm[n], T.Km[n], T.Cm[n]);
+               vr = wt * h.x;
+               vi = -wt * h.y;
             }
-            // Q = h1 conj(h3)
-            const double Qr = h1v.x * h3v.x + h1v.y * h3v.y;
-            const double Qi = h1v.y * h3v.x - h1v.x * h3v.y;
-            const double w0 = wa * (1.0 - t), w1 = wa * t;
-            W0 += w0;
-            W1 += w1;
-            A0r += w0 * Qr;
-            A0i += w0 * Qi;
-            A1r += w1 * Qr;
-            A1i += w1 * Qi;
+            Vs[(2 * row) * sh.ldv + r2] = vr;
+            Vs[(2 * row + 1) * sh.ldv + r2] = vi;
          }
+         d4 acc[RT];
 #pragma unroll
-         for (int j = 0; j < MSH_NQ; ++j) {
-            const double e0 = (1.0 - sv) * b00[j] + sv * b01[j];
-            const double e1 = (1.0 - sv) * b10[j] + sv * b11[j];
-            const double Dr = e0 * A0r + e1 * A1r, Di = e0 * A0i + e1 * A1i;
-            const double2 h2v = H2[(size_t)b * nm + min(n0 + j, nm - 1)];
-            sf[j] += wb * (e0 * W0 + e1 * W1);
-            sr[j] += wb * (h2v.x * Dr - h2v.y * Di);
+         for (int r = 0; r < RT; ++r) acc[r] = (d4){0.0, 0.0, 0.0, 0.0};
+         const int bb = min(rb + w * rpw + bsub, r1 - 1);
+         const double f3b = T.f3a + (double)(cj * T.s2 + bb) * T.dh2;
+         for (int a0 = 0; a0 < na; a0 += sh.ac) {
+            const int an = min(sh.ac, na - a0), as = (an + 3) & ~3;
+            if (lci != ci || na > sh.ac) {
+               __syncthreads();                            // the previous chunk is consumed
+               for (int t = tid; t < as * RT * 4; t += NT) {
+                  const int aa = t / (RT * 4), m = t % (RT * 4);
+                  double l0r = 0.0, l0i = 0.0, l1r = 0.0, l1i = 0.0;
+                  if (aa < an && m < nm) {
+                     const int a = ci * T.s1 + a0 + aa;
+                     const double x = (a0 + aa) * inv1;
+                     const double wa = (a == 0 || a == NA) ? 0.5 : 1.0;
+                     const double2 h = msh_frf(TWO_PI * (T.f1a + (double)a * T.dh1), T.Mm[m], T.Km[m], T.Cm[m]);
+                     const double w0 = wa * (1.0 - x), w1 = wa * x;
+                     l0r = w0 * h.x;
+                     l0i = w0 * h.y;
+                     l1r = w1 * h.x;
+                     l1i = w1 * h.y;
+                  }
+                  double *d = L + (size_t)aa * sh.ldl + m * 4;
+                  d[0] = l0r;
+                  d[1] = l0i;
+                  d[2] = l1r;
+                  d[3] = l1i;
+               }
+               lci = ci;
+            }
+            __syncthreads();
+            const double *Lp = L + (size_t)lk * sh.ldl;
+            for (int st = 0; st < as; st += 4) {
+               const double a = (double)(ci * T.s1 + a0 + min(st + lk, an - 1));
+               const double2 h = msh_frf(TWO_PI * (f3b + a * T.dh1), Mp, Kp, Cp);
+               double x1[RT], x2[RT];
+#pragma unroll
+               for (int r = 0; r < RT; ++r) {
+                  x1[r] = Lp[r * 16 + o1];
+                  x2[r] = sg2 * Lp[r * 16 + o2];
+               }
+#pragma unroll
+               for (int r = 0; r < RT; ++r)
+                  acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1[r], h.x, acc[r], 0, 0, 0);
+#pragma unroll
+               for (int r = 0; r < RT; ++r)
+                  acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x2[r], h.y, acc[r], 0, 0, 0);
+               Lp += 4 * sh.ldl;
+            }
          }
+         // A_k(m, p; b) to LDS: accumulator register t of a lane holds quantity t of
+         // mode 4 rt + lane / 16
+         if (colok) {
+            const int row = w * rpw + bsub;
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+               const int m = 4 * r + lk;
+               if (m < nm) {
+                  double *d = As + (size_t)(2 * row) * lda + m * pc + pl;
+                  d[0] = acc[r][0];
+                  d[lda] = acc[r][1];
+                  d[nm * pc] = acc[r][2];
+                  d[lda + nm * pc] = acc[r][3];
+               }
+            }
+         }
+         __syncthreads();
+         const int kn = 2 * min(RB, r1 - rb);              // rows beyond: Vs is zero
+         for (int k = 0; k < kn; k += 4) {
+            double v[RT2];
+#pragma unroll
+            for (int i = 0; i < RT2; ++i) v[i] = Vs[(size_t)(k + lk) * sh.ldv + i * 16 + lr];
+#pragma unroll
+            for (int j = 0; j < CPW; ++j) {
+               const int ct = w + NW * j;
+               if (ct < nct) {                          // uniform per wave
+                  const double x = As[(size_t)(k + lk) * lda + ct * 16 + lr];
+#pragma unroll
+                  for (int i = 0; i < RT2; ++i)
+                     acc2[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[i], x, acc2[i][j], 0, 0, 0);
+               }
+            }
+         }
+         __syncthreads();                                  // As, Vs are consumed
+      }
+      // sums over the rows of w_b S_l and over the cell's points of w_a T_k (force;
+      // half weights at the tile's edges)
+      const double ss = inv2 * 0.5 * (double)(r1 - r0) * (double)(r0 + r1 - 1);
+      const double sb0 = (double)(r1 - r0) - ss - (cj == 0 && r0 == 0 ? 0.5 : 0.0);
+      const double sb1 = ss - (cj == nc2 - 1 && r1 == T.s2 + 1 ? 0.5 : 0.0);
+      const double sa0 = 0.5 * (T.s1 + 1) - (ci == 0 ? 0.5 : 0.0);
+      const double sa1 = 0.5 * (T.s1 - 1) + (ci == nc1 - 1 ? 0.5 : 0.0);
+      const double *B = T.bf + ((size_t)ci + (size_t)cj * T.ldq) * (size_t)(nm2 * nm);
+      int pcv = pc, nmv = nm;
+      asm volatile("" : "+s"(pcv), "+s"(nmv));      // the indexes below are formed per cell, not kept in registers
+#pragma unroll
+      for (int j = 0; j < CPW; ++j) {
+         const int col = (w + NW * j) * 16 + lr;
+         if (col >= ncol) continue;
+         const int k = col >= nm * pcv ? 1 : 0, mp = col - k * nm * pcv;
+         const int m = mp / pcv, p = mp % pcv;
+#pragma unroll
+         for (int i = 0; i < RT2; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+               const int r2 = i * 16 + lk + 4 * t;
+               if (r2 < 2 * nmv) {
+                  const int l = r2 >= nmv ? 1 : 0, n = r2 - l * nmv;
+                  const double bv = B[((size_t)k + (l ? (size_t)T.ldq : 0)) * (size_t)(nm2 * nm) +
+                                      m + n * nmv + (p0 + p) * nm2];
+                  const int e = (p * nmv + n) * nmv + m;
+                  atomicAdd(accr + e, acc2[i][j][t] * bv);
+                  atomicAdd(accf + e, (k ? sa1 : sa0) * (l ? sb1 : sb0) * bv);
+               }
+            }
       }
    }
-#pragma unroll
-   for (int j = 0; j < MSH_NQ; ++j)
-      if (j < nn) {
-         atomicAdd(T.m3f + e[j], sf[j] * T.ws);
-         atomicAdd(T.m3r + e[j], sr[j] * T.ws);
-      }
+   __syncthreads();
+   for (int t = tid; t < nm2 * pc; t += NT) {
+      atomicAdd(T.m3f + (size_t)p0 * nm2 + t, accf[t] * T.wf);
+      atomicAdd(T.m3r + (size_t)p0 * nm2 + t, accr[t] * T.ws);
+   }
 }
 
 // ---------------------------------------------------------------------------
@@ -921,31 +1058,89 @@ struct MshJob {
    long brm = 0;                  // BRM points integrated
 };
 
+// Launch shape of k_msh_quad for nm modes (NW waves): the chunk of modes p that
+// needs the fewest stage-1 passes per row (sum over the chunks of one over the rows a
+// wave takes, plus 3 % per chunk for its own operands), among those whose buffers fit
+// the LDS of a workgroup.
+size_t msh_shape(int nm, int RT, int RT2, int CPW, int NW, MshShape &S)
+{
+   S.ac = nm <= 4 ? 128 : (nm <= 16 ? 64 : 32);
+   S.rcap = nm <= 8 ? 8 : (nm <= 24 ? 4 : 2);
+   S.ldl = msh_odd16(RT);
+   S.ldv = msh_odd16(RT2);
+   size_t best = 0;
+   double cbest = 1e300;
+   const int pmax = std::min({nm, nm <= 8 ? 16 : (nm <= 16 ? 8 : 4), CPW * NW * 8 / nm});
+   for (int pc = 1; pc <= pmax; ++pc) {
+      double c = 0.0;
+      int as = 0, vs = 0;
+      for (int p0 = 0; p0 < nm; p0 += pc) {
+         const int k = std::min(pc, nm - p0), rpw = std::min(16 / k, S.rcap), rows = 2 * NW * rpw;
+         c += 1.0 / rpw + 0.03;
+         as = std::max(as, rows * msh_odd16((2 * nm * k + 15) / 16));
+         vs = std::max(vs, rows * S.ldv);
+      }
+      const size_t lds = sizeof(double) * ((size_t)S.ac * S.ldl + as + vs + 2 * (size_t)nm * nm * pc);
+      if (lds > 160 * 1024 || c >= cbest) continue;
+      cbest = c;
+      best = lds;
+      S.pcmax = pc;
+      S.as = as;
+      S.vs = vs;
+   }
+   return best;
+}
+
+template <int RT, int RT2, int CPW, int NW>
+int msh_quad_launch(int nm, size_t nitems, const MshTileRun *tr, const MshItem *items)
+{
+   MshShape S{};
+   const size_t lds = msh_shape(nm, RT, RT2, CPW, NW, S);
+   if (lds == 0) return fail(BSAHIP_EUNSUPPORTED, "the Mesher supports at most 32 modes");
+   HIPC(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_msh_quad<RT, RT2, CPW, NW>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+   const dim3 gr((unsigned)nitems, (unsigned)((nm + S.pcmax - 1) / S.pcmax));
+   k_msh_quad<RT, RT2, CPW, NW><<<gr, NW * 64, lds, g.s>>>(tr, items, S);
+   HIPC(hipGetLastError());
+   return 0;
+}
+
+// Template by modes: RT tiles of 4 modes m, RT2 tiles of the 2 nm (l, n) rows, CPW
+// column tiles per wave of the 2 nm pc (k, m, p) columns.
+int msh_quad(int nm, size_t nitems, const MshTileRun *tr, const MshItem *items)
+{
+   if (nm <= 4) return msh_quad_launch<1, 1, 1, 8>(nm, nitems, tr, items);
+   if (nm <= 8) return msh_quad_launch<2, 1, 1, 8>(nm, nitems, tr, items);
+   if (nm <= 12) return msh_quad_launch<3, 2, 3, 4>(nm, nitems, tr, items);
+   if (nm <= 16) return msh_quad_launch<4, 2, 4, 4>(nm, nitems, tr, items);
+   if (nm <= 24) return msh_quad_launch<6, 3, 3, 4>(nm, nitems, tr, items);
+   return msh_quad_launch<8, 4, 4, 4>(nm, nitems, tr, items);
+}
+
 // The quadrature of the visited tiles of one or more structures (all of the
-// full model, or all ONLY_DIAG) in two launches: FRF tables of every tile
-// (k_frf_segs), then k_msh_integrate_full / k_msh_integrate over (tile, cell
-// range) items.  Scratch buffers come from the first structure's buffers.
+// full model, or all ONLY_DIAG): k_msh_quad over (tile, cell range) items, one launch
+// per mode count, or (ONLY_DIAG) the FRF tables of every tile (k_frf_segs) and
+// k_msh_integrate.  Scratch buffers come from the first structure's buffers.
 int msh_integrate_jobs(const std::vector<MshJob *> &jobs)
 {
    size_t ntr = 0;
    for (MshJob *J : jobs) ntr += J->refs.size();
    if (ntr == 0) return 0;
    const bool diag = jobs[0]->M->diag;
-   int bx = 1;
    std::vector<MshSeg> seg;
    std::vector<long> eoff(1, 0);
    std::vector<MshTileRun> tr;
    std::vector<long> ncell_of;
    tr.reserve(ntr);
+   int bx = 1;
    long ncells = 0;
+   double cost = 0.0;                      // rows of BRM points, each weighed by its length
+   auto row_cost = [](const MshTileRun &T) { return T.s1 + 16.0; };
    for (MshJob *J : jobs) {
       bsahip_mesher *M = J->M;
       Prob &D = M->D;
       if (M->diag != diag) return fail(BSAHIP_EINVAL, "a Mesher batch mixes the ONLY_DIAG and full models");
-      // threads per item: one per entry (ONLY_DIAG), or one per (m, p) and
-      // MSH_NQ n (full model)
-      const int nthr = diag ? M->nc : D.nm * D.nm * ((D.nm + MSH_NQ - 1) / MSH_NQ);
-      bx = std::max(bx, (nthr + 255) / 256);
+      bx = std::max(bx, (M->nc + 255) / 256);
       auto add_seg = [&](double f0, double h, int n) -> long {
          const long off = eoff.back();
          seg.push_back(MshSeg{f0, h, off, D.Mm, D.Km, D.Cm, D.nm});
@@ -955,7 +1150,6 @@ int msh_integrate_jobs(const std::vector<MshJob *> &jobs)
       for (const MshRef &R : J->refs) {
          const MshTile &t = M->tiles[R.k];
          const MshBrmGrid G = msh_brm_grid(t, R.l);
-         const bool eq = std::fabs(G.h1 - G.h2) <= 1e-13 * std::max(std::fabs(G.h1), std::fabs(G.h2));
          MshTileRun T;
          T.bf = R.bf;
          T.m3f = J->m3f;
@@ -964,56 +1158,106 @@ int msh_integrate_jobs(const std::vector<MshJob *> &jobs)
          T.Km = D.Km;
          T.Cm = D.Cm;
          T.ldq = R.ldq;
-         T.h1 = add_seg(t.a1, G.h1, G.NA + 1);
-         T.h2 = add_seg(t.a2, G.h2, G.NB + 1);
-         T.h3 = eq ? add_seg(t.a1 + t.a2, G.h1, G.NA + G.NB + 1) : -1;
+         T.h1 = T.h2 = T.h3 = -1;
+         if (diag) {
+            const bool eq = std::fabs(G.h1 - G.h2) <= 1e-13 * std::max(std::fabs(G.h1), std::fabs(G.h2));
+            T.h1 = add_seg(t.a1, G.h1, G.NA + 1);
+            T.h2 = add_seg(t.a2, G.h2, G.NB + 1);
+            T.h3 = eq ? add_seg(t.a1 + t.a2, G.h1, G.NA + G.NB + 1) : -1;
+         }
          T.nm = D.nm;
          T.nb1 = R.nb1;
          T.nb2 = R.nb2;
          T.s1 = G.s1;
          T.s2 = G.s2;
+         T.f1a = t.a1;
+         T.f2a = t.a2;
          T.f3a = t.a1 + t.a2;
          T.dh1 = G.h1;
          T.dh2 = G.h2;
          T.ws = (2.0 * M_PI * G.h1) * (2.0 * M_PI * G.h2);
+         T.wf = T.ws;
          tr.push_back(T);
          ncell_of.push_back((long)(R.nb1 - 1) * (R.nb2 - 1));
          ncells += ncell_of.back();
+         cost += (double)ncell_of.back() * T.s2 * row_cost(T);
          J->brm += (long)(G.NA + 1) * (G.NB + 1);
       }
    }
-   // items: each tile's cells cut in ranges of at most `per` cells, so that
-   // the launch holds some 8192 (item, thread block) workgroups or more
-   const long per = std::max<long>(1, ncells * bx / 8192);
-   std::vector<int> it;
-   std::vector<int2> cr;
-   for (size_t r = 0; r < tr.size(); ++r)
-      for (long c0 = 0; c0 < ncell_of[r]; c0 += per) {
-         it.push_back((int)r);
-         cr.push_back(make_int2((int)c0, (int)std::min<long>(ncell_of[r], c0 + per)));
-      }
-   if ((long)it.size() * bx > 0x7fffffffL)
-      return fail(BSAHIP_EUNSUPPORTED, "Mesher post-mesh launch above 2^31 workgroups");
    Bufs &B = jobs[0]->M->B;
-   MshSeg *dseg;
-   long *doff;
-   double2 *H;
    MshTileRun *dtr;
-   int *dit;
-   int2 *dcr;
-   CHK(upload(B, "m_seg", seg, &dseg));
-   CHK(upload(B, "m_segoff", eoff, &doff));
-   CHK(B.get("m_H", (size_t)eoff.back(), &H));
-   CHK(upload(B, "m_tiles_run", tr, &dtr));
-   CHK(upload(B, "m_items", it, &dit));
-   CHK(upload(B, "m_ranges", cr, &dcr));
-   k_frf_segs<<<(unsigned)((eoff.back() + 255) / 256), 256, 0, g.s>>>(dseg, doff, (int)seg.size(), H);
-   HIPC(hipGetLastError());
-   if (diag)
+   if (diag) {
+      // items: each tile's cells cut in ranges of at most `per` cells, so that
+      // the launch holds some 8192 (item, thread block) workgroups or more
+      const long per = std::max<long>(1, ncells * bx / 8192);
+      std::vector<int> it;
+      std::vector<int2> cr;
+      for (size_t r = 0; r < tr.size(); ++r)
+         for (long c0 = 0; c0 < ncell_of[r]; c0 += per) {
+            it.push_back((int)r);
+            cr.push_back(make_int2((int)c0, (int)std::min<long>(ncell_of[r], c0 + per)));
+         }
+      if ((long)it.size() * bx > 0x7fffffffL)
+         return fail(BSAHIP_EUNSUPPORTED, "Mesher post-mesh launch above 2^31 workgroups");
+      MshSeg *dseg;
+      long *doff;
+      double2 *H;
+      int *dit;
+      int2 *dcr;
+      CHK(upload(B, "m_seg", seg, &dseg));
+      CHK(upload(B, "m_segoff", eoff, &doff));
+      CHK(B.get("m_H", (size_t)eoff.back(), &H));
+      CHK(upload(B, "m_tiles_run", tr, &dtr));
+      CHK(upload(B, "m_items", it, &dit));
+      CHK(upload(B, "m_ranges", cr, &dcr));
+      k_frf_segs<<<(unsigned)((eoff.back() + 255) / 256), 256, 0, g.s>>>(dseg, doff, (int)seg.size(), H);
+      HIPC(hipGetLastError());
       k_msh_integrate<<<(unsigned)(it.size() * bx), 256, 0, g.s>>>(dtr, dit, dcr, bx, 1, H);
-   else
-      k_msh_integrate_full<<<(unsigned)(it.size() * bx), 256, 0, g.s>>>(dtr, dit, dcr, bx, H);
-   HIPC(hipGetLastError());
+      HIPC(hipGetLastError());
+   } else {
+      // items of about equal cost, some 4096 of them: runs of cells of one tile, or,
+      // where one cell costs more, runs of that cell's rows; the launch of a mode
+      // count takes a contiguous range of the list
+      const double per = cost / 4096.0;
+      std::vector<int> nms;
+      for (const MshTileRun &T : tr) nms.push_back(T.nm);
+      std::sort(nms.begin(), nms.end());
+      nms.erase(std::unique(nms.begin(), nms.end()), nms.end());
+      std::vector<MshItem> it;
+      std::vector<size_t> first;
+      for (int nm : nms) {
+         first.push_back(it.size());
+         for (size_t r = 0; r < tr.size(); ++r) {
+            const MshTileRun &T = tr[r];
+            if (T.nm != nm) continue;
+            const int nc2 = T.nb2 - 1, nc = (int)ncell_of[r];
+            const double ccost = T.s2 * row_cost(T);
+            if (ccost <= per || T.s2 < 64) {
+               const int run = std::max(1, (int)std::min<double>(nc, per / ccost));
+               for (int c = 0; c < nc; c += run)
+                  it.push_back(MshItem{(int)r, c, std::min(nc, c + run), 0, -1});
+            } else {
+               const int run = std::max(64, (int)(per / row_cost(T)));
+               for (int c = 0; c < nc; ++c) {
+                  const int nb = (c % nc2 == nc2 - 1) ? T.s2 + 1 : T.s2;
+                  // an even cut: a last run of one row would cost a whole pass
+                  const int ns = std::max(1, nb / run);
+                  for (int k = 0; k < ns; ++k)
+                     it.push_back(MshItem{(int)r, c, c + 1, nb * k / ns, nb * (k + 1) / ns});
+               }
+            }
+         }
+      }
+      first.push_back(it.size());
+      if (it.size() > 0x7fffffUL)
+         return fail(BSAHIP_EUNSUPPORTED, "Mesher post-mesh launch above 2^23 workgroups");
+      MshItem *dit;
+      CHK(upload(B, "m_tiles_run", tr, &dtr));
+      CHK(upload(B, "m_qitems", it, &dit));
+      for (size_t k = 0; k < nms.size(); ++k)
+         if (first[k + 1] > first[k])
+            CHK(msh_quad(nms[k], first[k + 1] - first[k], dtr, dit + first[k]));
+   }
    for (MshJob *J : jobs) J->refs.clear();
    return 0;
 }
