@@ -240,6 +240,15 @@ __global__ void k_msh_copy_pts(const double *__restrict__ lv0, const long *__res
    fine[dst[q] * nm3 + e] = lv0[src[q] * nm3 + e];
 }
 
+// lv0[q][e] = lv0[npts - 1 - q][e] for the n points from q0 (a copy: HBM-bound)
+__global__ void k_msh_mirror(double *__restrict__ lv0, long q0, long n, long npts, int nc)
+{
+   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+   if (t >= n * nc) return;
+   const long q = q0 + t / nc, e = t % nc;
+   lv0[q * nc + e] = lv0[(npts - 1 - q) * nc + e];
+}
+
 // One tile of a batched post-mesh (tiles of several structures may share a
 // launch: the modal data and accumulators are per tile).
 struct MshTileRun {
@@ -858,6 +867,35 @@ void msh_tiles(const std::vector<MshAxisCell> &ax, const bsahip_mesher_cfg *cfg,
       }
 }
 
+// The tile that is the mirror image (-f1, -f2) of each tile, same cells and BRM grid,
+// or -1.  The spectra are even in f and Re[H_m(f1) H_n(f2) conj H_p(f1+f2)] is even
+// under (f1, f2) -> (-f1, -f2), so such a pair contributes twice one tile's moments:
+// a post-mesh evaluates and integrates one of the two (when their levels agree), to
+// the rounding of the mirrored frequencies.  Layouts whose intervals are cut unevenly
+// have tiles without an image; those are integrated alone.
+std::vector<long> msh_mirror(const std::vector<MshTile> &tiles)
+{
+   // tiles are the tensor product of the axis segments, f1 fastest
+   size_t ns = 0;
+   while (ns < tiles.size() && tiles[ns].a2 == tiles[0].a2) ++ns;
+   std::vector<long> seg(ns, -1), out(tiles.size(), -1);
+   const double eps = 1e-12 * std::max(std::fabs(tiles[0].a1), std::fabs(tiles[ns - 1].b1));
+   for (size_t i = 0; i < ns; ++i)
+      for (size_t j = 0; j < ns; ++j)
+         if (std::fabs(tiles[i].a1 + tiles[j].b1) <= eps && std::fabs(tiles[i].b1 + tiles[j].a1) <= eps &&
+             tiles[i].n1 == tiles[j].n1) {
+            seg[i] = (long)j;
+            break;
+         }
+   for (size_t k = 0; k < tiles.size(); ++k) {
+      const long i = seg[k % ns], j = seg[k / ns];
+      if (i < 0 || j < 0) continue;
+      const MshTile &m = tiles[(size_t)j * ns + i];
+      if (m.sub1 == tiles[k].sub1 && m.sub2 == tiles[k].sub2) out[k] = j * (long)ns + i;
+   }
+   return out;
+}
+
 // Level-0 nodes of the whole axis (the tiles' level-0 grids are sub-grids of
 // the tensor product of these nodes).
 std::vector<double> msh_axis_nodes(const std::vector<MshTile> &tiles)
@@ -879,6 +917,7 @@ struct bsahip_mesher {
    Prob D;
    int nmp = 0;
    std::vector<MshTile> tiles;
+   std::vector<long> mirror;  // the tile at (-f1, -f2), -1: none (msh_mirror)
    double dfref = 0.0;
    int nc = 0;                // bispectrum entries per point: NM^3, or NM (ONLY_DIAG)
    bool diag = false;         // the ONLY_DIAG model
@@ -1046,6 +1085,7 @@ struct MshRef {
    int l, nb1, nb2;
    const double *bf;
    long ldq;
+   bool twice;      // stands for its mirror image too
 };
 
 // The visited tiles of one structure awaiting their quadrature: its m3f
@@ -1055,7 +1095,8 @@ struct MshJob {
    std::vector<MshRef> refs;
    double *m3f = nullptr;
    std::function<double *(size_t)> m3r_of;
-   long brm = 0;                  // BRM points integrated
+   bool per_tile = false;         // m3r_of is the tile's own slot: its image's is a copy
+   long brm = 0;                  // BRM points integrated, mirror images included
 };
 
 // Launch shape of k_msh_quad for nm modes (NW waves): the chunk of modes p that
@@ -1176,12 +1217,13 @@ int msh_integrate_jobs(const std::vector<MshJob *> &jobs)
          T.dh1 = G.h1;
          T.dh2 = G.h2;
          T.ws = (2.0 * M_PI * G.h1) * (2.0 * M_PI * G.h2);
-         T.wf = T.ws;
+         T.wf = R.twice ? 2.0 * T.ws : T.ws;
+         if (!J->per_tile) T.ws = T.wf;
          tr.push_back(T);
          ncell_of.push_back((long)(R.nb1 - 1) * (R.nb2 - 1));
          ncells += ncell_of.back();
          cost += (double)ncell_of.back() * T.s2 * row_cost(T);
-         J->brm += (long)(G.NA + 1) * (G.NB + 1);
+         J->brm += (R.twice ? 2 : 1) * (long)(G.NA + 1) * (G.NB + 1);
       }
    }
    Bufs &B = jobs[0]->M->B;
@@ -1262,15 +1304,25 @@ int msh_integrate_jobs(const std::vector<MshJob *> &jobs)
    return 0;
 }
 
+// the mirror image of tile k that its visit stands for, or -1
+long msh_image(const bsahip_mesher *m, const int32_t *levels, size_t k)
+{
+   const long j = m->mirror[k];
+   if (j < 0 || j == (long)k) return -1;
+   const int lk = levels ? levels[k] : m->tiles[k].rule, lj = levels ? levels[j] : m->tiles[j].rule;
+   return lk == lj ? j : -1;
+}
+
 // Post-mesh traversal shared by the run and the export: level-1 tiles read the
 // resident level-0 BFM in place; refined tiles are evaluated in groups whose
 // fine grids fit the staging buffer.  `done(last)`, when given, is called once
 // the tiles visited so far may be consumed: after each group, before its
 // staging buffer is reused (last = false), and at the end (last = true; those
-// tiles stay valid until this Mesher's next post-mesh).  Returns the
-// refinement evaluations.
-int msh_post(bsahip_mesher *m, const int32_t *levels, const MshVisit &visit, long &evals_post,
-             const std::function<int(bool)> &done = nullptr)
+// tiles stay valid until this Mesher's next post-mesh).  `half`: of two mirrored
+// tiles at one level only the first is evaluated and visited (msh_image).  Returns
+// the refinement evaluations, those of the mirror images included.
+int msh_post(bsahip_mesher *m, const int32_t *levels, bool half, const MshVisit &visit,
+             long &evals_post, const std::function<int(bool)> &done = nullptr)
 {
    const size_t nm3 = (size_t)m->nc, nt = m->tiles.size();
    const size_t cap = std::max<size_t>(66049, ((size_t)1 << 29) / nm3);   // points (4 GiB)
@@ -1329,6 +1381,13 @@ int msh_post(bsahip_mesher *m, const int32_t *levels, const MshVisit &visit, lon
    for (size_t i = 0; i < nt; ++i) {
       const MshTile &t = m->tiles[i];
       const int l = levels ? levels[i] : t.rule;
+      if (half) {
+         const long j = msh_image(m, levels, i);
+         if (j >= 0 && j < (long)i) {
+            evals_post += (long)(t.n1 * l + 1) * (t.n2 * l + 1) - (long)(t.n1 + 1) * (t.n2 + 1);
+            continue;
+         }
+      }
       if (l == 1) {
          CHK(visit(i, t, 1, m->lv0 + msh_lv0_at(m, t) * nm3, m->nx, t.n1 + 1, t.n2 + 1));
          continue;
@@ -1388,6 +1447,7 @@ int msh_setup(const bsahip_problem *p, const bsahip_mesher_cfg *cfg, int32_t fla
    std::vector<MshAxisCell> ax;
    CHK(msh_full_axis(cfg, D.nm, ax, M->dfref));
    msh_tiles(ax, cfg, D.nm, M->dfref, M->tiles);
+   M->mirror = msh_mirror(M->tiles);
    CHK(M->B.get("m_PB", (size_t)D.K * M->nmp, &M->PB));
    k_pbt<<<(unsigned)((D.K * M->nmp + 255) / 256), 256, 0, g.s>>>(D.pb_k, D.nm, D.K, M->nmp, M->PB);
    HIPC(hipGetLastError());
@@ -1431,17 +1491,33 @@ int bsahip_mesher_create(const bsahip_problem *p, const bsahip_mesher_cfg *cfg, 
    std::vector<double> x;
    CHK(msh_setup(p, cfg, flags, M, x));
    // pre-mesh: the level-0 BFM on the global grid (every tile's level-0 points
-   // once, shared edges and corners included once), kept resident
-   const size_t npts = x.size() * x.size();
-   std::vector<double> f1, f2;
-   std::vector<long> slot;
-   for (size_t j = 0; j < x.size(); ++j)
-      for (size_t i = 0; i < x.size(); ++i) {
-         f1.push_back(x[i]);
-         f2.push_back(x[j]);
-         slot.push_back((long)(i + j * x.size()));
-      }
+   // once, shared edges and corners included once), kept resident.  The BFM is even
+   // under (f1, f2) -> (-f1, -f2): on an axis that is its own mirror image one of
+   // two mirrored points is evaluated and the other copied
+   const size_t nx = x.size(), npts = nx * nx;
+   bool even = true;
+   for (size_t i = 0; i < nx; ++i)
+      even = even && std::fabs(x[i] + x[nx - 1 - i]) <= 1e-12 * std::fabs(x[nx - 1]);
+   const size_t neval = even ? (npts + 1) / 2 : npts;
+   std::vector<double> f1(neval), f2(neval);
+   std::vector<long> slot(neval);
+   for (size_t q = 0; q < neval; ++q) {
+      f1[q] = x[q % nx];
+      f2[q] = x[q / nx];
+      slot[q] = (long)q;
+   }
    CHK(msh_eval(M.get(), f1, f2, slot, M->lv0));
+   if (neval < npts) {
+      // point q's mirror image is npts - 1 - q
+      const long n = (long)(npts - neval), nc = M->nc;
+      const long part = 0x7fffffL * 256 / nc;            // one launch's 2^32 threads
+      for (long q0 = 0; q0 < n; q0 += part) {
+         const long k = std::min(part, n - q0);
+         k_msh_mirror<<<(unsigned)((k * nc + 255) / 256), 256, 0, g.s>>>(M->lv0, (long)neval + q0, k,
+                                                                         (long)npts, (int)nc);
+      }
+      HIPC(hipGetLastError());
+   }
    HIPC(hipStreamSynchronize(g.s));
    M->evals_lv0 = (long)npts;
    *out = M.release();
@@ -1537,10 +1613,11 @@ int bsahip_mesher_run_tiles(bsahip_mesher *m, const int32_t *levels, double *til
    job.M = m;
    job.m3f = acc;
    job.m3r_of = [&](size_t k) { return tile_m3mr ? acc + 2 * nm3 + k * nm3 : acc + nm3; };
+   job.per_tile = tile_m3mr != nullptr;
    CHK(msh_post(
-      m, levels,
+      m, levels, true,
       [&](size_t k, const MshTile &, int l, const double *bf, long ldq, int nb1, int nb2) {
-         job.refs.push_back(MshRef{k, l, nb1, nb2, bf, ldq});
+         job.refs.push_back(MshRef{k, l, nb1, nb2, bf, ldq, msh_image(m, levels, k) >= 0});
          return 0;
       },
       evals_post, [&](bool) { return msh_integrate_jobs({&job}); }));
@@ -1556,6 +1633,9 @@ int bsahip_mesher_run_tiles(bsahip_mesher *m, const int32_t *levels, double *til
          // tile by tile, so that each pass reads one contiguous slot
          std::fill(m3mr, m3mr + nm3, 0.0);
          for (size_t k = 0; k < nt; ++k) {
+            const long j = msh_image(m, levels, k);      // an image: the slot of its first tile
+            if (j >= 0 && j < (long)k)
+               std::copy(tile_m3mr + j * nm3, tile_m3mr + (j + 1) * nm3, tile_m3mr + k * nm3);
             const double *c = tile_m3mr + k * nm3;
             for (size_t q = 0; q < nm3; ++q) m3mr[q] += c[q];
          }
@@ -1597,6 +1677,7 @@ int bsahip_mesher_run_batch(int32_t n, bsahip_mesher *const *ms, const int32_t *
       CHK(m->B.get("m_acc", 2 * nm3, &acc[i]));
       CHK(fill(acc[i], 2 * nm3, 0.0));
       MshJob &J = jobs[i];
+      const int32_t *lv = levels ? levels[i] : nullptr;
       J.M = m;
       J.m3f = acc[i];
       double *r = acc[i] + nm3;
@@ -1604,9 +1685,9 @@ int bsahip_mesher_run_batch(int32_t n, bsahip_mesher *const *ms, const int32_t *
       // each Mesher's last group of tiles waits for the shared launch below;
       // earlier groups (their staging buffer is reused) are integrated at once
       CHK(msh_post(
-         m, levels ? levels[i] : nullptr,
-         [&J](size_t k, const MshTile &, int l, const double *bf, long ldq, int nb1, int nb2) {
-            J.refs.push_back(MshRef{k, l, nb1, nb2, bf, ldq});
+         m, lv, true,
+         [&J, lv](size_t k, const MshTile &, int l, const double *bf, long ldq, int nb1, int nb2) {
+            J.refs.push_back(MshRef{k, l, nb1, nb2, bf, ldq, msh_image(J.M, lv, k) >= 0});
             return 0;
          },
          evals[i], [&J](bool last) { return last ? 0 : msh_integrate_jobs({&J}); }));
@@ -1795,7 +1876,7 @@ int bsahip_mesher_export(bsahip_mesher *m, const int32_t *levels, int32_t ncol, 
       CHK(upload(m->B, "m_xcoef", cc, &dcoef));
    }
    long evals = 0;
-   CHK(msh_post(m, levels,
+   CHK(msh_post(m, levels, false,
                 [&](size_t k, const MshTile &t, int l, const double *bf, long ldq, int nb1, int nb2) {
                    MshBrmGrid G = msh_brm_grid(t, l);
                    CHK(msh_frf_tables(m, t, G));

@@ -66,3 +66,32 @@ def test_long_cells_and_row_runs(gpu_lib, nm, rfmnt, tile, brm):
     M = _mesher(nm, rfmnt, tile, brm)
     _check(M, 1)
     M.close()
+
+
+@pytest.mark.parametrize("only_diag", [False, True])
+def test_mirrored_tiles_at_unequal_levels(gpu_lib, only_diag):
+    """Tiles (f1, f2) and (-f1, -f2) are integrated once when their levels agree: the
+    same levels on both, on one of them only, and a layout whose pre-peak gap is cut
+    unevenly (tiles without a mirror image) must all give the exported integrand's
+    sums, and the evaluation counts of every tile."""
+    p = synth.tower(nn=5, nm=2, comps=(1, 3), natf=np.array([0.4, 1.5]),
+                    xi=np.array([0.05, 0.04]), nfreqs=9, df=0.5, seed=4)
+    M = abi.Mesher(p, bkg_base_rfmnt=4, tile_cells=2, bkg_peakw=0.15, only_diag=only_diag)
+    geom, rule = M.tiles()
+    key = {tuple(np.round(g[:4], 9)): k for k, g in enumerate(geom)}
+    twin = [key.get(tuple(np.round([-g[1], -g[0], -g[3], -g[2]], 9)), -1) for g in geom]
+    assert any(t < 0 for t in twin) and any(t >= 0 and t != k for k, t in enumerate(twin))
+    rng = np.random.default_rng(0)
+    same = rng.choice([1, 2, 4], size=M.ntiles).astype(np.int32)
+    for k, t in enumerate(twin):
+        if t > k:
+            same[t] = same[k]
+    for lv in (np.ones(M.ntiles, np.int32), same,
+               rng.choice([1, 2, 4], size=M.ntiles).astype(np.int32)):
+        _check(M, lv)
+        n = (geom[:, 4] * lv + 1) * (geom[:, 5] * lv + 1) - (geom[:, 4] + 1) * (geom[:, 5] + 1)
+        r = M.run(levels=lv)
+        assert r["evals_post"] == int(n.sum())
+        assert r["brm_points"] == int(np.sum(np.prod(M.export(levels=lv)["dims"].astype(np.int64),
+                                                     axis=1)))
+    M.close()
