@@ -313,7 +313,6 @@ int set_pod(const bsahip_problem *p, Prob &D)
    return 0;
 }
 
-// A table on a list of |f| values (device array fl): U[K][ldU], rows y*rows_per_mode + q.
 #define BLASC(x)                                                                             \
    do {                                                                                      \
       rocblas_status st_ = (x);                                                              \
@@ -398,32 +397,91 @@ int pod_project(Bufs &B, const Prob &D, const double *sq, const double *fl, int 
    return 0;
 }
 
-int build_table(Bufs &B, const Prob &D, const double *fl, int nfl, int rows_per_mode, double *U,
-                long ldU)
+// Neighbouring frequencies per wave of k_project: 8 (64-byte stores, loads of ln rho
+// and Psi_a shared by eight) while that still leaves 2 waves per SIMD of the chip, fewer
+// for small tables, where latency counts; at most 4 beyond 16 modes (accumulators).
+int project_group(long ncoltile, int nfl, int planes, int mt)
 {
-   if (nfl > 65535) return fail(BSAHIP_EUNSUPPORTED, "more than 65535 distinct frequencies in one table");
-   double *sq;
-   CHK(B.get("sq", (size_t)D.ntc * nfl * D.nnl, &sq));
-   CHK(fill(U, (size_t)D.K * ldU, 0.0));
-   dim3 gp((D.nnl + 63) / 64, nfl, D.ntc);
-   k_psd_sqrt<<<gp, 64, 0, g.s>>>(fl, nfl, D.prm, D.formula, D.nnl, D.ntc, D.pulsation, sq);
-   HIPC(hipGetLastError());
-   if (D.pod_nmodes > 0 || D.pod_lim > 0.0)
-      return pod_project(B, D, sq, fl, nfl, rows_per_mode, U, ldU);
-   // modes in chunks of at most 64 (grid z = component + NTC * chunk)
-   const int mt = (D.nm + 15) / 16;
-   const int nchunk = (D.nm + 63) / 64;
-   dim3 gpm(gp.x, gp.y, (unsigned)(D.ntc * nchunk));
-#define LAUNCH_PROJ(MT)                                                                       \
-   k_project<MT><<<gpm, 256, 0, g.s>>>(D.pa_t, D.lnr, sq, fl, nfl, D.nnl, D.nm, D.nnlp,       \
-                                       rows_per_mode, U, ldU, D.ntc)
-   if (mt <= 1) LAUNCH_PROJ(1);
-   else if (mt <= 2) LAUNCH_PROJ(2);
-   else if (mt <= 3) LAUNCH_PROJ(3);
-   else LAUNCH_PROJ(4);
+   int F = mt == 1 ? 8 : (mt == 2 ? 4 : 2);
+   while (F > 1 && ncoltile * ((nfl + F - 1) / F) * planes < 2048) F /= 2;
+   return F;
+}
+
+// Projection tables at the |f| list fl (nodal sqrt-PSDs sq): k_project in the layout
+// U[k*ldU + y*rows + q], or (vlay) the Mesher's U[(q*K + k)*ldU + y] with every padding
+// entry written.
+int project(const Prob &D, const double *sq, const double *fl, int nfl, int rows, double *U, long ldU,
+            bool vlay)
+{
+   const int nch = (D.nm + 63) / 64, mt = D.nm <= 64 ? (D.nm + 15) / 16 : 4;
+   // modes in chunks of at most 64 (grid z); the point layout's tiles cover its padding rows
+   const int ntile = ((vlay ? D.nnl + D.K - D.kv : D.nnl) + 15) / 16;
+   const int F = project_group(ntile, nfl, D.ntc * nch, mt);
+   const long nwave = (long)ntile * ((nfl + F - 1) / F);
+   const dim3 gr((unsigned)((nwave + 3) / 4), (unsigned)D.ntc, (unsigned)nch);
+#define LAUNCH_PROJ(MT, F, V)                                                                  \
+   k_project<MT, F, V><<<gr, 256, 0, g.s>>>(D.pa_k, D.lnr, sq, fl, nfl, D.nnl, D.nm, D.nnlp,    \
+                                            D.K, rows, U, ldU, D.ntc, ntile, nwave)
+#define LAUNCH_PROJ_F(MT, FM)                                                                  \
+   do {                                                                                        \
+      if (vlay) {                                                                              \
+         if (F == FM) LAUNCH_PROJ(MT, FM, true);                                               \
+         else if (F * 2 == FM) LAUNCH_PROJ(MT, (FM / 2 ? FM / 2 : 1), true);                   \
+         else if (F * 4 == FM) LAUNCH_PROJ(MT, (FM / 4 ? FM / 4 : 1), true);                   \
+         else LAUNCH_PROJ(MT, 1, true);                                                        \
+      } else {                                                                                 \
+         if (F == FM) LAUNCH_PROJ(MT, FM, false);                                              \
+         else if (F * 2 == FM) LAUNCH_PROJ(MT, (FM / 2 ? FM / 2 : 1), false);                  \
+         else if (F * 4 == FM) LAUNCH_PROJ(MT, (FM / 4 ? FM / 4 : 1), false);                  \
+         else LAUNCH_PROJ(MT, 1, false);                                                       \
+      }                                                                                        \
+   } while (0)
+   if (mt <= 1) LAUNCH_PROJ_F(1, 8);
+   else if (mt <= 2) LAUNCH_PROJ_F(2, 4);
+   else if (mt <= 3) LAUNCH_PROJ_F(3, 2);
+   else LAUNCH_PROJ_F(4, 2);
+#undef LAUNCH_PROJ_F
 #undef LAUNCH_PROJ
    HIPC(hipGetLastError());
    return 0;
+}
+
+// Nodal sqrt-PSD table [tc][nfl][nnl] at the |f| list fl
+int psd_table(Bufs &B, const Prob &D, const double *fl, int nfl, double **sq)
+{
+   if (nfl > 65535) return fail(BSAHIP_EUNSUPPORTED, "more than 65535 distinct frequencies in one table");
+   CHK(B.get("sq", (size_t)D.ntc * nfl * D.nnl, sq));
+   dim3 gp((D.nnl + 63) / 64, nfl, D.ntc);
+   k_psd_sqrt<<<gp, 64, 0, g.s>>>(fl, nfl, D.prm, D.formula, D.nnl, D.ntc, D.pulsation, *sq);
+   HIPC(hipGetLastError());
+   return 0;
+}
+
+// The entries of a table U[K][ldU] that no projection writes: the K rows from kv on and
+// the columns from nm*rows on.
+int zero_padding(const Prob &D, int rows, double *U, long ldU)
+{
+   CHK(fill(U + (size_t)D.kv * ldU, (size_t)(D.K - D.kv) * ldU, 0.0));
+   const long c0 = (long)D.nm * rows, n = (ldU - c0) * D.kv;
+   if (n > 0) {
+      k_zero_tail<<<(unsigned)((n + 255) / 256), 256, 0, g.s>>>(U, ldU, c0, n);
+      HIPC(hipGetLastError());
+   }
+   return 0;
+}
+
+// A table on a list of nfl = rows_per_mode |f| values (device array fl): U[K][ldU], rows
+// y*rows_per_mode + q, everything outside the valid rows and columns zero (padded: the
+// caller's U already holds those zeros).
+int build_table(Bufs &B, const Prob &D, const double *fl, int nfl, int rows_per_mode, double *U,
+                long ldU, bool padded = false)
+{
+   double *sq;
+   CHK(psd_table(B, D, fl, nfl, &sq));
+   if (!padded) CHK(zero_padding(D, rows_per_mode, U, ldU));
+   if (D.pod_nmodes > 0 || D.pod_lim > 0.0)
+      return pod_project(B, D, sq, fl, nfl, rows_per_mode, U, ldU);
+   return project(D, sq, fl, nfl, rows_per_mode, U, ldU, false);
 }
 
 int launch_frf(const Prob &D, int nft, double df, double2 *H)
@@ -602,6 +660,7 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    for (int u = 0; u < P->nu; ++u) fl[u] = (double)u * df;
    CHK(upload(P->B, "fl", fl, &P->fl));
    CHK(P->B.get("U", (size_t)P->D.K * P->ldU, &P->U));
+   CHK(zero_padding(P->D, P->nhp, P->U, P->ldU));      // the runs write the valid entries only
    CHK(P->B.get("H", (size_t)P->D.nm * P->nft, &P->H));
    const size_t nm3 = (size_t)P->D.nm * P->D.nm * P->D.nm, nm2 = (size_t)P->D.nm * P->D.nm;
    CHK(P->B.get("m3", 2 * nm3, &P->m3));
@@ -633,7 +692,7 @@ int plan_prepare(bsahip_plan *P)
 {
    Prob &D = P->D;
    const size_t nm3 = (size_t)D.nm * D.nm * D.nm;
-   CHK(build_table(P->B, D, P->fl, P->nu, P->nhp, P->U, P->ldU));
+   CHK(build_table(P->B, D, P->fl, P->nu, P->nhp, P->U, P->ldU, true));
    CHK(launch_frf(D, P->nft, P->df, P->H));
    if (!(P->flags & BSAHIP_NO_BISP)) {
       CHK(fill(P->m3, 2 * nm3, 0.0));

@@ -34,6 +34,15 @@ __global__ void k_fill(double *__restrict__ p, size_t n, double v)
    for (; i < n; i += st) p[i] = v;
 }
 
+// U[k*ld + c] = 0 for c >= c0, the first n / (ld - c0) rows
+__global__ void k_zero_tail(double *__restrict__ U, long ld, long c0, long n)
+{
+   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+   if (t >= n) return;
+   const long w = ld - c0;
+   U[t / w * ld + c0 + t % w] = 0.0;
+}
+
 // Nodal one-sided PSD, then its square root, on a list of |f| values.
 // formula: 1 von Karman u (WindPSDImpl.F90:166-188), 2 von Karman v/w (:190-222),
 // 3 Davenport-Greisch (:249-277), 5 Davenport-Uliege (:283-316), 0 zero (Kaimal,
@@ -121,80 +130,208 @@ __global__ void k_frf_table(const double *__restrict__ Mm, const double *__restr
 
 // ---------------------------------------------------------------------------
 // projection A(y,i;f) = s_i(f) sum_j Psi_a(y,j) s_j(f) exp(|f| ln rho_ji) on
-// FP64 MFMA: per frequency an (MT*16 x nnl) x (nnl x 64) product whose right
-// operand, the coherence tile rho_ji^|f|, is generated in LDS chunk by chunk.
-// grid (ceil(nnl/64), nfl, ntc * mode chunks), block 256 = 4 waves; a block
-// takes the modes y0 .. y0 + 16 MT - 1 of its chunk (y0 = chunk * 16 MT); wave
-// w owns the 16 node columns 16w.. of the block's 64 and all MT row blocks of
-// 16 modes.
+// FP64 MFMA: per frequency an (MT*16 x nnl) x (nnl x 16) product per wave.  The right
+// operand s_j rho_ji^|f| is formed in the lane that feeds it to the MFMA, once for all
+// modes, so the waves need no LDS and no barrier.  A wave takes F frequencies that are
+// neighbours in the table: they share its loads of ln rho and Psi_a, and its stores
+// become runs of F values (a table row is contiguous in the frequency).  Bound by the
+// FP64 exp (about 25 multiply-adds each); the form this replaces staged 8 nodes of a
+// 64-node coherence tile in LDS between two barriers and stored single doubles a table
+// row apart: 1000 nodes, 30 modes, 2 components, 513 frequencies 3.0 -> 1.8 ms; 200
+// nodes, 10 modes, some 4600 frequencies of the Mesher's point layout 1.7 (with the
+// transpose it no longer needs) -> 0.85 ms.  The f64 MFMAs and the FP64 vector
+// instructions add up here: 128 + 80 of the 255 cycles per 64 coherences and 32 modes.
+// Waves: column tile of 16 nodes x group of F frequencies x component x chunk of 64
+// modes; F from project_group() so that small tables still fill the chip.
 // v_mfma_f64_16x16x4f64: A lane l holds (row l%16, k l/16), B (k l/16, col l%16),
 // D register t of lane l holds (row l/16 + 4t, col l%16).
+// VLAY: the point layout U[(q*K + k)*ldU + y] of the Mesher (ldU modes, zero from nm
+// on, K rows) instead of U[k*ldU + y*row_stride + q]; its padding rows k are cleared.
 // ---------------------------------------------------------------------------
-#define PKC 8    // node (j) chunk staged in LDS
+// exp(x) of the projection's inner loop: x = n ln 2 + r, |r| <= ln 2 / 2 (Cody-Waite,
+// the high part of ln 2 cut to 33 bits so that n times it is exact), a degree-11
+// polynomial on r whose coefficients interpolate (e^r - 1 - r) / r^2 at the Chebyshev
+// nodes (relative error 2e-17), and a power of two.  0.85 ulp at most (5000 arguments
+// from -690 to 0 against 60 digits), within the 1 ulp of the library's exp, whose
+// steps these are; here the coefficients stay in scalar registers, where the library
+// call reloads eighteen vector registers with them for every value.  As there, results
+// below the subnormals are 0, those above the largest double infinite, NaN stays.
+struct ExpC {
+   double magic, inv, hi, lo, c3, c4, c5, c6, c7, c8, c9, c10, c11;
+};
 
-template <int MT>
-__global__ __launch_bounds__(256) void k_project(
-   const double *__restrict__ pa,      // [tc][nm][nnl]
+__device__ __forceinline__ ExpC exp_consts()
+{
+   ExpC e = {0x1.8p52, 0x1.71547652b82fep+0, 0x1.62e42fef00000p-1, 0x1.473de6af278edp-34,
+             0x1.5555555555555p-3, 0x1.5555555553d63p-5, 0x1.11111111109b3p-7,
+             0x1.6c16c1788bd90p-10, 0x1.a01a01a7c41d5p-13, 0x1.a019b90d2ae7ap-16,
+             0x1.71de0dae63bb3p-19, 0x1.289185613a3d6p-22, 0x1.af38a9b0ec855p-26};
+   // opaque to the compiler, so that they are not rematerialised in the loop
+   asm volatile("" : "+v"(e.magic), "+s"(e.inv), "+s"(e.hi), "+s"(e.lo), "+s"(e.c3), "+s"(e.c4),
+                     "+s"(e.c5), "+s"(e.c6), "+s"(e.c7), "+s"(e.c8), "+s"(e.c9), "+s"(e.c10));
+   asm volatile("" : "+v"(e.c11));
+   return e;
+}
+
+// `one`: 1, or NaN where x is to give NaN (the clamps drop it)
+__device__ __forceinline__ double exp_fast(double x, double one, const ExpC &e)
+{
+   x = __builtin_fmin(__builtin_fmax(x, -800.0), 720.0);
+   const double t = __builtin_fma(x, e.inv, e.magic);
+   const int n = (int)(uint32_t)__double_as_longlong(t);   // rounded to nearest
+   const double nf = t - e.magic;
+   double r = __builtin_fma(-nf, e.hi, x);
+   r = __builtin_fma(-nf, e.lo, r);
+   double p = __builtin_fma(e.c11, r, e.c10);
+   p = __builtin_fma(p, r, e.c9);
+   p = __builtin_fma(p, r, e.c8);
+   p = __builtin_fma(p, r, e.c7);
+   p = __builtin_fma(p, r, e.c6);
+   p = __builtin_fma(p, r, e.c5);
+   p = __builtin_fma(p, r, e.c4);
+   p = __builtin_fma(p, r, e.c3);
+   p = __builtin_fma(p, r, 0.5);
+   p = __builtin_fma(p, r, 1.0);
+   p = __builtin_fma(p, r, one);
+   return __builtin_amdgcn_ldexp(p, n);
+}
+
+// Two waves per SIMD at least: 256 registers, so that the accumulators stay in ordinary
+// ones (with 512 the compiler moves them to and from the accumulation registers).
+template <int MT, int F, bool VLAY>
+__global__ __launch_bounds__(256, 2) void k_project(
+   const double *__restrict__ pak,     // [nm][K]  Psi_a per K index
    const double *__restrict__ lnr,     // [tc][nnl][nnl]  ln rho_ji (row j, col i)
    const double *__restrict__ sq,      // [tc][nfl][nnl]  sqrt(S)
-   const double *__restrict__ fabs_list, int nfl, int nnl, int nm, int nnlp,
+   const double *__restrict__ fabs_list, int nfl, int nnl, int nm, int nnlp, int K,
    int row_stride,                     // rows per mode in U (nhp)
-   double *__restrict__ U, long ldU, int ntc)
+   double *__restrict__ U, long ldU, int ntc, int ncoltile, long nwave)
 {
-   constexpr int NR = MT * 16;
-   __shared__ double ps[PKC][NR];
-   __shared__ double ee[PKC][64];
-   const int tc = blockIdx.z % ntc;
-   const int y0 = (blockIdx.z / ntc) * NR;
-   const int q = blockIdx.y;
-   const int i0 = blockIdx.x * 64;
-   const int tid = threadIdx.x, lane = tid & 63;
-   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-   const double af = fabs_list[q];
-   const double *sqq = sq + ((size_t)tc * nfl + q) * nnl;
-   const double *lnt = lnr + (size_t)tc * nnl * nnl;
-   const double *pat = pa + (size_t)tc * nm * nnl;
-   d4 acc[MT];
+   const int lane = threadIdx.x & 63;
+   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const long wid = (long)blockIdx.x * 4 + w;
+   if (wid >= nwave) return;
+   const int y0 = blockIdx.z * (MT * 16);
+   const int tc = blockIdx.y;
+   // consecutive waves take consecutive frequency groups of one column tile: they
+   // share its ln rho lines
+   const long nqg = nwave / ncoltile;
+   const int i0 = (int)(wid / nqg) * 16;
+   const int q0 = (int)(wid % nqg) * F;
+   const int lr = lane & 15, lk = lane >> 4;
+   const int i = i0 + lr;
+   const int ic = min(i, nnl - 1);
+   const double *lnt = lnr + (size_t)tc * nnl * nnl + ic;
+   const double *pat[MT];              // rows y >= nm repeat the last mode: not stored
 #pragma unroll
-   for (int r = 0; r < MT; ++r) acc[r] = (d4){0.0, 0.0, 0.0, 0.0};
-
-   for (int j0 = 0; j0 < nnl; j0 += PKC) {
-      for (int t = tid; t < PKC * NR; t += 256) {
-         const int jj = t / NR, y = t % NR;
-         const int j = j0 + jj;
-         ps[jj][y] = (j < nnl && y0 + y < nm) ? pat[(size_t)(y0 + y) * nnl + j] * sqq[j] : 0.0;
-      }
-      for (int t = tid; t < PKC * 64; t += 256) {
-         const int jj = t >> 6, ii = t & 63;
-         const int j = j0 + jj, i = i0 + ii;
-         double e = 0.0;
-         if (j < nnl && i < nnl) {
-            const double l = lnt[(size_t)j * nnl + i];
-            e = (af == 0.0) ? 1.0 : exp(af * l);     // rho^0 == 1 even for rho == 0
-         }
-         ee[jj][ii] = e;
-      }
-      __syncthreads();
+   for (int r = 0; r < MT; ++r)
+      pat[r] = pak + (size_t)min(y0 + 16 * r + lr, nm - 1) * K + tc * nnlp;
+   const double *sqt = sq + (size_t)tc * nfl * nnl;
+   double af[F];
+   const double *sqq[F];
 #pragma unroll
-      for (int kk = 0; kk < PKC; kk += 4) {
-         const int kr = kk + (lane >> 4);
-         const double b = ee[kr][16 * w + (lane & 15)];
+   for (int f = 0; f < F; ++f) {
+      const int q = min(q0 + f, nfl - 1);
+      af[f] = fabs_list[q];
+      sqq[f] = sqt + (size_t)q * nnl;
+   }
+   d4 acc[F][MT];
+#pragma unroll
+   for (int f = 0; f < F; ++f)
+#pragma unroll
+      for (int r = 0; r < MT; ++r) acc[f][r] = (d4){0.0, 0.0, 0.0, 0.0};
+   const ExpC ec = exp_consts();
+   // one MFMA step: ln rho l of the lane's (j, i), Psi_a a of its (y, j), s_j
+   auto step = [&](double l, const double (&a)[MT], const double (&sj)[F]) {
+      // |f| = 0 gives 1 even for rho == 0: the infinity becomes a finite number
+      const double one = l == l ? 1.0 : l;
+      const double lc = __builtin_fmin(__builtin_fmax(l, -0x1.fffffffffffffp1023), 0x1.fffffffffffffp1023);
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+         const double e = exp_fast(af[f] * lc, one, ec) * sj[f];
 #pragma unroll
          for (int r = 0; r < MT; ++r)
-            acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(ps[kr][16 * r + (lane & 15)], b, acc[r],
-                                                          0, 0, 0);
+            acc[f][r] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], e, acc[f][r], 0, 0, 0);
       }
-      __syncthreads();
+   };
+   // pairs of steps: lane group lk takes the nodes j0 + 2 lk and j0 + 2 lk + 1, so that
+   // Psi_a and s_j come as 16-byte loads; the next pair's operands are loaded while
+   // this one's are used
+   struct pair { double v[2]; };
+   auto ld2 = [](const double *p) {
+      pair v;
+      __builtin_memcpy(&v, p, sizeof(v));
+      return v;
+   };
+   double l0, l1;
+   pair a2[MT], s2[F];
+   auto load = [&](int j0) {
+      const int j = j0 + 2 * lk;
+      l0 = lnt[(size_t)j * nnl];
+      l1 = lnt[(size_t)(j + 1) * nnl];
+#pragma unroll
+      for (int r = 0; r < MT; ++r) a2[r] = ld2(pat[r] + j);
+#pragma unroll
+      for (int f = 0; f < F; ++f) s2[f] = ld2(sqq[f] + j);
+   };
+   const int n8 = nnl & ~7;
+   if (n8 > 0) load(0);
+   for (int j0 = 0; j0 < n8; j0 += 8) {
+      const double c0 = l0, c1 = l1;
+      double a0[MT], a1[MT], x0[F], x1[F];
+#pragma unroll
+      for (int r = 0; r < MT; ++r) {
+         a0[r] = a2[r].v[0];
+         a1[r] = a2[r].v[1];
+      }
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+         x0[f] = s2[f].v[0];
+         x1[f] = s2[f].v[1];
+      }
+      if (j0 + 8 < n8) load(j0 + 8);
+      step(c0, a0, x0);
+      step(c1, a1, x1);
    }
-   const int i = i0 + 16 * w + (lane & 15);
-   if (i < nnl) {
-      const double si = sqq[i];
+   for (int j0 = n8; j0 < nnl; j0 += 4) {
+      const int j = j0 + lk, jc = min(j, nnl - 1);
+      double a[MT], x[F];
+#pragma unroll
+      for (int r = 0; r < MT; ++r) a[r] = j < nnl ? pat[r][jc] : 0.0;
+#pragma unroll
+      for (int f = 0; f < F; ++f) x[f] = j < nnl ? sqq[f][jc] : 0.0;
+      step(lnt[(size_t)jc * nnl], a, x);
+   }
+   const int k = tc * nnlp + i;
+   const bool ok = i < nnl;
+   if constexpr (VLAY) {
+      if (!ok && !(tc == ntc - 1 && k < K)) return;
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+         if (q0 + f >= nfl) break;
+         const double si = ok ? sqq[f][i] : 0.0;
+         double *d = U + ((size_t)(q0 + f) * K + k) * ldU + y0 + lk;
+#pragma unroll
+         for (int r = 0; r < MT; ++r)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+               d[16 * r + 4 * t] = ok && y0 + lk + 16 * r + 4 * t < nm ? acc[f][r][t] * si : 0.0;
+      }
+   } else {
+      if (!ok) return;
+      double si[F];
+#pragma unroll
+      for (int f = 0; f < F; ++f) si[f] = sqq[f][i];
 #pragma unroll
       for (int r = 0; r < MT; ++r)
 #pragma unroll
          for (int t = 0; t < 4; ++t) {
-            const int y = y0 + 16 * r + (lane >> 4) + 4 * t;
-            if (y < nm) U[((size_t)tc * nnlp + i) * ldU + (size_t)y * row_stride + q] = acc[r][t] * si;
+            const int y = y0 + 16 * r + lk + 4 * t;
+            if (y >= nm) continue;
+            double *d = U + (size_t)k * ldU + (size_t)y * row_stride + q0;
+#pragma unroll
+            for (int f = 0; f < F; ++f)
+               if (q0 + f < nfl) d[f] = acc[f][r][t] * si[f];
          }
    }
 }

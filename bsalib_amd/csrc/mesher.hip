@@ -34,7 +34,8 @@
 
 // ---------------------------------------------------------------------------
 // V table for point evaluation: V[(u*K + k)*NMP + y] = A(y, k; |f_u|), zero for
-// y >= nm.  Built from the U table U[k*ldU + y*nu + u].
+// y >= nm.  k_project writes it directly; the truncated POD's comes from its U table
+// U[k*ldU + y*nu + u] through this kernel.
 // grid (ceil(nu/64), K), block 256
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_vtable(const double *__restrict__ U, long ldU, int nu,
@@ -369,7 +370,7 @@ __device__ __forceinline__ double2 msh_frf(double w, double M, double K, double 
 }
 
 template <int RT, int RT2, int CPW, int NW>
-__global__ __launch_bounds__(NW * 64) void k_msh_quad(const MshTileRun *__restrict__ tr,
+__global__ __launch_bounds__(NW * 64, NW == 4 && RT < 8 ? 2 : 1) void k_msh_quad(const MshTileRun *__restrict__ tr,
                                                       const MshItem *__restrict__ items,
                                                       MshShape sh)
 {
@@ -985,12 +986,19 @@ int msh_eval_chunk(bsahip_mesher *M, int npts, const double *f1p, const double *
    const long ldU = (long)D.nm * nu;
    double *fl, *U, *V;
    CHK(upload(M->B, "m_fl", uq, &fl));
-   CHK(M->B.get("m_U", (size_t)D.K * ldU, &U));
-   CHK(build_table(M->B, D, fl, nu, nu, U, ldU));
    CHK(M->B.get("m_V", (size_t)nu * D.K * M->nmp, &V));
-   dim3 gv((nu + 63) / 64, D.K);
-   k_vtable<<<gv, 256, 0, g.s>>>(U, ldU, nu, D.nm, D.K, M->nmp, V);
-   HIPC(hipGetLastError());
+   if (D.pod_nmodes > 0 || D.pod_lim > 0.0) {
+      CHK(M->B.get("m_U", (size_t)D.K * ldU, &U));
+      CHK(build_table(M->B, D, fl, nu, nu, U, ldU));
+      dim3 gv((nu + 63) / 64, D.K);
+      k_vtable<<<gv, 256, 0, g.s>>>(U, ldU, nu, D.nm, D.K, M->nmp, V);
+      HIPC(hipGetLastError());
+   } else {
+      // the projection writes the point layout itself
+      double *sq;
+      CHK(psd_table(M->B, D, fl, nu, &sq));
+      CHK(project(D, sq, fl, nu, nu, V, M->nmp, true));
+   }
    int *d1, *d2, *d3;
    long *ds;
    CHK(upload(M->B, "m_i1", i1, &d1));
