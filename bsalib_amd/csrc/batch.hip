@@ -1,12 +1,13 @@
 // Batches of structures of uneven size (node, mode, component and frequency
-// counts): every structure is a resident plan; one step runs all their tables
-// (spread over worker streams), then ONE persistent G-contraction launch whose
-// workgroups take work items (structure, tile pair, mode) from a device queue,
-// while the worker streams compute the modal PSD moments.  The step is
-// captured once in a HIP graph (forked and joined streams become parallel
-// branches) and replayed.  The item list is ordered by decreasing cost per
-// item (longest-processing-time first) and split into one queue per XCD; a
-// small autotuner picks the persistent grid size and the items per ticket.
+// counts): every structure is a resident plan; one step builds all their tables
+// in one launch per kind (PSD, FRF and cleared sums; projection; operand split),
+// then ONE persistent G-contraction launch whose workgroups take work items
+// (structure, tile pair, mode) from a device queue, while one launch on a side
+// stream computes every structure's modal PSD moments.  The step is captured once
+// in a HIP graph (the side stream becomes a parallel branch) and replayed.  The
+// item list is ordered by decreasing cost per item (longest-processing-time
+// first) and split into one queue per XCD; a small autotuner picks the persistent
+// grid size and the items per ticket.
 
 __device__ __forceinline__ long uniform_long(long v)
 {
@@ -98,6 +99,84 @@ __global__ __launch_bounds__(256, 2) void k_gsym_f32_batch(
    });
 }
 
+// The table launches over every structure: block (or wave) -> structure by binary
+// search over the offsets, then the single-structure kernel's work.  A launch per
+// structure and table kind left the chip to one small structure at a time and cost
+// eight launches each: 64 towers (NN 20-60, NM 3-6, 65-129 points a side) 1.67 ms
+// a step, 0.52 ms with these.
+struct BatchTab {
+   const double *fl, *prm, *Mm, *Km, *Cm;
+   const int *formula;
+   double *sq, *m3, *m2;
+   double2 *H;
+   double df;
+   int nu, nnl, nm, nft, pulsation;
+   long npsd, nfrf, nm3, nm2;          // values of each kind (sums to clear: nm3, nm2)
+};
+
+__global__ __launch_bounds__(256) void k_batch_tables(const BatchTab *__restrict__ tab,
+                                                      const long *__restrict__ offs, int ns)
+{
+   const int s = batch_struct(offs, ns, blockIdx.x);
+   const BatchTab T = tab[s];
+   long t = ((long)blockIdx.x - offs[s]) * 256 + threadIdx.x;
+   if (t < T.npsd) {
+      const int i = (int)(t % T.nnl);
+      const long r = t / T.nnl;                       // tc * nu + q
+      const int q = (int)(r % T.nu), tc = (int)(r / T.nu);
+      T.sq[t] = psd_sqrt(T.prm + ((size_t)tc * T.nnl + i) * 4, T.formula[tc], T.fl[q], T.pulsation);
+      return;
+   }
+   t -= T.npsd;
+   if (t < T.nfrf) {
+      T.H[t] = frf_grid(T.Mm, T.Km, T.Cm, (int)(t / T.nft), (int)(t % T.nft), T.df);
+      return;
+   }
+   t -= T.nfrf;
+   if (t < T.nm3) T.m3[t] = 0.0;
+   else if (t - T.nm3 < T.nm2) T.m2[t - T.nm3] = 0.0;
+}
+
+template <int MT, int F>
+__global__ __launch_bounds__(256, 2) void k_project_batch(const ProjArgs *__restrict__ args,
+                                                          const long *__restrict__ offs, int ns)
+{
+   const long wid = (long)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   if (wid >= offs[ns]) return;
+   const int s = batch_struct(offs, ns, wid);
+   const ProjArgs P = args[s];
+   const long l = wid - offs[s], per = P.nqg * P.ncoltile;
+   const int r = (int)(l / per);
+   project_wave<MT, F, false>(P, l % per, r % P.ntc, (r / P.ntc) * (MT * 16));
+}
+
+struct SplitArgs {
+   const double *U;
+   float *UR;
+   uint16_t *Ch, *Cl;
+   long ldU;
+   int K;
+};
+
+__global__ __launch_bounds__(256) void k_split_batch(const SplitArgs *__restrict__ args,
+                                                     const long *__restrict__ offs, int ns)
+{
+   const int s = batch_struct(offs, ns, blockIdx.x);
+   const SplitArgs a = args[s];
+   const long l = (long)blockIdx.x - offs[s], nr = a.ldU / 32;
+   split_tile((int)(l % nr) * 32, (int)(l / nr) * 32, a.U, a.ldU, a.K, (int)a.ldU, a.K, a.UR, a.Ch, a.Cl);
+}
+
+template <int MT>
+__global__ __launch_bounds__(256, 2) void k_m2_batch(const M2Args *__restrict__ args,
+                                                     const long *__restrict__ offs, int ns)
+{
+   const int s = batch_struct(offs, ns, blockIdx.x);
+   const M2Args a = args[s];
+   const int l = (int)((long)blockIdx.x - offs[s]), nby = (a.nh + 63) / 64;
+   m2_block<MT>(a, l % a.nm, (l / a.nm) % nby, l / (a.nm * nby) * 16 * MT);
+}
+
 // results of every structure into one contiguous buffer: array j = srcs[j]
 // (lens[j] doubles) to dst + offs[j]; one block per array
 __global__ void k_pack(const double *const *__restrict__ srcs, const long *__restrict__ lens,
@@ -127,11 +206,25 @@ struct bsahip_batch {
    hipGraph_t graph = nullptr;
    hipGraphExec_t gexec = nullptr;
    double ms_total = 0.0, ms_gsym = 0.0;
-   // worker streams (default priority) for the per-structure table and PSD
-   // moment kernels, forked from and joined to the library stream
-   std::vector<hipStream_t> ws;
-   hipEvent_t ev_fork = nullptr;
-   std::vector<hipEvent_t> ev_prep, ev_m2;
+   // side stream (default priority) of the PSD moments, forked from and joined to
+   // the library stream
+   hipStream_t side = nullptr;
+   hipEvent_t ev_fork = nullptr, ev_m2 = nullptr;
+   // launches over every structure: descriptors and their block (wave) offsets, the
+   // structures of one template instance together
+   BatchTab *tab = nullptr;
+   SplitArgs *split = nullptr;
+   long *tab_offs = nullptr, *split_offs = nullptr;
+   long tab_blocks = 0, split_blocks = 0;
+   struct Group {
+      int mt, F, n;              // template arguments, structures
+      long total;                // blocks or waves
+      long *offs;
+      ProjArgs *proj;
+      M2Args *m2;
+   };
+   std::vector<Group> proj, m2;
+   bool joint = true;            // one table launch per kind (batch_descriptors)
    // packed results: per structure m3 (m3f, m3r) then m2 (f, r, o)
    const double **psrc = nullptr;
    long *plen = nullptr, *poff = nullptr;
@@ -143,10 +236,9 @@ struct bsahip_batch {
       if (hpack) (void)hipHostFree(hpack);
       if (gexec) (void)hipGraphExecDestroy(gexec);
       if (graph) (void)hipGraphDestroy(graph);
-      for (auto e : ev_prep) (void)hipEventDestroy(e);
-      for (auto e : ev_m2) (void)hipEventDestroy(e);
+      if (ev_m2) (void)hipEventDestroy(ev_m2);
       if (ev_fork) (void)hipEventDestroy(ev_fork);
-      for (auto st : ws) (void)hipStreamDestroy(st);
+      if (side) (void)hipStreamDestroy(side);
    }
 };
 
@@ -180,21 +272,141 @@ int batch_launch(bsahip_batch *b)
    return 0;
 }
 
-// the library stream is g.s; run f with g.s switched to another stream
-template <class F>
-int on_stream(hipStream_t st, F f)
+// descriptors of the launches over every structure, on the device
+int batch_descriptors(bsahip_batch *b)
 {
-   const hipStream_t keep = g.s;
-   g.s = st;
-   const int rc = f();
-   g.s = keep;
-   return rc;
+   const bool bisp = !(b->flags & BSAHIP_NO_BISP), psd = !(b->flags & BSAHIP_NO_PSD);
+   const int n = (int)b->plans.size();
+   auto up = [&](const char *name, const auto &h, auto **d) -> int { return upload(b->B, name, h, d); };
+   std::vector<BatchTab> tab;
+   std::vector<SplitArgs> sp;
+   std::vector<long> toff(1, 0), soff(1, 0);
+   for (auto &P : b->plans) {
+      const Prob &D = P->D;
+      BatchTab T;
+      CHK(P->B.get("sq", (size_t)D.ntc * P->nu * D.nnl, &T.sq));
+      T.fl = P->fl;
+      T.prm = D.prm;
+      T.Mm = D.Mm;
+      T.Km = D.Km;
+      T.Cm = D.Cm;
+      T.formula = D.formula;
+      T.m3 = P->m3;
+      T.m2 = P->m2;
+      T.H = P->H;
+      T.df = P->df;
+      T.nu = P->nu;
+      T.nnl = D.nnl;
+      T.nm = D.nm;
+      T.nft = P->nft;
+      T.pulsation = D.pulsation;
+      T.npsd = (long)D.ntc * P->nu * D.nnl;
+      T.nfrf = (long)D.nm * P->nft;
+      T.nm3 = bisp ? 2L * D.nm * D.nm * D.nm : 0;
+      T.nm2 = psd ? 3L * D.nm * D.nm : 0;
+      tab.push_back(T);
+      toff.push_back(toff.back() + (T.npsd + T.nfrf + T.nm3 + T.nm2 + 255) / 256);
+      sp.push_back(SplitArgs{P->U, P->UR, P->Ch, P->Cl, P->ldU, D.K});
+      soff.push_back(soff.back() + P->ldU / 32 * ((D.K + 31) / 32));
+   }
+   b->tab_blocks = toff.back();
+   b->split_blocks = bisp && b->prec != BSAHIP_PREC_FP64 ? soff.back() : 0;
+   CHK(up("bt_tab", tab, &b->tab));
+   CHK(up("bt_toff", toff, &b->tab_offs));
+   CHK(up("bt_split", sp, &b->split));
+   CHK(up("bt_soff", soff, &b->split_offs));
+   for (int mt = 1; mt <= 4; ++mt) {
+      // one frequency group size per template, as if the structures were one table
+      std::vector<int> in;
+      long tiles = 0;
+      int nfl = 1;
+      for (int i = 0; i < n; ++i) {
+         const bsahip_plan *P = b->plans[i].get();
+         if (proj_mt(P->D.nm) != mt) continue;
+         in.push_back(i);
+         nfl = std::max(nfl, P->nu);
+      }
+      if (in.empty()) continue;
+      std::vector<ProjArgs> pa;
+      for (int i : in) {
+         const bsahip_plan *P = b->plans[i].get();
+         pa.push_back(proj_args(P->D, tab[i].sq, P->fl, P->nu, P->nhp, P->U, P->ldU, false));
+         tiles += (long)pa.back().ncoltile * P->D.ntc * proj_chunks(P->D.nm) * P->nu / nfl + 1;
+      }
+      bsahip_batch::Group G;
+      G.mt = mt;
+      G.F = project_group(tiles, nfl, 1, mt);
+      G.n = (int)in.size();
+      std::vector<long> off(1, 0);
+      for (size_t k = 0; k < in.size(); ++k) {
+         ProjArgs &A = pa[k];
+         A.nqg = (A.nfl + G.F - 1) / G.F;
+         off.push_back(off.back() + A.nqg * A.ncoltile * A.ntc * proj_chunks(A.nm));
+      }
+      G.total = off.back();
+      G.m2 = nullptr;
+      const std::string id = std::to_string(mt);
+      CHK(up(("bt_proj" + id).c_str(), pa, &G.proj));
+      CHK(up(("bt_poff" + id).c_str(), off, &G.offs));
+      b->proj.push_back(G);
+   }
+   for (int mt = 1; psd && mt <= 2; ++mt) {
+      std::vector<M2Args> a;
+      std::vector<long> off(1, 0);
+      for (auto &P : b->plans) {
+         const int nm = P->D.nm;
+         if ((nm <= 16 ? 1 : 2) != mt) continue;
+         a.push_back(plan_m2_args(P.get()));
+         off.push_back(off.back() + (long)nm * ((P->nh + 63) / 64) * ((nm + 16 * mt - 1) / (16 * mt)));
+      }
+      if (a.empty()) continue;
+      bsahip_batch::Group G;
+      G.mt = mt;
+      G.F = 0;
+      G.n = (int)a.size();
+      G.total = off.back();
+      G.proj = nullptr;
+      const std::string id = std::to_string(mt);
+      CHK(up(("bt_m2" + id).c_str(), a, &G.m2));
+      CHK(up(("bt_m2off" + id).c_str(), off, &G.offs));
+      b->m2.push_back(G);
+   }
+   // a launch holds at most 2^32 threads: batches beyond that (thousands of large
+   // structures) build their tables structure by structure
+   b->joint = b->tab_blocks <= 0xffffffL && b->split_blocks <= 0xffffffL;
+   for (const auto *v : {&b->proj, &b->m2})
+      for (const auto &G : *v) b->joint = b->joint && G.total <= 0xffffffL;
+   return 0;
+}
+
+// tables of every structure on the library stream
+int batch_tables(bsahip_batch *b)
+{
+   const int n = (int)b->plans.size();
+   if (!b->joint) {
+      for (auto &P : b->plans) CHK(plan_prepare(P.get()));
+      return 0;
+   }
+   k_batch_tables<<<(unsigned)b->tab_blocks, 256, 0, g.s>>>(b->tab, b->tab_offs, n);
+   HIPC(hipGetLastError());
+   for (const auto &G : b->proj) {
+      proj_dispatch(G.mt, G.F, [&](auto MT, auto F) {
+         k_project_batch<decltype(MT)::value, decltype(F)::value>
+            <<<(unsigned)((G.total + 3) / 4), 256, 0, g.s>>>(G.proj, G.offs, G.n);
+      });
+      HIPC(hipGetLastError());
+   }
+   if (b->split_blocks) {
+      k_split_batch<<<(unsigned)b->split_blocks, 256, 0, g.s>>>(b->split, b->split_offs, n);
+      HIPC(hipGetLastError());
+   }
+   return 0;
 }
 
 // one step, stream-ordered, no host synchronisation (capturable).
-// mode 1: everything on the library stream, one G launch per structure.
-// mode 0: tables on the worker streams, then the persistent G launch on the
-// library stream while the workers compute the PSD moments.
+// mode 1: everything on the library stream, one launch per structure and kind.
+// mode 0: the tables of every structure, then the persistent G launch on the
+// library stream while the side stream computes the PSD moments.
 int batch_step(bsahip_batch *b, int mode)
 {
    const bool bisp = !(b->flags & BSAHIP_NO_BISP), psd = !(b->flags & BSAHIP_NO_PSD);
@@ -208,25 +420,29 @@ int batch_step(bsahip_batch *b, int mode)
       HIPC(hipGetLastError());
       return 0;
    }
-   const int nw = (int)b->ws.size();
-   const hipStream_t main = g.s;
-   HIPC(hipEventRecord(b->ev_fork, main));
-   for (int w = 0; w < nw; ++w) HIPC(hipStreamWaitEvent(b->ws[w], b->ev_fork, 0));
-   for (size_t i = 0; i < b->plans.size(); ++i)
-      CHK(on_stream(b->ws[i % nw], [&] { return plan_prepare(b->plans[i].get()); }));
-   for (int w = 0; w < nw; ++w) {
-      HIPC(hipEventRecord(b->ev_prep[w], b->ws[w]));
-      HIPC(hipStreamWaitEvent(main, b->ev_prep[w], 0));
+   CHK(batch_tables(b));
+   if (psd) {
+      HIPC(hipEventRecord(b->ev_fork, g.s));
+      HIPC(hipStreamWaitEvent(b->side, b->ev_fork, 0));
+      if (!b->joint) {
+         const hipStream_t keep = g.s;
+         int rc = 0;
+         g.s = b->side;
+         for (size_t i = 0; i < b->plans.size() && rc == 0; ++i) rc = plan_m2(b->plans[i].get());
+         g.s = keep;
+         CHK(rc);
+      }
+      for (const auto &G : b->m2) {
+         if (!b->joint) break;
+         if (G.mt == 1) k_m2_batch<1><<<(unsigned)G.total, 256, 0, b->side>>>(G.m2, G.offs, G.n);
+         else k_m2_batch<2><<<(unsigned)G.total, 256, 0, b->side>>>(G.m2, G.offs, G.n);
+         HIPC(hipGetLastError());
+      }
+      HIPC(hipEventRecord(b->ev_m2, b->side));
    }
    if (bisp) CHK(batch_launch(b));
-   if (psd)
-      for (size_t i = 0; i < b->plans.size(); ++i)
-         CHK(on_stream(b->ws[i % nw], [&] { return plan_m2(b->plans[i].get()); }));
-   for (int w = 0; w < nw; ++w) {
-      HIPC(hipEventRecord(b->ev_m2[w], b->ws[w]));
-      HIPC(hipStreamWaitEvent(main, b->ev_m2[w], 0));
-   }
-   k_pack<<<(unsigned)(2 * b->plans.size()), 256, 0, main>>>(b->psrc, b->plen, b->poff, b->pack);
+   if (psd) HIPC(hipStreamWaitEvent(g.s, b->ev_m2, 0));
+   k_pack<<<(unsigned)(2 * b->plans.size()), 256, 0, g.s>>>(b->psrc, b->plen, b->poff, b->pack);
    HIPC(hipGetLastError());
    return 0;
 }
@@ -319,15 +535,8 @@ int bsahip_batch_create(const bsahip_problem *const *probs, const int32_t *nfh, 
    else
       HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_gsym_f64_batch, 256, 0));
    B->occ = std::max(1, occ);
-   const int nw = std::min(8, n);
-   B->ws.resize(nw, nullptr);
-   B->ev_prep.resize(nw, nullptr);
-   B->ev_m2.resize(nw, nullptr);
-   for (int w = 0; w < nw; ++w) {
-      HIPC(hipStreamCreateWithFlags(&B->ws[w], hipStreamNonBlocking));
-      HIPC(hipEventCreateWithFlags(&B->ev_prep[w], hipEventDisableTiming));
-      HIPC(hipEventCreateWithFlags(&B->ev_m2[w], hipEventDisableTiming));
-   }
+   HIPC(hipStreamCreateWithFlags(&B->side, hipStreamNonBlocking));
+   HIPC(hipEventCreateWithFlags(&B->ev_m2, hipEventDisableTiming));
    HIPC(hipEventCreateWithFlags(&B->ev_fork, hipEventDisableTiming));
    {
       std::vector<const double *> src;
@@ -356,6 +565,7 @@ int bsahip_batch_create(const bsahip_problem *const *probs, const int32_t *nfh, 
       HIPC(hipMemcpyAsync(B->poff, off.data(), off.size() * sizeof(long), hipMemcpyHostToDevice, g.s));
       HIPC(hipHostMalloc((void **)&B->hpack, (size_t)o * sizeof(double), hipHostMallocDefault));
    }
+   CHK(batch_descriptors(B.get()));
    // warm-up run: every buffer reaches its size before a graph is captured
    CHK(batch_step(B.get(), 1));
    HIPC(hipStreamSynchronize(g.s));

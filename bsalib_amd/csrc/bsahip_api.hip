@@ -25,6 +25,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -409,39 +410,65 @@ int project_group(long ncoltile, int nfl, int planes, int mt)
 
 // Projection tables at the |f| list fl (nodal sqrt-PSDs sq): k_project in the layout
 // U[k*ldU + y*rows + q], or (vlay) the Mesher's U[(q*K + k)*ldU + y] with every padding
-// entry written.
+// entry written.  proj_args leaves nqg to the caller, who knows F.
+ProjArgs proj_args(const Prob &D, const double *sq, const double *fl, int nfl, int rows, double *U,
+                   long ldU, bool vlay)
+{
+   ProjArgs P;
+   P.pak = D.pa_k;
+   P.lnr = D.lnr;
+   P.sq = sq;
+   P.fabs_list = fl;
+   P.nfl = nfl;
+   P.nnl = D.nnl;
+   P.nm = D.nm;
+   P.nnlp = D.nnlp;
+   P.K = D.K;
+   P.row_stride = rows;
+   P.ntc = D.ntc;
+   // the point layout's tiles cover its padding rows
+   P.ncoltile = ((vlay ? D.nnl + D.K - D.kv : D.nnl) + 15) / 16;
+   P.U = U;
+   P.ldU = ldU;
+   P.nqg = 0;
+   return P;
+}
+
+// 16-mode tiles of a projection wave, chunks of modes (grid z)
+int proj_mt(int nm) { return nm <= 64 ? (nm + 15) / 16 : 4; }
+int proj_chunks(int nm) { return (nm + 63) / 64; }
+
+// f(integral constants MT, F) for the tiles mt and the group F of project_group
+template <class Fn>
+void proj_dispatch(int mt, int F, Fn f)
+{
+   auto g = [&](auto MT, auto FM) {
+      constexpr int M = decltype(MT)::value, X = decltype(FM)::value;
+      if (F >= X) f(MT, FM);
+      else if (F >= 4 && X > 4) f(MT, std::integral_constant<int, X < 4 ? X : 4>());
+      else if (F >= 2 && X > 2) f(MT, std::integral_constant<int, X < 2 ? X : 2>());
+      else f(MT, std::integral_constant<int, 1>());
+      (void)M;
+   };
+   if (mt <= 1) g(std::integral_constant<int, 1>(), std::integral_constant<int, 8>());
+   else if (mt <= 2) g(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
+   else if (mt <= 3) g(std::integral_constant<int, 3>(), std::integral_constant<int, 2>());
+   else g(std::integral_constant<int, 4>(), std::integral_constant<int, 2>());
+}
+
 int project(const Prob &D, const double *sq, const double *fl, int nfl, int rows, double *U, long ldU,
             bool vlay)
 {
-   const int nch = (D.nm + 63) / 64, mt = D.nm <= 64 ? (D.nm + 15) / 16 : 4;
-   // modes in chunks of at most 64 (grid z); the point layout's tiles cover its padding rows
-   const int ntile = ((vlay ? D.nnl + D.K - D.kv : D.nnl) + 15) / 16;
-   const int F = project_group(ntile, nfl, D.ntc * nch, mt);
-   const long nwave = (long)ntile * ((nfl + F - 1) / F);
-   const dim3 gr((unsigned)((nwave + 3) / 4), (unsigned)D.ntc, (unsigned)nch);
-#define LAUNCH_PROJ(MT, F, V)                                                                  \
-   k_project<MT, F, V><<<gr, 256, 0, g.s>>>(D.pa_k, D.lnr, sq, fl, nfl, D.nnl, D.nm, D.nnlp,    \
-                                            D.K, rows, U, ldU, D.ntc, ntile, nwave)
-#define LAUNCH_PROJ_F(MT, FM)                                                                  \
-   do {                                                                                        \
-      if (vlay) {                                                                              \
-         if (F == FM) LAUNCH_PROJ(MT, FM, true);                                               \
-         else if (F * 2 == FM) LAUNCH_PROJ(MT, (FM / 2 ? FM / 2 : 1), true);                   \
-         else if (F * 4 == FM) LAUNCH_PROJ(MT, (FM / 4 ? FM / 4 : 1), true);                   \
-         else LAUNCH_PROJ(MT, 1, true);                                                        \
-      } else {                                                                                 \
-         if (F == FM) LAUNCH_PROJ(MT, FM, false);                                              \
-         else if (F * 2 == FM) LAUNCH_PROJ(MT, (FM / 2 ? FM / 2 : 1), false);                  \
-         else if (F * 4 == FM) LAUNCH_PROJ(MT, (FM / 4 ? FM / 4 : 1), false);                  \
-         else LAUNCH_PROJ(MT, 1, false);                                                       \
-      }                                                                                        \
-   } while (0)
-   if (mt <= 1) LAUNCH_PROJ_F(1, 8);
-   else if (mt <= 2) LAUNCH_PROJ_F(2, 4);
-   else if (mt <= 3) LAUNCH_PROJ_F(3, 2);
-   else LAUNCH_PROJ_F(4, 2);
-#undef LAUNCH_PROJ_F
-#undef LAUNCH_PROJ
+   ProjArgs P = proj_args(D, sq, fl, nfl, rows, U, ldU, vlay);
+   const int mt = proj_mt(D.nm), nch = proj_chunks(D.nm);
+   const int F = project_group(P.ncoltile, nfl, D.ntc * nch, mt);
+   P.nqg = (nfl + F - 1) / F;
+   const dim3 gr((unsigned)((P.nqg * P.ncoltile + 3) / 4), (unsigned)D.ntc, (unsigned)nch);
+   proj_dispatch(mt, F, [&](auto MT, auto FF) {
+      constexpr int M = decltype(MT)::value, X = decltype(FF)::value;
+      if (vlay) k_project<M, X, true><<<gr, 256, 0, g.s>>>(P);
+      else k_project<M, X, false><<<gr, 256, 0, g.s>>>(P);
+   });
    HIPC(hipGetLastError());
    return 0;
 }
@@ -763,15 +790,39 @@ int plan_gsym(bsahip_plan *P)
    return 0;
 }
 
+M2Args plan_m2_args(const bsahip_plan *P)
+{
+   const Prob &D = P->D;
+   const size_t nm2 = (size_t)D.nm * D.nm;
+   M2Args a;
+   a.U = P->U;
+   a.ldU = P->ldU;
+   a.pa = D.pa_k;
+   a.K = D.K;
+   a.nm = D.nm;
+   a.nhp = P->nhp;
+   a.nh = P->nh;
+   a.H = P->H;
+   a.nft = P->nft;
+   a.d = P->d;
+   a.om_step = 2.0 * M_PI * P->df;
+   a.m2f = P->m2;
+   a.m2r = P->m2 + nm2;
+   a.m2o = P->m2 + 2 * nm2;
+   a.m2part = P->m2part;
+   return a;
+}
+
 int plan_m2(bsahip_plan *P)
 {
    Prob &D = P->D;
    const size_t nm2 = (size_t)D.nm * D.nm;
-   CHK(fill(P->m2, 3 * nm2, 0.0));
-   const int nby = (P->nh + 63) / 64;
-   dim3 gm((unsigned)(D.nm * D.nm), (unsigned)nby);
-   k_m2<<<gm, 256, 0, g.s>>>(P->U, P->ldU, D.pa_k, D.K, D.nm, P->nhp, P->nh, P->H, P->nft, P->d,
-                             2.0 * M_PI * P->df, P->m2, P->m2 + nm2, P->m2 + 2 * nm2, P->m2part);
+   const int nby = (P->nh + 63) / 64, mt = D.nm <= 16 ? 1 : 2;
+   if (!P->m2part) CHK(fill(P->m2, 3 * nm2, 0.0));
+   const dim3 gm((unsigned)D.nm, (unsigned)nby, (unsigned)((D.nm + 16 * mt - 1) / (16 * mt)));
+   const M2Args a = plan_m2_args(P);
+   if (mt == 1) k_m2<1><<<gm, 256, 0, g.s>>>(a);
+   else k_m2<2><<<gm, 256, 0, g.s>>>(a);
    HIPC(hipGetLastError());
    if (P->m2part) {
       const long n = 3 * (long)nm2;

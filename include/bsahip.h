@@ -478,8 +478,8 @@ int bsahip_batch_create(const bsahip_problem *const *probs, const int32_t *nfh, 
  * {1,4,16} items per queue ticket on a quarter of the queue; keeps the fastest */
 int bsahip_batch_autotune(bsahip_batch *b, int32_t *grid_mult, int32_t *chunk);
 /* mode 0: the captured graph of the step; 1: one G launch per structure, all on
- * the library stream; 2: the step of mode 0 launched directly (the worker
- * streams then run concurrently on the hardware queues).  Per-structure outputs
+ * the library stream; 2: the step of mode 0 launched directly (the side stream
+ * of the modal PSD moments then runs concurrently).  Per-structure outputs
  * (arrays of n host pointers, each NM_s^3 or NM_s^2; any may be NULL). */
 int bsahip_batch_run(bsahip_batch *b, int32_t mode, double *const *m3mf, double *const *m3mr,
                      double *const *m2mr);
