@@ -64,14 +64,14 @@ __device__ __forceinline__ void batch_drain(const long *__restrict__ offs, int n
    }
 }
 
-__global__ __launch_bounds__(256, 4) void k_gsym_f64_batch(const GsymArgs *__restrict__ args,
+__global__ __launch_bounds__(256, 2) void k_gsym_f64_batch(const GsymArgs *__restrict__ args,
                                                         const long *__restrict__ offs, int ns,
                                                         const long *__restrict__ qbeg,
                                                         unsigned long long *counters, int chunk)
 {
    batch_drain(offs, ns, qbeg, counters, chunk, [&](int s, long li) {
       const GsymArgs a = args[s];
-      gsym_f64_item(a, (int)(li % a.nm), li / a.nm);
+      gsym_f64_wave<2, 2, false>(a, (int)(li % a.nm), li / a.nm);
    });
 }
 
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(256, 2) void k_m2_batch(const M2Args *__restrict__ 
    const int s = batch_struct(offs, ns, blockIdx.x);
    const M2Args a = args[s];
    const int l = (int)((long)blockIdx.x - offs[s]), nby = (a.nh + 63) / 64;
-   m2_block<MT>(a, l % a.nm, (l / a.nm) % nby, l / (a.nm * nby) * 16 * MT);
+   m2_block<MT>(a, l % a.nm, (l / a.nm) % nby, l / (a.nm * nby) * 16 * MT, 0);
 }
 
 // results of every structure into one contiguous buffer: array j = srcs[j]
@@ -357,6 +357,7 @@ int batch_descriptors(bsahip_batch *b)
          const int nm = P->D.nm;
          if ((nm <= 16 ? 1 : 2) != mt) continue;
          a.push_back(plan_m2_args(P.get()));
+         a.back().kper = a.back().K;               // one slice
          off.push_back(off.back() + (long)nm * ((P->nh + 63) / 64) * ((nm + 16 * mt - 1) / (16 * mt)));
       }
       if (a.empty()) continue;
@@ -492,6 +493,7 @@ int bsahip_batch_create(const bsahip_problem *const *probs, const int32_t *nfh, 
    B->flags = flags;
    for (int i = 0; i < n; ++i) {
       std::unique_ptr<bsahip_plan> P(new bsahip_plan());
+      P->f64_br = P->f64_bc = 2;               // the persistent kernel's tile
       const int rc = plan_setup(P.get(), probs[i], nfh[i], df[i], flags, 0);
       if (rc) {
          g_err = "structure " + std::to_string(i) + ": " + g_err;

@@ -563,6 +563,7 @@ struct bsahip_plan {
    Prob D;
    int32_t flags = 0, prec = 0;
    int nh = 0, nf = 0, nu = 0, nhp = 0, rows = 0, ntile = 0, nft = 0;
+   int f64_br = 0, f64_bc = 0;           // FP64 wave tile in blocks of 16 (0: f64_shape's)
    long ldU = 0;
    double df = 0.0, d = 0.0;
    double *fl = nullptr, *U = nullptr, *m3 = nullptr, *m2 = nullptr;
@@ -590,6 +591,37 @@ void host_pair(long t, int &R, int &Q)
    R = (int)(t - q * (q + 1) / 2);
 }
 
+// FP64 wave tile (blocks of 16 rows x columns) for `rows` table rows and nm modes x: the
+// larger tiles load and scale less per MFMA, the smaller ones give more waves.  Measured
+// in us at (rows, nm, K), tiles 1x1 / 2x2 / 4x2: full model (17, 1, 32) 9 / 11 / -,
+// (66, 2, 32) 14 / 20 / -, (195, 3, 32) 22 / 20 / 30, (606, 6, 128) 53 / 34 / 39,
+// (909, 9, 320) 173 / 110 / 116, (1300, 20, 96) 400 / 227 / 224, (2570, 10, 608)
+// 1911 / 987 / 890; diagonal model, no accumulators shared between modes,
+// (257, 4, 608) 33 / 39 / -, (65, 60, 128) 11 / 14 / -, (257, 20, 3008) 297 / 243 / -.
+// `least` is the count of waves from which 2x2 is the faster.
+void f64_shape(long rows, int nm, double least, int &br, int &bc)
+{
+   const auto waves = [&](int r, int c) { return (double)rows * (double)rows / (512.0 * r * c) * nm; };
+   if (waves(4, 2) >= 4096.0) {
+      br = 4;
+      bc = 2;
+   } else if (waves(2, 2) >= least) {
+      br = bc = 2;
+   } else {
+      br = bc = 1;
+   }
+}
+
+constexpr double F64_LEAST = 32.0, F64_LEAST_DIAG = 384.0;
+
+// workgroups of one G launch
+long plan_items(const bsahip_plan *P)
+{
+   const long t = P->prec == BSAHIP_PREC_FP64 ? f64_tiles(P->rows, P->f64_br, P->f64_bc)
+                                              : (long)P->ntile * (P->ntile + 1) / 2;
+   return t * P->D.nm;
+}
+
 // Slot lists of the fixed-order mode: the flushes of every wave of every G
 // item in the order epi_wave makes them (kernels.hip), each with the twelve m3
 // entries of epi_flush (m3f entries 0 .. NM^3-1, m3r entries NM^3 .. 2 NM^3-1).
@@ -600,17 +632,24 @@ void det_slot_lists(const bsahip_plan *P, std::vector<long> &off, std::vector<lo
 {
    const int nm = P->D.nm, nhp = P->nhp;
    const bool f64 = (P->prec == BSAHIP_PREC_FP64);
-   const int T = f64 ? TILE : T2, WT = f64 ? 32 : 64, BR = WT / 16, BC = BR;
-   const long nm3 = (long)nm * nm * nm, nent = 2 * nm3;
-   const long npairs = (long)P->ntile * (P->ntile + 1) / 2, nitems = npairs * nm;
+   const int BR = f64 ? P->f64_br : 4, BC = f64 ? P->f64_bc : 4;
+   const long nm3 = (long)nm * nm * nm, nent = 2 * nm3, nitems = plan_items(P);
    auto walk = [&](auto emit) {
       for (long lid = 0; lid < nitems; ++lid) {
          const int x = (int)(lid % nm);
          int R, Q;
-         host_pair(lid / nm, R, Q);
-         const bool diag = (R == Q);
+         if (f64) f64_tile(lid / nm, 4 * BC / BR, Q, R);
+         else host_pair(lid / nm, R, Q);
          for (int w = 0; w < 4; ++w) {
-            const int rw0 = R * T + (w >> 1) * WT, cw0 = Q * T + (w & 1) * WT;
+            int rw0 = R * T2 + (w >> 1) * 64, cw0 = Q * T2 + (w & 1) * 64;
+            bool diag = (R == Q);
+            if (f64) {                     // gsym_f64_wave
+               const int c = 4 * Q + w, q = c * BC / BR;
+               if (R > q || c * 16 * BC >= P->rows) continue;
+               rw0 = R * 16 * BR;
+               cw0 = c * 16 * BC;
+               diag = (R == q);
+            }
             const int y0 = rw0 / nhp, y1 = (rw0 + 16 * BR - 1) / nhp;
             const int z0 = cw0 / nhp, z1 = (cw0 + 16 * BC - 1) / nhp;
             int f = 0;
@@ -672,8 +711,9 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    // block may span two modes, and the epilogue masks the other mode's rows
    P->nhp = P->nu;
    P->rows = P->D.nm * P->nhp;
-   const int tile = (P->prec == BSAHIP_PREC_FP64) ? TILE : T2;
+   const int tile = (P->prec == BSAHIP_PREC_FP64) ? 64 : T2;
    P->ntile = (P->rows + tile - 1) / tile;
+   if (P->f64_br == 0) f64_shape(P->rows, P->D.nm, F64_LEAST, P->f64_br, P->f64_bc);
    P->ldU = (long)round_up(P->rows, T2);
    P->nft = 2 * P->nu - 1;
    P->d = p->pulsation ? df * 2.0 * M_PI : df;
@@ -697,7 +737,7 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
       det_slot_lists(P, off, idx, P->mflush);
       CHK(upload(P->B, "det_off", off, &P->det_off));
       CHK(upload(P->B, "det_idx", idx, &P->det_idx));
-      CHK(P->B.get("det_slots", (size_t)npairs * P->D.nm * 4 * P->mflush * 12, &P->slots));
+      CHK(P->B.get("det_slots", (size_t)plan_items(P) * 4 * P->mflush * 12, &P->slots));
    }
    if ((flags & BSAHIP_DETERMINISTIC) && !(flags & BSAHIP_NO_PSD))
       CHK(P->B.get("m2part", (size_t)((P->nh + 63) / 64) * 3 * nm2, &P->m2part));
@@ -744,8 +784,6 @@ void plan_args(const bsahip_plan *P, GsymArgs &a, GsymArgs16 &b16)
    a.nhp = P->nhp;
    a.nh = P->nh;
    a.nu = P->nu;
-   a.ntile = P->ntile;
-   a.npairs = (long)P->ntile * (P->ntile + 1) / 2;
    a.H = P->H;
    a.nft = P->nft;
    a.d2 = P->d * P->d;
@@ -762,11 +800,6 @@ void plan_args(const bsahip_plan *P, GsymArgs &a, GsymArgs16 &b16)
    b16.ldk = D.K;
 }
 
-long plan_items(const bsahip_plan *P)
-{
-   return (long)P->ntile * (P->ntile + 1) / 2 * P->D.nm;
-}
-
 int plan_gsym(bsahip_plan *P)
 {
    GsymArgs a;
@@ -777,8 +810,12 @@ int plan_gsym(bsahip_plan *P)
       k_gsym_bf16x3<<<dim3((unsigned)nwg), 256, 0, g.s>>>(a, b16);
    else if (P->prec == BSAHIP_PREC_FP32)
       k_gsym_f32<<<dim3((unsigned)nwg), 256, 0, g.s>>>(a, b16);
+   else if (P->f64_br == 4)
+      k_gsym_f64<4, 2><<<dim3((unsigned)nwg), 256, 0, g.s>>>(a);
+   else if (P->f64_br == 2)
+      k_gsym_f64<2, 2><<<dim3((unsigned)nwg), 256, 0, g.s>>>(a);
    else
-      k_gsym_f64<<<dim3((unsigned)nwg), 256, 0, g.s>>>(a);
+      k_gsym_f64<1, 1><<<dim3((unsigned)nwg), 256, 0, g.s>>>(a);
    HIPC(hipGetLastError());
    if (P->slots) {
       // fixed order: every m3 entry sums its slots in ascending order
@@ -788,6 +825,14 @@ int plan_gsym(bsahip_plan *P)
       HIPC(hipGetLastError());
    }
    return 0;
+}
+
+// K rows per slice of k_m2 so that some `want` blocks run (each at least 64 rows, 4 MFMA
+// steps per wave: shorter slices are all reduction); want 1: no slices
+int m2_slice(int want, long blocks, int K)
+{
+   const int n = (int)std::max<long>(1, std::min<long>(want / std::max<long>(1, blocks), K / 64));
+   return round_up((K + n - 1) / n, 16);
 }
 
 M2Args plan_m2_args(const bsahip_plan *P)
@@ -810,6 +855,8 @@ M2Args plan_m2_args(const bsahip_plan *P)
    a.m2r = P->m2 + nm2;
    a.m2o = P->m2 + 2 * nm2;
    a.m2part = P->m2part;
+   a.diag = 0;
+   a.kper = m2_slice(P->m2part ? 1 : 1024, (long)D.nm * ((P->nh + 63) / 64), D.K);
    return a;
 }
 
@@ -819,8 +866,9 @@ int plan_m2(bsahip_plan *P)
    const size_t nm2 = (size_t)D.nm * D.nm;
    const int nby = (P->nh + 63) / 64, mt = D.nm <= 16 ? 1 : 2;
    if (!P->m2part) CHK(fill(P->m2, 3 * nm2, 0.0));
-   const dim3 gm((unsigned)D.nm, (unsigned)nby, (unsigned)((D.nm + 16 * mt - 1) / (16 * mt)));
    const M2Args a = plan_m2_args(P);
+   const dim3 gm((unsigned)D.nm, (unsigned)nby,
+                 (unsigned)(((D.nm + 16 * mt - 1) / (16 * mt)) * ((D.K + a.kper - 1) / a.kper)));
    if (mt == 1) k_m2<1><<<gm, 256, 0, g.s>>>(a);
    else k_m2<2><<<gm, 256, 0, g.s>>>(a);
    HIPC(hipGetLastError());
@@ -1018,35 +1066,47 @@ int bsahip_classic_run_noalloc(const bsahip_problem *p, int32_t nfh, double df, 
 
 namespace {
 
-// Tables of the ONLY_DIAG model on the half grid u df, u < nh: X (K, nh) the
-// nodal PSDs, T (nm, nh, nh) the per-mode GEMM T_m = S W_m S^T (when with_T),
-// H (nm, 2 nh - 1) the FRFs.
-int diag_tables(Bufs &B, const Prob &D, int nh, double df, bool with_T, double **X, double **T,
-                double2 **H)
+// Tables of the ONLY_DIAG model on the half grid u df, u < nh: X (K, ldX) the nodal
+// PSDs, W and A2 (nm, K) the weights Psi_q Psi_l^2 and Psi_l^2, H (nm, 2 nh - 1) the FRFs.
+struct DiagTab {
+   double *X, *W, *A2;
+   double2 *H;
+   long ldX;
+};
+
+int diag_tables(Bufs &B, const Prob &D, int nh, double df, DiagTab &T)
 {
    const int nft = 2 * nh - 1, nm = D.nm, K = D.K;
    std::vector<double> fl(nh);
    for (int u = 0; u < nh; ++u) fl[u] = (double)u * df;
-   double *dfl, *sq, *Y;
+   double *dfl;
+   T.ldX = round_up(nh, 128);
    CHK(upload(B, "fl", fl, &dfl));
-   CHK(B.get("sq", (size_t)D.ntc * nh * D.nnl, &sq));
-   CHK(B.get("dg_X", (size_t)K * nh, X));
-   CHK(B.get("dg_Y", (size_t)nm * K * nh, &Y));
-   CHK(B.get("dg_H", (size_t)nm * nft, H));
-   dim3 gp((D.nnl + 63) / 64, nh, D.ntc);
-   k_psd_sqrt<<<gp, 64, 0, g.s>>>(dfl, nh, D.prm, D.formula, D.nnl, D.ntc, D.pulsation, sq);
+   CHK(B.get("dg_X", (size_t)K * T.ldX, &T.X));
+   CHK(B.get("dg_W", (size_t)nm * K, &T.W));
+   CHK(B.get("dg_A2", (size_t)nm * K, &T.A2));
+   CHK(B.get("dg_H", (size_t)nm * nft, &T.H));
+   k_diag_psd<<<dim3((unsigned)((T.ldX + 63) / 64), (unsigned)K), 64, 0, g.s>>>(
+      dfl, nh, D.nnl, D.kv, D.prm, D.formula, D.pulsation, T.ldX, T.X);
    HIPC(hipGetLastError());
-   k_diag_tables<<<dim3((unsigned)((nh + 63) / 64), (unsigned)K), 64, 0, g.s>>>(
-      sq, nh, D.nnl, D.kv, D.pa_k, D.pb_k, K, nm, *X, Y);
+   const long n = (long)nm * K;
+   k_diag_weights<<<(unsigned)((n + 255) / 256), 256, 0, g.s>>>(D.pa_k, D.pb_k, n, T.W, T.A2);
    HIPC(hipGetLastError());
-   CHK(launch_frf(D, nft, df, *H));
-   *T = nullptr;
-   if (with_T) {
-      CHK(B.get("dg_T", (size_t)nm * nh * nh, T));
-      CHK(dgemm_sb(0, 1, nh, nh, K, 1.0, *X, nh, 0, Y, nh, (long)K * nh, 0.0, *T, nh, (long)nh * nh,
-                   nm));
-   }
-   return 0;
+   return launch_frf(D, nft, df, T.H);
+}
+
+// T (nm, nh, nh) = X W_m X^T per mode, for the bispectra
+int diag_products(Bufs &B, const Prob &D, int nh, const DiagTab &T, double **out)
+{
+   double *Y;
+   const int nm = D.nm, K = D.K;
+   CHK(B.get("dg_Y", (size_t)nm * K * T.ldX, &Y));
+   CHK(B.get("dg_T", (size_t)nm * nh * nh, out));
+   k_diag_scaled<<<dim3((unsigned)((T.ldX + 63) / 64), (unsigned)K, (unsigned)nm), 64, 0, g.s>>>(
+      T.X, T.ldX, T.W, K, Y);
+   HIPC(hipGetLastError());
+   return dgemm_sb(0, 1, nh, nh, K, 1.0, T.X, T.ldX, 0, Y, T.ldX, (long)K * T.ldX, 0.0, *out, nh,
+                   (long)nh * nh, nm);
 }
 
 // The ONLY_DIAG Classic model (diag.hip): outputs have NM entries each.
@@ -1059,31 +1119,60 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
    Bufs &B = oneshot_bufs();
    Prob D;
    CHK(load_problem(p, 0, B, D));
-   const int nh = nfh, nf = 2 * nh - 1, nft = 2 * nh - 1, nm = D.nm, K = D.K;
-   const int rule = (flags & BSAHIP_QUAD_MASK) >> 4;
+   const int nh = nfh, nft = 2 * nh - 1, nm = D.nm, K = D.K;
    const double d = p->pulsation ? df * 2.0 * M_PI : df;
-   double *X, *T, *mom;
-   double2 *H;
-   CHK(diag_tables(B, D, nh, df, !(flags & BSAHIP_NO_BISP), &X, &T, &H));
+   const bool psd = !(flags & BSAHIP_NO_PSD), bisp = !(flags & BSAHIP_NO_BISP);
+   DiagTab T;
+   double *mom;
+   CHK(diag_tables(B, D, nh, df, T));
    CHK(B.get("dg_mom", 5 * (size_t)nm, &mom));
    CHK(fill(mom, 5 * (size_t)nm, 0.0));
    double *m2f = mom, *m2r = mom + nm, *m2o = mom + 2 * nm, *m3f = mom + 3 * nm, *m3r = mom + 4 * nm;
-   if (!(flags & BSAHIP_NO_BISP)) {
-      k_diag_m3<<<dim3((unsigned)nf, (unsigned)nm), 256, 0, g.s>>>(T, nh, H, nft, rule, d * d, m3f, m3r);
+   if (psd) {
+      // beside the third moments, on the side stream
+      HIPC(hipEventRecord(g.e2, g.s));
+      HIPC(hipStreamWaitEvent(g.s2, g.e2, 0));
+      const int nby = (nh + 63) / 64, mt = nm <= 16 ? 1 : 2, np = (nm + 16 * mt - 1) / (16 * mt);
+      M2Args a{T.X, T.ldX, T.A2, K, nm, 0, nh, T.H, nft, d, 2.0 * M_PI * df, m2f, m2r, m2o, nullptr, 1,
+               m2_slice(256, (long)nby * np, K)};
+      const dim3 gm(1, (unsigned)nby, (unsigned)(np * ((K + a.kper - 1) / a.kper)));
+      if (mt == 1) k_m2<1><<<gm, 256, 0, g.s2>>>(a);
+      else k_m2<2><<<gm, 256, 0, g.s2>>>(a);
+      HIPC(hipGetLastError());
+      HIPC(hipEventRecord(g.e3, g.s2));
+   }
+   if (bisp) {
+      GsymArgs a{};
+      a.U = T.X;
+      a.ldU = T.ldX;
+      a.pb = T.W;
+      a.K = K;
+      a.nm = 1;
+      a.nhp = a.nh = a.nu = nh;
+      a.H = T.H;
+      a.nft = nft;
+      a.d2 = d * d;
+      a.rule = (flags & BSAHIP_QUAD_MASK) >> 4;
+      a.epi_plain = (flags & BSAHIP_EPI_GENERIC) ? 1 : 0;
+      a.m3f = m3f;
+      a.m3r = m3r;
+      int br, bc;
+      f64_shape(nh, nm, F64_LEAST_DIAG, br, bc);
+      const long items = f64_tiles(nh, br, bc) * nm;
+      if (items > 0xffffffL)
+         return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: use a coarser grid or fewer modes");
+      if (br == 4) k_gsym_diag<4, 2><<<(unsigned)items, 256, 0, g.s>>>(a, nm);
+      else if (br == 2) k_gsym_diag<2, 2><<<(unsigned)items, 256, 0, g.s>>>(a, nm);
+      else k_gsym_diag<1, 1><<<(unsigned)items, 256, 0, g.s>>>(a, nm);
       HIPC(hipGetLastError());
    }
-   if (!(flags & BSAHIP_NO_PSD)) {
-      k_diag_m2<<<dim3((unsigned)((nh + 63) / 64), (unsigned)nm), 64, 0, g.s>>>(
-         X, nh, D.pa_k, K, H, nft, d, 2.0 * M_PI * df, m2f, m2r, m2o);
-      HIPC(hipGetLastError());
-   }
+   if (psd) HIPC(hipStreamWaitEvent(g.s, g.e3, 0));
    std::vector<double> h(5 * (size_t)nm);
    HIPC(hipMemcpyAsync(h.data(), mom, h.size() * sizeof(double), hipMemcpyDeviceToHost, g.s));
    HIPC(hipStreamSynchronize(g.s));
    auto put = [&](double *dst, int slot, bool on) {
       if (dst && on) std::memcpy(dst, h.data() + (size_t)slot * nm, nm * sizeof(double));
    };
-   const bool psd = !(flags & BSAHIP_NO_PSD), bisp = !(flags & BSAHIP_NO_BISP);
    put(m2mf, 0, psd);
    put(m2mr, 1, psd);
    put(m2o2mr, 2, psd);
@@ -1268,10 +1357,11 @@ int bsahip_classic_bispectra_sel(const bsahip_problem *p, int32_t nfh, double df
    if (brm) CHK(B.get("bisp_sel_r", nout, &orr));
    const dim3 gs((unsigned)((npts + 255) / 256), (unsigned)nsel);
    if (diag) {
-      double *X, *T;
-      double2 *H;
-      CHK(diag_tables(B, D, nh, df, true, &X, &T, &H));
-      k_diag_bisp_sel<<<gs, 256, 0, g.s>>>(T, nh, H, 2 * nh - 1, dsel, ob, orr);
+      DiagTab X;
+      double *T;
+      CHK(diag_tables(B, D, nh, df, X));
+      CHK(diag_products(B, D, nh, X, &T));
+      k_diag_bisp_sel<<<gs, 256, 0, g.s>>>(T, nh, X.H, 2 * nh - 1, dsel, ob, orr);
    } else {
       const int nu = exact ? nf : nh;
       const long ldU = (long)D.nm * nu;

@@ -5,108 +5,55 @@
 // index k = (component, node) and S_k the nodal PSD,
 //   B_m(f1, f2) = 2 sum_k W_m(k) [S_k(f1) S_k(f2) + S_k(f1+f2) S_k(f2) + S_k(f1+f2) S_k(f1)]
 //               = 2 [T_m(|f1|, |f2|) + T_m(|f1+f2|, |f2|) + T_m(|f1+f2|, |f1|)],
-//   T_m(u, v)   = sum_k S_k(u) W_m(k) S_k(v)     (one FP64 GEMM per mode),
+//   T_m(u, v)   = sum_k S_k(u) W_m(k) S_k(v),
 // with S(f1+f2) = 0 beyond +-fmax (the reference's zero padding), and
 // psd_m(f) = sum_k Psi_l^2 S_k(f).  The moments integrate B_m and psd_m with
 // the response factors Re[H_m(f1) H_m(f2) conj H_m(f1+f2)] and |H_m(f)|^2.
+// T_m is G[m](m,u; m,v) of the full model for a structure of that one mode with the
+// table S and Psi_b = W_m: the third moments are its contraction with the plane
+// epilogue (k_gsym_diag), each T value formed once and never stored, and the second
+// moments its modal PSD kernel (k_m2 with diag).  Bound by launches and latency at
+// these sizes: T stored by a GEMM per mode, read back over the whole plane and a
+// serial loop over k per PSD value took 530 us for 20 modes, 1000 nodes and
+// components, 257 frequencies; now 89 us, with the 15 us of k_m2 beside.  Selected bispectra
+// still store their T_m (one GEMM per mode).
 
-// X[k*nh + u] = S_k(u df); Y[(m*K + k)*nh + u] = W_m(k) S_k(u df).
-// grid (ceil(nh/64), K), block 64
-__global__ void k_diag_tables(const double *__restrict__ sq, int nh, int nnl, int kv,
-                              const double *__restrict__ pa, const double *__restrict__ pb, int K,
-                              int nm, double *__restrict__ X, double *__restrict__ Y)
+// X[k*ldX + u] = S_k(u df), zero for u >= nh and in the padding rows k >= kv; from the
+// nodal parameters prm, formula as k_psd_sqrt.  grid (ceil(ldX/64), K), block 64
+__global__ void k_diag_psd(const double *__restrict__ fl, int nh, int nnl, int kv,
+                           const double *__restrict__ prm, const int *__restrict__ formula,
+                           int pulsation, long ldX, double *__restrict__ X)
 {
    const int u = blockIdx.x * 64 + threadIdx.x;
    const int k = blockIdx.y;
-   if (u >= nh) return;
-   const int c = k / nnl, n = k % nnl;                // rows k >= kv are padding
-   const double s = (k < kv) ? sq[((size_t)c * nh + u) * nnl + n] : 0.0;
-   const double S = s * s;
-   X[(size_t)k * nh + u] = S;
-   for (int m = 0; m < nm; ++m) {
-      const double a = pa[(size_t)m * K + k], q = pb[(size_t)m * K + k];
-      Y[((size_t)m * K + k) * nh + u] = q * a * a * S;
-   }
+   if (u >= ldX) return;
+   double s = 0.0;
+   if (k < kv && u < nh) s = psd_sqrt(prm + (size_t)k * 4, formula[k / nnl], fl[u], pulsation);
+   X[(size_t)k * ldX + u] = s * s;
 }
 
-// Third moments of mode m = blockIdx.y over grid row i = blockIdx.x (threads
-// over the columns j), quadrature weight qweight(rule); sums added to m3f[m],
-// m3r[m].  T[m][u + v*nh] symmetric.  grid (nf, nm), block 256
-__global__ __launch_bounds__(256) void k_diag_m3(const double *__restrict__ T, int nh,
-                                                 const double2 *__restrict__ H, int nft, int rule,
-                                                 double d2, double *__restrict__ m3f,
-                                                 double *__restrict__ m3r)
+// W[m*K + k] = Psi_q Psi_l^2, A2[m*K + k] = Psi_l^2
+__global__ void k_diag_weights(const double *__restrict__ pa, const double *__restrict__ pb, long n,
+                               double *__restrict__ W, double *__restrict__ A2)
 {
-   __shared__ double red[2][4];
-   const int m = blockIdx.y;
-   const int n = nh - 1;
-   const int F1 = (int)blockIdx.x - n;
-   const int a1 = abs(F1);
-   const double *Tm = T + (size_t)m * nh * nh;
-   const double2 h1 = hget(H, nft, m, F1);
-   double sf = 0.0, sr = 0.0;
-   for (int j = threadIdx.x; j < 2 * nh - 1; j += 256) {
-      const int F2 = j - n, a2 = abs(F2), s = F1 + F2, as = abs(s);
-      double b = Tm[a1 + (size_t)a2 * nh];
-      if (as <= n) b += Tm[as + (size_t)a2 * nh] + Tm[as + (size_t)a1 * nh];
-      b *= 2.0;
-      const double w = qweight(F1, F2, n, rule, d2);
-      const double r = re3(h1, hget(H, nft, m, F2), hget(H, nft, m, s));
-      sf += w * b;
-      sr += w * b * r;
-   }
-   sf = wave_sum(sf);
-   sr = wave_sum(sr);
-   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-   if (lane == 0) {
-      red[0][wv] = sf;
-      red[1][wv] = sr;
-   }
-   __syncthreads();
-   if (threadIdx.x == 0) {
-      atomicAdd(m3f + m, red[0][0] + red[0][1] + red[0][2] + red[0][3]);
-      atomicAdd(m3r + m, red[1][0] + red[1][1] + red[1][2] + red[1][3]);
-   }
+   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+   if (t >= n) return;
+   const double a = pa[t];
+   W[t] = pb[t] * a * a;
+   A2[t] = a * a;
 }
 
-// Second moments of mode m = blockIdx.y (vectorised rule: every point d, the
-// two ends d/2; +u and -u), psd_m(u) = sum_k Psi_l(m,k)^2 S_k(u).
-// grid (ceil(nh/64), nm), block 64
-__global__ void k_diag_m2(const double *__restrict__ X, int nh, const double *__restrict__ pa,
-                          int K, const double2 *__restrict__ H, int nft, double d, double om_step,
-                          double *__restrict__ m2f, double *__restrict__ m2r,
-                          double *__restrict__ m2o)
+// Y[(m*K + k)*ldX + u] = W_m(k) X[k*ldX + u]; grid (ceil(ldX/64), K, nm), block 64
+__global__ void k_diag_scaled(const double *__restrict__ X, long ldX, const double *__restrict__ W,
+                              int K, double *__restrict__ Y)
 {
-   const int m = blockIdx.y;
    const int u = blockIdx.x * 64 + threadIdx.x;
-   double sf = 0.0, sr = 0.0, so = 0.0;
-   if (u < nh) {
-      double v = 0.0;
-      for (int k = 0; k < K; ++k) {
-         const double a = pa[(size_t)m * K + k];
-         v = fma(a * a, X[(size_t)k * nh + u], v);
-      }
-      double w = (u == nh - 1) ? 0.5 * d : d;
-      if (u > 0) w *= 2.0;
-      const double2 h = H[(size_t)m * nft + u];
-      const double fr = h.x * h.x + h.y * h.y;
-      const double om = om_step * u;
-      sf = w * v;
-      sr = w * v * fr;
-      so = w * v * fr * om * om;
-   }
-   sf = wave_sum(sf);
-   sr = wave_sum(sr);
-   so = wave_sum(so);
-   if (threadIdx.x == 0) {
-      if (m2f) atomicAdd(m2f + m, sf);
-      if (m2r) atomicAdd(m2r + m, sr);
-      if (m2o) atomicAdd(m2o + m, so);
-   }
+   const int k = blockIdx.y, m = blockIdx.z;
+   if (u < ldX) Y[((size_t)m * K + k) * ldX + u] = W[(size_t)m * K + k] * X[(size_t)k * ldX + u];
 }
 
-// Diagonal bispectra of selected modes on the Classic grid from T, the terms
-// of k_diag_m3: out[q1 + nf*q2 + nf*nf*s] for mode sel[s] (the reference's
+// Diagonal bispectra of selected modes on the Classic grid from T, by the
+// formula of B_m above: out[q1 + nf*q2 + nf*nf*s] for mode sel[s] (the reference's
 // bisp(i, j, m) of getFM_diag_tnlm_vect_cls_ / getRM_diag_vect_cls_).
 // grid (ceil(nf*nf/256), nsel), block 256
 __global__ __launch_bounds__(256) void k_diag_bisp_sel(const double *__restrict__ T, int nh,

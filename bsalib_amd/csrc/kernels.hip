@@ -19,10 +19,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-#define KC 32          // K chunk staged in LDS by k_gsym_f64
-#define TILE 64        // G tile edge (rows (y,u) x cols (z,v))
+#define KC 32          // table K rows are padded to a multiple of this
 
 // ---------------------------------------------------------------------------
 // small helpers
@@ -416,8 +417,6 @@ struct GsymArgs {
    int nm, nhp, nh;       // modes, rows per mode, half-grid points of the plane
    int nu;                // table rows holding A (nh, or 2nh-1 when S(f1+f2)
                           // is evaluated beyond the plane)
-   int ntile;             // tiles per side
-   long npairs;           // ntile*(ntile+1)/2
    const double2 *H;      // [nm][nft]
    int nft;               // >= 2*nu - 1
    double d2;             // (2 pi df)^2 or df^2
@@ -448,39 +447,257 @@ __device__ __forceinline__ double qw(bool ep, bool op, bool eq, bool oq, const Q
    return (op || oq) ? 0.0 : ((ep && eq) ? r.c_corner : ((ep || eq) ? r.c_edge : 1.0));
 }
 
-// Plane epilogue of one 16x16 block of G[x] values (rows r0.., cols q0..),
-// mode rows y and cols z fixed per block.  Each lane holds four values of
-// column q0 + lane%16, rows given by the MFMA accumulator layout: interleaved
-// (f64: (l/16) + 4t) or grouped (f32 outputs: 4(l/16) + t).  Adds 2*G times
-// the quadrature weight / d^2 and the FRF product to nine per-lane sums:
+// Plane epilogue.  A G value G[x](y,u; z,v) enters the moments at up to twelve
+// (m,n,p,f1,f2) places; per lane they make nine sums:
 //   s0 force (x,y,z)=(x,z,y)  s1 resp (x,y,z)  s2 force (y,x,z)=(y,z,x)
 //   s3 resp (y,x,z)  s4 resp (y,z,x)  s5 resp (x,z,y)
 //   s6 force (z,x,y)=(z,y,x)  s7 resp (z,x,y)  s8 resp (z,y,x)
-// (transposed entries s5..s8 only when !DIAG; a compile-time flag keeps the
-// four rows of a lane in one basic block, so their loads can overlap).
-// Re[a b conj c] is unchanged when all three factors are conjugated, so of the
-// eight FRF products these sums weight only four differ:
-//   (y,z,x) at (v,u-v):  Re[H_y(v) H_z(u-v) conj H_x(u)]       = F1o
-//   (y,z,x) at (-v,u+v): Re[conj H_y(v) H_z(u+v) conj H_x(u)]  = F1s
-//   (z,y,x) at (u,v-u):  Re[H_z(u) H_y(v-u) conj H_x(v)]       = F2s
-//   (z,y,x) at (-u,u+v): Re[conj H_z(u) H_y(u+v) conj H_x(v)]  = F2o
-template <bool DIAG>
-__device__ __forceinline__ void epi_accum(const GsymArgs &a, int x, int y, int z, int ur0,
-                                          int vq0, int lane, const double (&gval)[4],
-                                          bool interleaved, double (&s)[9])
+// (s5..s8 and the second entry of s0 only off the tile diagonal).  Re[a b conj c] does
+// not change when all three factors are conjugated, so of the eight FRF products that
+// weight them four differ:
+//   F1s = Re[H_x(u) H_y(v) conj H_z(u+v)]         F1o = Re[H_x(u) conj H_y(v) conj H_z(u-v)]
+//   F2s = Re[H_y(u-v) H_x(v) conj H_z(u)]         F2o = Re[H_y(u+v) conj H_x(v) conj H_z(u)]
+// and with the sign multiplicities ms, mo of (+-u, +-v) and the weights W of the places
+//   s0 += g Wa (ms + mo)            s1 += g Wa (ms F1s + mo F1o)
+//   s2 += g (ms Wb + mo Wd)         s3 += g (ms Wb F2s + mo Wd F2o)
+//   s4 += g (ms Wb F1o + mo Wd F1s) s5 += g Wa (ms F2o + mo F2s)
+//   s6 += g (ms We + mo Wf)         s7 += g (ms We F1o + mo Wf F1s)
+//   s8 += g (ms We F2s + mo Wf F2o)
+// Wa = w(u,v), Wb = w(|u-v|,v), Wd = w(u+v,v), We = w(|u-v|,u), Wf = w(u+v,u).  H(0) is
+// real, so at u = 0 or v = 0 the s and the o terms are equal and the multiplicities (2, 0)
+// and (1, 0) act as (1, 1) and (1/2, 1/2): a factor 1/2 on g per zero.  All sums are
+// kept in units of 4 g (interior multiplicity 2, B = 2 G).
+//
+// Each 16x16 block is handled by its class, uniform per wave (epi_class):
+//   1  u, v < n and u + v < n: every weight 1
+//   2  u, v < n and u + v > n: Wd = Wf = 0
+//   3  u + v on both sides of n, or with the edge u = n or v = n
+//   4  holds (n,n), (n,0) or (0,n), where two edges meet, or lies beyond the plane
+//      (SUM_EXACT): every weight by the rule, qw()
+// In classes 1 to 3 one factor each of u and of v goes onto g: 1/2 at 0, the edge weight
+// c at n, 0 for rows (columns) of another mode.  That is Wa; Wb and Wd have no factor of
+// u and We and Wf none of v, so the row u = n gets the missing (1 - c) of s2..s4 by itself
+// (w(u+v) is 0 there) and the column v = n its s6..s8 divided by c.  The sums over a lane's
+// rows are taken before the factors of its column: sum h H_x(u) conj H_z(u+v) first,
+// H_y(v) once per column block (21 FP64 instructions per value of class 1 instead of 33).
+// The FRF values at u+v and u-v are read from a window in LDS, those of the rows
+// broadcast from registers (a lane of each 16-lane row holds one row's).  With one
+// window load per value and two passes (interior, then edges point by point) the BF16x3
+// kernel took 842 us at 333 nodes, 17 modes, 193 frequencies and 208 us at 40, 20, 65,
+// now 741 and 150, of which 388 and 21 are the contraction.
+
+// FRF values of a wave's (y, z) pair in LDS, indexed by the offset from its origin
+// (ub, vb) within the modes (either may be negative; entries of points outside the modes
+// are never used):
+//   [0, 128)   H_z(u+v)      at u+v - (ub+vb)
+//   [128, 256) H_y(u+v)      at u+v - (ub+vb)
+//   [256, 384) H_y(u-v)      at u-v - (ub-vb-16BC+1), conjugated for u < v
+//   [384, 512) H_z(u-v)      likewise
+//   [512, 576) H_x(u), [576, 640) H_z(u)   at u - ub
+//   [640, 704) H_x(v), [704, 768) H_y(v)   at v - vb
+template <int BR, int BC>
+__device__ __forceinline__ void epi_window(const GsymArgs &a, int x, int y, int z, int ub, int vb,
+                                           int lane, double2 *win)
 {
-   const int n = a.nh - 1;
-   const QRule qr = qrule(a.rule);
+   constexpr int NS = 16 * (BR + BC);
+   static_assert(NS <= 128 && 16 * BR <= 64 && 16 * BC <= 64, "FRF windows of 128 and 64 entries");
    const double2 *Hx = a.H + (size_t)x * a.nft;
    const double2 *Hy = a.H + (size_t)y * a.nft;
    const double2 *Hz = a.H + (size_t)z * a.nft;
-   // branch-free over the lanes: out-of-range rows/columns read row/column 0
-   // and contribute with weight 0 (divergent exits would make the compiler
-   // copy the nine accumulators at every join)
+   const int wsb = ub + vb, wdb = ub - vb - (16 * BC - 1);
+   // the previous pair's reads before these writes
+   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+   __builtin_amdgcn_wave_barrier();
+   for (int e = lane; e < NS; e += 64) {
+      const int sp = min(abs(wsb + e), a.nft - 1);
+      const int dm = wdb + e;
+      const int ad = min(abs(dm), a.nft - 1);
+      double2 hym = Hy[ad], hzm = Hz[ad];
+      if (dm < 0) {
+         hym.y = -hym.y;
+         hzm.y = -hzm.y;
+      }
+      win[e] = Hz[sp];
+      win[128 + e] = Hy[sp];
+      win[256 + e] = hym;
+      win[384 + e] = hzm;
+   }
+   if (lane < 16 * BR) {
+      const int u = min(max(ub + lane, 0), a.nft - 1);
+      win[512 + lane] = Hx[u];
+      win[576 + lane] = Hz[u];
+   }
+   if (lane < 16 * BC) {
+      const int v = min(max(vb + lane, 0), a.nft - 1);
+      win[640 + lane] = Hx[v];
+      win[704 + lane] = Hy[v];
+   }
+   // the wave's own LDS writes before its reads (other waves never touch it)
+   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+   __builtin_amdgcn_wave_barrier();
+   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Class of the 16x16 block at (u0, v0) within the modes, see above.
+__device__ __forceinline__ int epi_class(const GsymArgs &a, int u0, int v0)
+{
+   const int n = a.nh - 1;
+   const bool ue = u0 + 15 >= n, ve = v0 + 15 >= n;
+   if (a.epi_plain || (a.nu != a.nh && (ue || ve))) return 4;
+   if ((ue && (ve || v0 <= 0)) || (ve && u0 <= 0)) return 4;
+   if (ue || ve) return 3;
+   if (u0 + v0 + 30 <= n - 1) return 1;
+   return u0 + v0 >= n + 1 ? 2 : 3;
+}
+
+// broadcast within each 16-lane row from its lane C
+template <int C>
+__device__ __forceinline__ double row_bcast(double v)
+{
+   const long b = __double_as_longlong(v);
+   const int lo = __builtin_amdgcn_mov_dpp((int)b, 0x150 + C, 0xf, 0xf, true);
+   const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0x150 + C, 0xf, 0xf, true);
+   return __longlong_as_double(((long)hi << 32) | (unsigned)lo);
+}
+
+// Sums of a column block (classes 1 to 3) before the column's factors; w: the part of h
+// that w(u+v) leaves to the u + v terms (class 1: all), r: the rest (class 2: all).
+struct EpiZ {
+   double z1wr, z1wi, z1rr, z1ri;      // sum h H_x(u) conj H_z(u+v)
+   double z2r, z2i;                    // sum h H_x(u) conj H_z(u-v)
+   double z3r, z3i;                    // sum h H_y(u-v) conj H_z(u)
+   double z4wr, z4wi, z4rr, z4ri;      // sum h H_y(u+v) conj H_z(u)
+   double hw, hr;                      // sum h
+};
+
+// Value T of row block I, column block at window offsets ps (u+v) and pd (u-v), class 1,
+// 2 or 3 (w: w(u+v)).  rx, rz: the lane's row of H_x(u), H_z(u) (lane c = 4 i + t of each
+// 16-lane row holds row register t of block i).  ST: u step of the row registers.
+template <int CLS, int I, int T, int ST>
+__device__ __forceinline__ void epi_value(const double2 *ps, const double2 *pd, double h, double w,
+                                          const double2 &rx, const double2 &rz, EpiZ &Z)
+{
+   const double2 hzs = ps[ST * T], hys = ps[128 + ST * T];
+   const double2 hyd = pd[ST * T], hzd = pd[128 + ST * T];
+   const double xr = h * row_bcast<4 * I + T>(rx.x), xi = h * row_bcast<4 * I + T>(rx.y);
+   const double zr = h * row_bcast<4 * I + T>(rz.x), zi = h * row_bcast<4 * I + T>(rz.y);
+   if constexpr (CLS == 1) {
+      Z.z1wr = fma(xi, hzs.y, fma(xr, hzs.x, Z.z1wr));
+      Z.z1wi = fma(-xr, hzs.y, fma(xi, hzs.x, Z.z1wi));
+      Z.z4wr = fma(zi, hys.y, fma(zr, hys.x, Z.z4wr));
+      Z.z4wi = fma(-zi, hys.x, fma(zr, hys.y, Z.z4wi));
+      Z.hw += h;
+   } else if constexpr (CLS == 2) {
+      Z.z1rr = fma(xi, hzs.y, fma(xr, hzs.x, Z.z1rr));
+      Z.z1ri = fma(-xr, hzs.y, fma(xi, hzs.x, Z.z1ri));
+      Z.z4rr = fma(zi, hys.y, fma(zr, hys.x, Z.z4rr));
+      Z.z4ri = fma(-zi, hys.x, fma(zr, hys.y, Z.z4ri));
+      Z.hr += h;
+   } else {
+      const double r = 1.0 - w;
+      const double p1r = fma(xi, hzs.y, xr * hzs.x), p1i = fma(-xr, hzs.y, xi * hzs.x);
+      const double p4r = fma(zi, hys.y, zr * hys.x), p4i = fma(-zi, hys.x, zr * hys.y);
+      Z.z1wr = fma(w, p1r, Z.z1wr);
+      Z.z1wi = fma(w, p1i, Z.z1wi);
+      Z.z4wr = fma(w, p4r, Z.z4wr);
+      Z.z4wi = fma(w, p4i, Z.z4wi);
+      Z.z1rr = fma(r, p1r, Z.z1rr);
+      Z.z1ri = fma(r, p1i, Z.z1ri);
+      Z.z4rr = fma(r, p4r, Z.z4rr);
+      Z.z4ri = fma(r, p4i, Z.z4ri);
+      Z.hw = fma(w, h, Z.hw);
+      Z.hr = fma(r, h, Z.hr);
+   }
+   Z.z2r = fma(xi, hzd.y, fma(xr, hzd.x, Z.z2r));
+   Z.z2i = fma(-xr, hzd.y, fma(xi, hzd.x, Z.z2i));
+   Z.z3r = fma(zi, hyd.y, fma(zr, hyd.x, Z.z3r));
+   Z.z3i = fma(-zi, hyd.x, fma(zr, hyd.y, Z.z3i));
+}
+
+// Row block I of a column block, class cls 1 to 3; win, ub, wdb: the wave's window.
+template <int I, int ST>
+__device__ __forceinline__ void epi_rows(const GsymArgs &a, int cls, int ur0, int vq0, int lane,
+                                         const double (&g)[4], const double2 *ps, const double2 *pd,
+                                         const double2 &rx, const double2 &rz, EpiZ &Z, double (&s)[9],
+                                         const double2 *win, int ub, int vb)
+{
+   const int n = a.nh - 1;
+   const double ce = qrule(a.rule).c_edge;
+   double h[4] = {g[0], g[1], g[2], g[3]};
+   const int v = vq0 + (lane & 15), ul = ur0 + (ST == 4 ? lane >> 4 : 4 * (lane >> 4));
+   if (ur0 <= 0 || vq0 <= 0 || ur0 + 15 >= n || vq0 + 15 >= n) {       // uniform
+      const bool vok = v >= 0 && v <= n;
+      const double fv = v == 0 ? 0.5 : (v == n ? ce : 1.0);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+         const int u = ul + ST * t;
+         const double fu = u == 0 ? 0.5 : (u == n ? ce : 1.0);
+         h[t] = vok && u >= 0 && u <= n ? h[t] * (fu * fv) : 0.0;
+      }
+      if (ur0 + 15 >= n && ce != 1.0) {
+         // the row u = n: one register of one lane group
+         const int rn = n - ur0, tn = ST == 4 ? rn >> 2 : rn & 3, kn = ST == 4 ? rn & 3 : rn >> 2;
+         const double gn = tn == 0 ? g[0] : (tn == 1 ? g[1] : (tn == 2 ? g[2] : g[3]));
+         const double c = vok && lane >> 4 == kn ? gn * (fv * (1.0 - ce)) : 0.0;
+         const double2 hxn = win[512 + n - ub], hzn = win[576 + n - ub];
+         const double2 hxv = win[640 + v - vb], hyv = win[704 + v - vb];
+         const double2 hyd = pd[n - ul], hzd = pd[128 + n - ul];
+         s[2] += c;
+         s[3] += c * re3(hyd, hxv, hzn);
+         s[4] += c * re3(hxn, make_double2(hyv.x, -hyv.y), hzd);
+      }
+   }
+   if (cls == 1) {
+      epi_value<1, I, 0, ST>(ps, pd, h[0], 1.0, rx, rz, Z);
+      epi_value<1, I, 1, ST>(ps, pd, h[1], 1.0, rx, rz, Z);
+      epi_value<1, I, 2, ST>(ps, pd, h[2], 1.0, rx, rz, Z);
+      epi_value<1, I, 3, ST>(ps, pd, h[3], 1.0, rx, rz, Z);
+   } else if (cls == 2) {
+      epi_value<2, I, 0, ST>(ps, pd, h[0], 0.0, rx, rz, Z);
+      epi_value<2, I, 1, ST>(ps, pd, h[1], 0.0, rx, rz, Z);
+      epi_value<2, I, 2, ST>(ps, pd, h[2], 0.0, rx, rz, Z);
+      epi_value<2, I, 3, ST>(ps, pd, h[3], 0.0, rx, rz, Z);
+   } else {
+      const int s0 = ul + v;
+      double w[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) w[t] = s0 + ST * t < n ? 1.0 : (s0 + ST * t == n ? ce : 0.0);
+      epi_value<3, I, 0, ST>(ps, pd, h[0], w[0], rx, rz, Z);
+      epi_value<3, I, 1, ST>(ps, pd, h[1], w[1], rx, rz, Z);
+      epi_value<3, I, 2, ST>(ps, pd, h[2], w[2], rx, rz, Z);
+      epi_value<3, I, 3, ST>(ps, pd, h[3], w[3], rx, rz, Z);
+   }
+}
+
+// Adds the nine contributions of one value: gas, gao weigh the (u, +-v) places, gbs, gdo
+// those at |u-v|, u+v with v, ges, gfo with u (units of 4 g).
+__device__ __forceinline__ void epi_nine(double (&s)[9], double gas, double gao, double gbs, double gdo,
+                                         double ges, double gfo, double F1s, double F1o, double F2s,
+                                         double F2o)
+{
+   s[0] += gas + gao;
+   s[1] += gas * F1s + gao * F1o;
+   s[2] += gbs + gdo;
+   s[3] += gbs * F2s + gdo * F2o;
+   s[4] += gbs * F1o + gdo * F1s;
+   s[5] += gas * F2o + gao * F2s;
+   s[6] += ges + gfo;
+   s[7] += ges * F1o + gfo * F1s;
+   s[8] += ges * F2s + gfo * F2o;
+}
+
+// Block of class 4: every weight of every point by the rule, FRF values from the window.
+template <int ST>
+__device__ __forceinline__ void epi_rule(const GsymArgs &a, int ur0, int vq0, int lane,
+                                         const double (&gval)[4], double (&s)[9], const double2 *win,
+                                         int ub, int vb, int wdb)
+{
+   const int n = a.nh - 1;
+   const QRule qr = qrule(a.rule);
    const int vr = vq0 + (lane & 15);
-   const bool vok = vr >= 0 && vr < a.nu;          // a block may start in the previous mode
-   const int v = vok ? vr : 0;
-   const double2 hxv = Hx[v], hyv = Hy[v];
+   const bool vok = vr >= 0 && vr < a.nu;
+   const int v = vok ? vr : max(vb, 0);                      // a column of the window
+   const double2 hxv = win[640 + v - vb], hyv = win[704 + v - vb];
    const double2 cyv = make_double2(hyv.x, -hyv.y);
    const double2 cxv = make_double2(hxv.x, -hxv.y);
    const bool ev = (v == n), ov = (v > n);
@@ -488,378 +705,199 @@ __device__ __forceinline__ void epi_accum(const GsymArgs &a, int x, int y, int z
    for (int t = 0; t < 4; ++t) {
       // rows past the mode's last row (the next mode's rows, or padding) add
       // nothing: stop once the lowest row of this register is one of them (uniform)
-      if (ur0 + (interleaved ? 4 * t : t) >= a.nu) break;
-      const int ur = ur0 + (interleaved ? ((lane >> 4) + 4 * t) : (4 * (lane >> 4) + t));
+      if (ur0 + ST * t >= a.nu) break;
+      const int ur = ur0 + (ST == 4 ? lane >> 4 : 4 * (lane >> 4)) + ST * t;
       const bool ok = vok && ur >= 0 && ur < a.nu;
-      const int u = ok ? ur : 0;
-      const double g = ok ? 2.0 * gval[t] : 0.0;   // B = 2 * sum of the three G terms
-      const double ms = (u == 0 && v == 0) ? 1.0 : 2.0;
-      const double mo = (u > 0 && v > 0) ? 2.0 : 0.0;
-      const int sp = u + v;
-      const int dm = u - v;
-      const int ad = dm < 0 ? -dm : dm;
-      const double2 hxu = Hx[u], hzu = Hz[u], hyp = Hy[sp], hzp = Hz[sp];
-      double2 hym = Hy[ad], hzm = Hz[ad];
-      if (dm < 0) {
-         hym.y = -hym.y;
-         hzm.y = -hzm.y;
-      }
-      const bool eu = (u == n), ou = (u > n), es = (sp == n), os = (sp > n);
-      const bool ed = (ad == n), od = (ad > n);
-      const double Wa = qw(eu, ou, ev, ov, qr);
-      const double Wb = qw(ed, od, ev, ov, qr);
-      const double Wd = qw(es, os, ev, ov, qr);
-      // FRF products Re[H_m(f1) H_n(f2) conj H_p(f1+f2)]; Re[conj w] = Re[w]
-      // makes the other eight of the twelve contributions reuse these four:
-      const double F1s = re3(hxu, hyv, hzp);      // (x,y,z) at (u,v);    = (z,x,y) at (v+u,-u)
-      const double F1o = re3(hxu, cyv, hzm);      // (x,y,z) at (u,-v)
-      const double F2s = re3(hym, hxv, hzu);      // (y,x,z) at (u-v,v);  = (x,z,y) at (v,-u)
-      const double F2o = re3(hyp, cxv, hzu);      // (y,x,z) at (u+v,-v); = (x,z,y) at (v,u)
-      const double ga = g * Wa, gbs = ms * g * Wb, gdo = mo * g * Wd;
-      s[0] += ga * (ms + mo);
-      s[1] += ga * (ms * F1s + mo * F1o);
-      s[2] += gbs + gdo;
-      s[3] += gbs * F2s + gdo * F2o;
-      s[4] += gbs * F1o + gdo * F1s;
-      if constexpr (!DIAG) {
-         const double We = qw(ed, od, eu, ou, qr);
-         const double Wf = qw(es, os, eu, ou, qr);
-         const double ges = ms * g * We, gfo = mo * g * Wf;
-         s[5] += ga * (ms * F2o + mo * F2s);
-         s[6] += ges + gfo;
-         s[7] += ges * F1o + gfo * F1s;
-         s[8] += ges * F2s + gfo * F2o;
-      }
-   }
-}
-
-// The same nine sums for a 16x16 block whose every point has the weight of
-// the plane's interior in all five quadrature weights (CLS 1: 1 <= u, v and
-// u + v <= n - 1) or lies beyond the plane's f1+f2 edge with the other four
-// weights interior (CLS 2: u, v <= n - 1 and u + v >= n + 1, so Wd = Wf = 0).
-// CLS 3: the band between them (u, v, |u-v| interior, u + v on both sides of
-// n), where Wd = Wf = w(u+v): 1 below n, the edge weight at n, 0 beyond.
-// With Wa = Wb = We = 1, ms = mo = 2 and h = 2 g = 4 G the contributions of
-// epi_accum reduce to three (CLS 1) or five (CLS 2, 3) distinct sums, kept per
-// block and spread over the nine at its end; no lane is out of range.
-template <int CLS, bool DIAG, bool WIN>
-__device__ __forceinline__ void epi_accum_inner(const GsymArgs &a, int x, int y, int z, int ur0,
-                                                int vq0, int lane, const double (&gval)[4],
-                                                bool interleaved, double (&s)[9],
-                                                const double2 *win, int wub, int wvb, int wdb)
-{
-   const double2 *Hx = a.H + (size_t)x * a.nft;
-   const double2 *Hy = a.H + (size_t)y * a.nft;
-   const double2 *Hz = a.H + (size_t)z * a.nft;
-   const int v = vq0 + (lane & 15);
-   const int wsb = wub + wvb;
-   double2 hxv, hyv;
-   if constexpr (WIN) {
-      hxv = win[640 + v - wvb];
-      hyv = win[704 + v - wvb];
-   } else {
-      hxv = Hx[v];
-      hyv = Hy[v];
-   }
-   const double2 cyv = make_double2(hyv.x, -hyv.y);
-   const double2 cxv = make_double2(hxv.x, -hxv.y);
-   // lh = sum h, lA = sum h (F1s + F1o), lB = sum h F2s (CLS 2), h (F2s + F2o)
-   // (CLS 1) or h (F2s + w F2o) (CLS 3), lC = sum h F1o (CLS 2) or h (F1o + w F1s)
-   // (CLS 3), lD = sum h (F2s + F2o) (CLS 2, 3), lW = sum h w (CLS 3)
-   const int n = a.nh - 1;
-   const double ce = qrule(a.rule).c_edge;
-   double lh = 0.0, lA = 0.0, lB = 0.0, lC = 0.0, lD = 0.0, lW = 0.0;
-#pragma unroll
-   for (int t = 0; t < 4; ++t) {
-      const int u = ur0 + (interleaved ? ((lane >> 4) + 4 * t) : (4 * (lane >> 4) + t));
-      const double h = 4.0 * gval[t];
-      const int sp = u + v;
-      const int dm = u - v;
-      const int ad = dm < 0 ? -dm : dm;
-      double2 hxu, hzu, hzp, hym, hzm;
-      if constexpr (WIN) {                           // the wave's LDS window
-         hxu = win[512 + u - wub];
-         hzu = win[576 + u - wub];
-         hzp = win[sp - wsb];
-         hym = win[256 + dm - wdb];
-         hzm = win[384 + dm - wdb];
-      } else {
-         hxu = Hx[u];
-         hzu = Hz[u];
-         hzp = Hz[sp];
-         hym = Hy[ad];
-         hzm = Hz[ad];
-         if (dm < 0) {
-            hym.y = -hym.y;
-            hzm.y = -hzm.y;
-         }
-      }
-      auto hys = [&]() {                                              // H_y(u+v)
-         if constexpr (WIN) return win[128 + sp - wsb];
-         else return Hy[sp];
-      };
+      const int u = ok ? ur : max(ub, 0);
+      const int sp = u + v, dm = u - v, ad = abs(dm);
+      const double2 hxu = win[512 + u - ub], hzu = win[576 + u - ub];
+      const double2 hzp = win[sp - ub - vb], hyp = win[128 + sp - ub - vb];
+      const double2 hym = win[256 + dm - wdb], hzm = win[384 + dm - wdb];
       const double F1s = re3(hxu, hyv, hzp);
       const double F1o = re3(hxu, cyv, hzm);
       const double F2s = re3(hym, hxv, hzu);
-      lh += h;
-      lA += h * (F1s + F1o);
-      if constexpr (CLS == 1) {
-         const double F2o = re3(hys(), cxv, hzu);
-         lB += h * (F2s + F2o);
-      } else if constexpr (CLS == 2) {
-         lB += h * F2s;
-         lC += h * F1o;
-         if constexpr (!DIAG) {
-            const double F2o = re3(hys(), cxv, hzu);
-            lD += h * (F2s + F2o);
-         }
-      } else {
-         const double w = sp < n ? 1.0 : (sp == n ? ce : 0.0);
-         const double F2o = re3(hys(), cxv, hzu);
-         const double hw = h * w;
-         lW += hw;
-         lB += h * F2s + hw * F2o;
-         lC += h * F1o + hw * F1s;
-         if constexpr (!DIAG) lD += h * (F2s + F2o);
-      }
-   }
-   if constexpr (CLS == 1) {
-      // s0 = s2 = s6 = 2h, s1 = s4 = s7 = h(F1s+F1o), s3 = s5 = s8 = h(F2s+F2o)
-      s[0] += 2.0 * lh;
-      s[1] += lA;
-      s[2] += 2.0 * lh;
-      s[3] += lB;
-      s[4] += lA;
-      if constexpr (!DIAG) {
-         s[5] += lB;
-         s[6] += 2.0 * lh;
-         s[7] += lA;
-         s[8] += lB;
-      }
-   } else if constexpr (CLS == 3) {
-      s[0] += 2.0 * lh;
-      s[1] += lA;
-      s[2] += lh + lW;
-      s[3] += lB;
-      s[4] += lC;
-      if constexpr (!DIAG) {
-         s[5] += lD;
-         s[6] += lh + lW;
-         s[7] += lC;
-         s[8] += lB;
-      }
-   } else {
-      // beyond f1+f2 = fmax: Wd = Wf = 0
-      s[0] += 2.0 * lh;
-      s[1] += lA;
-      s[2] += lh;
-      s[3] += lB;
-      s[4] += lC;
-      if constexpr (!DIAG) {
-         s[5] += lD;
-         s[6] += lh;
-         s[7] += lC;
-         s[8] += lB;
-      }
+      const double F2o = re3(hyp, cxv, hzu);
+      const double g = ok ? 0.5 * gval[t] : 0.0;             // sums in units of 4 g
+      const double ms = (u == 0 && v == 0) ? 1.0 : 2.0;
+      const double mo = (u > 0 && v > 0) ? 2.0 : 0.0;
+      const bool eu = (u == n), ou = (u > n), es = (sp == n), os = (sp > n);
+      const bool ed = (ad == n), od = (ad > n);
+      const double ga = g * qw(eu, ou, ev, ov, qr);
+      const double gas = ms * ga, gao = mo * ga;
+      const double gbs = ms * g * qw(ed, od, ev, ov, qr), gdo = mo * g * qw(es, os, ev, ov, qr);
+      const double ges = ms * g * qw(ed, od, eu, ou, qr), gfo = mo * g * qw(es, os, eu, ou, qr);
+      s[0] += gas + gao;
+      s[1] += gas * F1s + gao * F1o;
+      s[2] += gbs + gdo;
+      s[3] += gbs * F2s + gdo * F2o;
+      s[4] += gbs * F1o + gdo * F1s;
+      s[5] += gas * F2o + gao * F2s;
+      s[6] += ges + gfo;
+      s[7] += ges * F1o + gfo * F1s;
+      s[8] += ges * F2s + gfo * F2o;
    }
 }
 
-// Class of a 16x16 block with half-grid origin (u0, v0): 1, 2 or 3 as above,
-// 0 for every other block (edges of the plane, rows beyond it).
-__device__ __forceinline__ int epi_class(const GsymArgs &a, int u0, int v0)
+// One exchange of epi_flush: of the N values a lane holds it keeps the lower half (or,
+// with its bit `m` set, the upper one), summed with the partner's.
+template <int N, int M>
+__device__ __forceinline__ void epi_halve(double (&v)[9], int lane)
 {
-   const int n = a.nh - 1;
-   if (a.epi_plain || u0 < 1 || v0 < 1 || u0 + 15 > n - 1 || v0 + 15 > n - 1) return 0;
-   if (u0 + v0 + 30 <= n - 1) return 1;
-   if (u0 + v0 >= n + 1) return 2;
-   return 3;
-}
-
-template <bool WIN>
-__device__ __forceinline__ void epi_accum_any(const GsymArgs &a, int x, int y, int z, bool diag,
-                                              int ur0, int vq0, int lane, const double (&g)[4],
-                                              bool interleaved, double (&s)[9],
-                                              const double2 *win, int wub, int wvb, int wdb)
-{
-   const int cls = epi_class(a, ur0, vq0);           // uniform per block
-   if (diag) {
-      if (cls == 1)
-         epi_accum_inner<1, true, WIN>(a, x, y, z, ur0, vq0, lane, g, interleaved, s, win, wub, wvb, wdb);
-      else if (cls == 2)
-         epi_accum_inner<2, true, WIN>(a, x, y, z, ur0, vq0, lane, g, interleaved, s, win, wub, wvb, wdb);
-      else if (cls == 3)
-         epi_accum_inner<3, true, WIN>(a, x, y, z, ur0, vq0, lane, g, interleaved, s, win, wub, wvb, wdb);
-      else
-         epi_accum<true>(a, x, y, z, ur0, vq0, lane, g, interleaved, s);
-   } else {
-      if (cls == 1)
-         epi_accum_inner<1, false, WIN>(a, x, y, z, ur0, vq0, lane, g, interleaved, s, win, wub, wvb, wdb);
-      else if (cls == 2)
-         epi_accum_inner<2, false, WIN>(a, x, y, z, ur0, vq0, lane, g, interleaved, s, win, wub, wvb, wdb);
-      else if (cls == 3)
-         epi_accum_inner<3, false, WIN>(a, x, y, z, ur0, vq0, lane, g, interleaved, s, win, wub, wvb, wdb);
-      else
-         epi_accum<false>(a, x, y, z, ur0, vq0, lane, g, interleaved, s);
+   constexpr int H = (N + 1) / 2;
+   const bool up = (lane & M) != 0;
+#pragma unroll
+   for (int k = 0; k < H; ++k) {
+      const double hi = H + k < N ? v[H + k] : 0.0;
+      const double send = up ? v[k] : hi, keep = up ? hi : v[k];
+      v[k] = keep + __shfl_xor(send, M, 64);
    }
 }
 
-// Wave-reduce the nine sums and add them (times d^2) to the m3 entries, or
-// in the fixed-order mode store them in the wave's slot `f` (the order of the
-// twelve values is the one of the atomics below; bsahip_api.hip builds the
-// matching slot lists, det_slot_lists).
+// Reduce the nine sums over the wave and add them (times 4 d^2) to the m3 entries, or
+// in the fixed-order mode store them in the wave's slot `f` (det_slot_lists of
+// bsahip_api.hip builds the matching lists).  The exchanges halve the values a lane
+// holds as they halve the lanes that share one, 13 instead of 54, and leave sum k on
+// the lanes of one 4-lane group, so that the contributions (slot t: permutation t / 2 of
+// xyz, yxz, yzx, xzy, zxy, zyx; even force, odd response) leave as one atomic.
+// ONE: a structure of one mode, whose twelve contributions meet in two entries.
+template <bool ONE>
 __device__ __forceinline__ void epi_flush(const GsymArgs &a, int x, int y, int z, bool diag,
                                           int lane, double (&s)[9], long sbase, int f)
 {
-   const int nm = a.nm;
-   const size_t nm2 = (size_t)nm * nm;
+   const double d2 = 4.0 * a.d2;
+   if constexpr (ONE) {
+      s[0] = diag ? s[0] + 2.0 * s[2] : 2.0 * (s[0] + s[2] + s[6]);
+      s[1] = diag ? s[1] + s[3] + s[4] : (s[1] + s[3] + s[4]) + (s[5] + s[7] + s[8]);
+      epi_halve<2, 32>(s, lane);
+      const double r = s[0];
+      double q = r;
 #pragma unroll
-   for (int t = 0; t < 9; ++t) s[t] = wave_sum(s[t]) * a.d2;
-   if (a.slots) {
-      if (lane == 0) {
-         double *d = a.slots + sbase + (long)f * 12;
-         d[0] = s[0];
-         d[1] = s[1];
-         d[2] = s[2];
-         d[3] = s[3];
-         d[4] = s[2];
-         d[5] = s[4];
-         if (!diag) {
-            d[6] = s[0];
-            d[7] = s[5];
-            d[8] = s[6];
-            d[9] = s[7];
-            d[10] = s[6];
-            d[11] = s[8];
+      for (int o = 16; o >= 1; o >>= 1) q += __shfl_xor(q, o, 64);
+      if ((lane & 31) == 0) atomicAdd(lane ? a.m3r : a.m3f, q * d2);
+   } else {
+      epi_halve<9, 32>(s, lane);
+      epi_halve<5, 16>(s, lane);
+      epi_halve<3, 8>(s, lane);
+      epi_halve<2, 4>(s, lane);
+      double q = s[0];
+      q += __shfl_xor(q, 2, 64);
+      q += __shfl_xor(q, 1, 64);
+      q *= d2;
+      // value index of the lane's group; groups of padding (a lower half is the larger)
+      const int b5 = lane >> 5, b4 = (lane >> 4) & 1, b3 = (lane >> 3) & 1, b2 = (lane >> 2) & 1;
+      const int k = 5 * b5 + 3 * b4 + 2 * b3 + b2;
+      const bool pad = (b3 && (b4 || b2)) || (b5 && b4 && b2);
+      // slots of value k: {0,6} 1 {2,4} 3 5 7 {8,10} 9 11
+      const int second = lane & 3;
+      int t = -1;
+      if (!pad && second == 0) t = k == 0 ? 0 : (k <= 3 ? k : (k == 4 ? 5 : (k == 5 ? 7 : (k == 6 ? 8 : (k == 7 ? 9 : 11)))));
+      if (!pad && second == 1) t = k == 0 ? 6 : (k == 2 ? 4 : (k == 6 ? 10 : -1));
+      if (t >= 0 && !(diag && t >= 6)) {
+         if (a.slots) {
+            a.slots[sbase + (long)f * 12 + t] = q;
+         } else {
+            const int p = t >> 1;
+            const int i0 = p == 0 || p == 3 ? x : (p == 1 || p == 2 ? y : z);
+            const int i1 = p == 0 || p == 5 ? y : (p == 1 || p == 4 ? x : z);
+            const int i2 = p == 0 || p == 1 ? z : (p == 2 || p == 5 ? x : y);
+            const size_t e = i0 + (size_t)a.nm * (i1 + (size_t)a.nm * i2);
+            atomicAdd((t & 1 ? a.m3r : a.m3f) + e, q);
          }
-      }
-#pragma unroll
-      for (int t = 0; t < 9; ++t) s[t] = 0.0;
-      return;
-   }
-   if (lane == 0) {
-      const size_t i_xyz = x + (size_t)nm * y + nm2 * z;
-      const size_t i_yxz = y + (size_t)nm * x + nm2 * z;
-      const size_t i_yzx = y + (size_t)nm * z + nm2 * x;
-      atomicAdd(a.m3f + i_xyz, s[0]);
-      atomicAdd(a.m3r + i_xyz, s[1]);
-      atomicAdd(a.m3f + i_yxz, s[2]);
-      atomicAdd(a.m3r + i_yxz, s[3]);
-      atomicAdd(a.m3f + i_yzx, s[2]);
-      atomicAdd(a.m3r + i_yzx, s[4]);
-      if (!diag) {
-         const size_t i_xzy = x + (size_t)nm * z + nm2 * y;
-         const size_t i_zxy = z + (size_t)nm * x + nm2 * y;
-         const size_t i_zyx = z + (size_t)nm * y + nm2 * x;
-         atomicAdd(a.m3f + i_xzy, s[0]);
-         atomicAdd(a.m3r + i_xzy, s[5]);
-         atomicAdd(a.m3f + i_zxy, s[6]);
-         atomicAdd(a.m3r + i_zxy, s[7]);
-         atomicAdd(a.m3f + i_zyx, s[6]);
-         atomicAdd(a.m3r + i_zyx, s[8]);
       }
    }
 #pragma unroll
    for (int t = 0; t < 9; ++t) s[t] = 0.0;
 }
 
-// Epilogue of a wave's BR x BC blocks of 16x16 (rows rw0.., cols cw0..): one
-// accumulation / reduction when all blocks share (y,z), else one per (y,z) pair.
-// WIN: win holds 768 double2 of LDS owned by this wave (free after the K loop).
-// When all blocks share (y,z), the FRF values the interior classes read per
-// point are staged there first, each indexed by its offset from the wave's
-// origin (ub, vb) within the modes:
-//   [0, 128)   H_z(u+v)      at u+v - (ub+vb)
-//   [128, 256) H_y(u+v)      at u+v - (ub+vb)
-//   [256, 384) H_y(u-v)      at u-v - (ub-vb-16BC+1), conjugated for u < v
-//   [384, 512) H_z(u-v)      likewise
-//   [512, 576) H_x(u), [576, 640) H_z(u)   at u - ub
-//   [640, 704) H_x(v), [704, 768) H_y(v)   at v - vb
-// (u+v and u-v span 16(BR+BC)-1 <= 127 values over the wave's blocks).
-template <int BR, int BC, bool WIN, class GetVal>
+// Epilogue of a wave's BR x BC blocks of 16x16 (rows rw0.., cols cw0..), one accumulation
+// and reduction per (y, z) mode pair they meet: the rows of consecutive modes are packed,
+// so a block can hold the end of one mode and the start of the next and is then visited
+// for each, the other mode's rows (columns) masked.  win: 768 double2 of LDS owned by this
+// wave.  getv<i>(j, g): values of block (i, j).
+template <int BR, int BC, bool IL, bool ONE, class GetVal>
 __device__ __forceinline__ void epi_wave(const GsymArgs &a, int x, bool diag, int rw0, int cw0,
-                                         int lane, bool interleaved, long sbase, GetVal getv,
-                                         double2 *win)
+                                         int lane, long sbase, GetVal getv, double2 *win)
 {
-   static_assert(16 * (BR + BC) - 1 <= 128 && 16 * BR <= 64 && 16 * BC <= 64,
-                 "FRF windows of 128 and 64 entries");
+   constexpr int ST = IL ? 4 : 1;
    const int nm = a.nm;
    int f = 0;                                         // flushes of this wave so far
-   const int y0 = rw0 / a.nhp, y1 = (rw0 + 16 * BR - 1) / a.nhp;
-   const int z0 = cw0 / a.nhp, z1 = (cw0 + 16 * BC - 1) / a.nhp;
-   double s[9];
+   const int y0 = rw0 / a.nhp, y1 = min((rw0 + 16 * BR - 1) / a.nhp, nm - 1);
+   const int z0 = cw0 / a.nhp, z1 = min((cw0 + 16 * BC - 1) / a.nhp, nm - 1);
+   const int lr = lane & 15, lk = lane >> 4;
+#pragma unroll 1
+   for (int y = y0; y <= y1; ++y)
+#pragma unroll 1
+      for (int z = z0; z <= z1; ++z) {
+         const int ub = rw0 - y * a.nhp, vb = cw0 - z * a.nhp;
+         const int wdb = ub - vb - (16 * BC - 1);
+         epi_window<BR, BC>(a, x, y, z, ub, vb, lane, win);
+         double s[9];
 #pragma unroll
-   for (int t = 0; t < 9; ++t) s[t] = 0.0;
-   if (y0 == y1 && z0 == z1) {
-      if (y0 >= nm || z0 >= nm) return;
-      const int ub = rw0 - y0 * a.nhp, vb = cw0 - z0 * a.nhp;
-      const int wsb = ub + vb, wdb = ub - vb - (16 * BC - 1);
-      if constexpr (WIN) {
-         const double2 *Hy = a.H + (size_t)y0 * a.nft;
-         const double2 *Hz = a.H + (size_t)z0 * a.nft;
-         for (int e = lane; e < 128; e += 64) {
-            const int sp = min(wsb + e, a.nft - 1);   // entries past the wave's range unused
-            const int dm = wdb + e;
-            const int ad = min(dm < 0 ? -dm : dm, a.nft - 1);
-            double2 hym = Hy[ad], hzm = Hz[ad];
-            if (dm < 0) {
-               hym.y = -hym.y;
-               hzm.y = -hzm.y;
+         for (int t = 0; t < 9; ++t) s[t] = 0.0;
+         // row values of this lane: row register lr % 4 of block lr / 4 (of its lk group)
+         const int rr = min(16 * (lr >> 2) + (IL ? lk + 4 * (lr & 3) : 4 * lk + (lr & 3)), 16 * BR - 1);
+         const double2 rx = win[512 + rr], rz = win[576 + rr];
+         const int us = IL ? lk : 4 * lk;                  // u of row register 0 in its block
+         unsigned rule = 0;                                // blocks of class 4
+#pragma unroll 1
+         for (int j = 0; j < BC; ++j) {
+            const int v0 = vb + 16 * j;
+            if (v0 + 15 < 0 || v0 >= a.nu) continue;       // no column of this mode
+            EpiZ Z = {};
+            const double2 *ps = win + us + lr + 16 * j;
+            const double2 *pd = win + 256 + us - lr - 16 * j + 16 * BC - 1;
+            double g[4];
+            auto rows = [&](auto ic) {
+               constexpr int I = decltype(ic)::value;
+               if constexpr (I < BR) {
+                  const int u0 = ub + 16 * I;
+                  if (u0 + 15 < 0 || u0 >= a.nu) return;   // no row of this mode
+                  const int cls = epi_class(a, u0, v0);    // uniform per block
+                  if (cls == 4) {
+                     rule |= 1u << (I * BC + j);
+                     return;
+                  }
+                  getv(ic, j, g);
+                  epi_rows<I, ST>(a, cls, u0, v0, lane, g, ps + 16 * I, pd + 16 * I, rx, rz, Z, s, win, ub, vb);
+               }
+            };
+            rows(std::integral_constant<int, 0>());
+            rows(std::integral_constant<int, 1>());
+            rows(std::integral_constant<int, 2>());
+            rows(std::integral_constant<int, 3>());
+            const double2 hx = win[640 + 16 * j + lr], hy = win[704 + 16 * j + lr];
+            const double a1w = hy.x * Z.z1wr - hy.y * Z.z1wi, a1r = hy.x * Z.z1rr - hy.y * Z.z1ri;
+            const double a2 = hy.x * Z.z2r + hy.y * Z.z2i;
+            const double a3 = hx.x * Z.z3r - hx.y * Z.z3i;
+            const double a4w = hx.x * Z.z4wr + hx.y * Z.z4wi, a4r = hx.x * Z.z4rr + hx.y * Z.z4ri;
+            const double h2 = 2.0 * Z.hw + Z.hr, b1 = a2 + a1w, b3 = a3 + a4w;
+            const double iv = v0 + lr == a.nh - 1 ? 1.0 / qrule(a.rule).c_edge : 1.0;
+            s[0] += 2.0 * (Z.hw + Z.hr);
+            s[1] += b1 + a1r;
+            s[2] += h2;
+            s[3] += b3;
+            s[4] += b1;
+            s[5] += b3 + a4r;
+            s[6] += iv * h2;
+            s[7] += iv * b1;
+            s[8] += iv * b3;
+         }
+         while (rule) {                                    // uniform per wave
+            const int b = __builtin_ctz(rule);
+            rule &= rule - 1;
+            const int i = b / BC, j = b % BC;
+            double g[4];
+            switch (i) {
+            case 0: getv(std::integral_constant<int, 0>(), j, g); break;
+            case 1: if constexpr (BR > 1) getv(std::integral_constant<int, 1>(), j, g); break;
+            case 2: if constexpr (BR > 2) getv(std::integral_constant<int, 2>(), j, g); break;
+            default: if constexpr (BR > 3) getv(std::integral_constant<int, 3>(), j, g); break;
             }
-            win[e] = Hz[sp];
-            win[128 + e] = Hy[sp];
-            win[256 + e] = hym;
-            win[384 + e] = hzm;
+            const int u0 = ub + 16 * i, v0 = vb + 16 * j;
+            epi_rule<ST>(a, u0, v0, lane, g, s, win, ub, vb, wdb);
          }
-         if (lane < 16 * BR) {
-            const double2 *Hx = a.H + (size_t)x * a.nft;
-            win[512 + lane] = Hx[ub + lane];
-            win[576 + lane] = Hz[ub + lane];
-         }
-         if (lane < 16 * BC) {
-            const double2 *Hx = a.H + (size_t)x * a.nft;
-            win[640 + lane] = Hx[vb + lane];
-            win[704 + lane] = Hy[vb + lane];
-         }
-         // the wave's own LDS writes before its reads (other waves never touch it)
-         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-         __builtin_amdgcn_wave_barrier();
-         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+         epi_flush<ONE>(a, x, y, z, diag, lane, s, sbase, f++);
       }
-#pragma unroll 1
-      for (int b = 0; b < BR * BC; ++b) {
-         const int i = b / BC, j = b % BC;
-         double g[4];
-         getv(b, g);
-         epi_accum_any<WIN>(a, x, y0, z0, diag, ub + 16 * i, vb + 16 * j, lane, g, interleaved, s,
-                            win, ub, vb, wdb);
-      }
-      epi_flush(a, x, y0, z0, diag, lane, s, sbase, f++);
-   } else {
-      // the wave's rows (cols) span modes y0..y1 (z0..z1): one reduction per
-      // (y, z) pair over the blocks that meet both.  The rows of consecutive
-      // modes are packed, so a 16-block can hold the end of one mode and the
-      // start of the next: it is visited for each, the rows (cols) of the
-      // other mode masked by the generic epilogue (u < 0 or u >= nu there)
-#pragma unroll 1
-      for (int y = y0; y <= y1; ++y)
-#pragma unroll 1
-         for (int z = z0; z <= z1; ++z) {
-            if (y >= nm || z >= nm) continue;          // uniform per wave
-#pragma unroll 1
-            for (int b = 0; b < BR * BC; ++b) {
-               const int i = b / BC, j = b % BC;
-               const int r0 = rw0 + 16 * i, q0 = cw0 + 16 * j;
-               if (r0 / a.nhp > y || (r0 + 15) / a.nhp < y || q0 / a.nhp > z ||
-                   (q0 + 15) / a.nhp < z)
-                  continue;
-               double g[4];
-               getv(b, g);
-               epi_accum_any<false>(a, x, y, z, diag, r0 - y * a.nhp, q0 - z * a.nhp, lane, g,
-                                    interleaved, s, nullptr, 0, 0, 0);
-            }
-            epi_flush(a, x, y, z, diag, lane, s, sbase, f++);
-         }
-   }
 }
 
 __device__ __forceinline__ void pair_from_index(long t, int &R, int &Q)
@@ -883,95 +921,125 @@ __device__ __forceinline__ long xcd_lid()
    return lid;
 }
 
-// One work item of the FP64 G contraction: mode x, tile pair tp.
-__device__ __forceinline__ void gsym_f64_item(const GsymArgs &a, int x, long tp)
+// Tiles of the FP64 G kernel: waves of 16 BR table rows x 16 BC table columns (BC <= BR),
+// four waves of a workgroup on consecutive column tiles c = 4 Q2 + w and the same rows.
+// With column tiles grouped to the row tile's size, Q = c BC / BR, a wave works when
+// R <= Q (G is symmetric) and treats its block as a diagonal one when R == Q.
+// Item t of a mode: column group Q2, row tile R < rho (Q2 + 1), rho = 4 BC / BR.
+__host__ __device__ inline void f64_tile(long t, int rho, int &Q2, int &R)
 {
-   __shared__ double As[KC][TILE];
-   __shared__ double Bs[KC][TILE];
-   int R, Q;
-   pair_from_index(tp, R, Q);
-   const bool diag = (R == Q);
+   long q = (long)((sqrt(8.0 * (double)(t / rho) + 1.0) - 1.0) * 0.5);
+   while (rho * (q + 1) * (q + 2) / 2 <= t) ++q;
+   while (rho * q * (q + 1) / 2 > t) --q;
+   Q2 = (int)q;
+   R = (int)(t - rho * q * (q + 1) / 2);
+}
 
-   const int tid = threadIdx.x;
-   const int lane = tid & 63;
-   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
-   const int wr = w >> 1, wc = w & 1;
+__host__ __device__ inline long f64_tiles(int rows, int BR, int BC)
+{
+   const long n = (rows + 64 * BC - 1) / (64 * BC);
+   return 4 * BC / BR * n * (n + 1) / 2;
+}
 
-   // staging: each thread moves 8 consecutive doubles of one k row per tile
-   const int sk = tid >> 3;            // 0..31
-   const int so = (tid & 7) * 8;       // 0..56
-   const double *gA = a.U + (size_t)R * TILE + so;
-   const double *gB = a.U + (size_t)Q * TILE + so;
-   const double *pbx = a.pb + (size_t)x * a.K;
-
-   d4 acc[2][2];
+// One wave item of the FP64 G contraction: mode x, tile t.  The operands go from L1 / L2
+// straight into the MFMA fragments (a fragment row is 16 contiguous table rows, 128
+// bytes), D steps of 4 K rows ahead: no LDS, no barrier, so the two waves of a SIMD
+// run out of phase and each hides the other's loads and epilogue.  FP64 MFMA and FP64
+// vector instructions share one pipe (4 fma beside each MFMA cost their 16 cycles on
+// top of its 64), so what is left to win is the vector work: the scaling by Psi_b
+// (BR multiplies per 4 BR BC MFMAs) and the epilogue.  Staged through LDS with two
+// barriers per chunk of 32 K rows it took 254 ms at 1000 nodes, 30 modes, 513
+// frequencies (61 TFLOP/s where bare MFMA reaches 76.9) and 2686 / 259 us at 333, 17,
+// 193 / 40, 20, 65; now 236 ms, of which the epilogue 15, and 2466 / 222 us.
+template <int BR, int BC, bool ONE>
+__device__ __forceinline__ void gsym_f64_wave(const GsymArgs &a, int x, long t)
+{
+   constexpr int D = 4;                                      // K is a multiple of 32 = 8 D
+   __shared__ double2 wins[4 * 768];
+   int Q2, R;
+   f64_tile(t, 4 * BC / BR, Q2, R);
+   const int lane = threadIdx.x & 63;
+   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int c = 4 * Q2 + w, Q = c * BC / BR;
+   if (R > Q || c * 16 * BC >= a.nm * a.nhp) return;         // uniform per wave
+   const int lr = lane & 15, lk = lane >> 4;
+   const double *pA = a.U + (size_t)lk * a.ldU + R * 16 * BR + lr;
+   const double *pB = a.U + (size_t)lk * a.ldU + c * 16 * BC + lr;
+   const double *pbx = a.pb + (size_t)x * a.K + lk;
+   d4 acc[BR][BC];
 #pragma unroll
-   for (int i = 0; i < 2; ++i)
+   for (int i = 0; i < BR; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = (d4){0.0, 0.0, 0.0, 0.0};
-
-   double ra[8], rb[8];
-   double sc;
-   {
-      const double *pA = gA + (size_t)sk * a.ldU;
-      const double *pB = gB + (size_t)sk * a.ldU;
+      for (int j = 0; j < BC; ++j) acc[i][j] = (d4){0.0, 0.0, 0.0, 0.0};
+   double ra[D][BR], rb[D][BC], rp[D];
+   auto load = [&](int d, int k) {
+      const size_t o = (size_t)k * a.ldU;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) { ra[t] = pA[t]; rb[t] = pB[t]; }
-      sc = pbx[sk];
-   }
-   __builtin_amdgcn_s_setprio(1);   // K loop at raised wave priority, as k_gsym_bf16x3
-   for (int k0 = 0; k0 < a.K; k0 += KC) {
-      __syncthreads();
+      for (int i = 0; i < BR; ++i) ra[d][i] = pA[o + 16 * i];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) { As[sk][so + t] = ra[t] * sc; Bs[sk][so + t] = rb[t]; }
-      __syncthreads();
-      if (k0 + KC < a.K) {
-         const double *pA = gA + (size_t)(k0 + KC + sk) * a.ldU;
-         const double *pB = gB + (size_t)(k0 + KC + sk) * a.ldU;
+      for (int j = 0; j < BC; ++j) rb[d][j] = pB[o + 16 * j];
+      rp[d] = pbx[k];
+   };
 #pragma unroll
-         for (int t = 0; t < 8; ++t) { ra[t] = pA[t]; rb[t] = pB[t]; }
-         sc = pbx[k0 + KC + sk];
-      }
+   for (int d = 0; d < D; ++d) load(d, 4 * d);
+   for (int k0 = 0; k0 < a.K; k0 += 4 * D) {
+      const int kn = min(k0 + 4 * D, a.K - 4 * D);           // the last group again at the end: unused
 #pragma unroll
-      for (int kk = 0; kk < KC; kk += 4) {
-         const int kr = kk + (lane >> 4);
-         const double a0 = As[kr][wr * 32 + (lane & 15)];
-         const double a1 = As[kr][wr * 32 + 16 + (lane & 15)];
-         const double b0 = Bs[kr][wc * 32 + (lane & 15)];
-         const double b1 = Bs[kr][wc * 32 + 16 + (lane & 15)];
-         acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-         acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-         acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-         acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
+      for (int d = 0; d < D; ++d) {
+         double fa[BR], fb[BC];
+#pragma unroll
+         for (int i = 0; i < BR; ++i) fa[i] = ra[d][i] * rp[d];
+#pragma unroll
+         for (int j = 0; j < BC; ++j) fb[j] = rb[d][j];
+         load(d, kn + 4 * d);
+#pragma unroll
+         for (int i = 0; i < BR; ++i)
+#pragma unroll
+            for (int j = 0; j < BC; ++j)
+               acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
       }
    }
 
    // ---- epilogue: for v_mfma_f64_16x16x4f64, register t of lane l holds
    // D[(l/16) + 4t][l%16] of its 16x16 block (rows interleaved by 4).
-   const long sbase = ((tp * a.nm + x) * 4 + w) * (long)a.mflush * 12;
-   __builtin_amdgcn_s_setprio(0);
-   epi_wave<2, 2, false>(a, x, diag, R * TILE + wr * 32, Q * TILE + wc * 32, lane, true, sbase,
-                  [&](int b, double (&g)[4]) {
-                     d4 v;
-                     switch (b) {       // uniform branch: constant register indices
-                     case 0: v = acc[0][0]; break;
-                     case 1: v = acc[0][1]; break;
-                     case 2: v = acc[1][0]; break;
-                     default: v = acc[1][1]; break;
-                     }
+   const long sbase = ((t * a.nm + x) * 4 + w) * (long)a.mflush * 12;
+   epi_wave<BR, BC, true, ONE>(a, x, R == Q, R * 16 * BR, c * 16 * BC, lane, sbase,
+                  [&](auto ic, int j, double (&g)[4]) {
+                     constexpr int I = decltype(ic)::value;
 #pragma unroll
-                     for (int t = 0; t < 4; ++t) g[t] = v[t];
+                     for (int q = 0; q < 4; ++q) {
+                        double v = acc[I][0][q], u = acc[I][BC - 1][q];
+                        // opaque: a select of the two addresses would put acc into memory
+                        asm("" : "+v"(v), "+v"(u));
+                        g[q] = j == 0 ? v : u;
+                     }
                   },
-                  nullptr);
+                  wins + w * 768);
 }
 
-// Four workgroups per CU (at most 128 VGPRs: a few spill in the epilogue):
-// more waves hide the barriers and loads of the single-buffered K chunks,
-// 337 -> 277 ms at the deck against two workgroups per CU.
-__global__ __launch_bounds__(256, 4) void k_gsym_f64(GsymArgs a)
+template <int BR, int BC>
+__global__ __launch_bounds__(256, 2) void k_gsym_f64(GsymArgs a)
 {
    const long lid = xcd_lid();
-   gsym_f64_item(a, (int)(lid % a.nm), lid / a.nm);
+   gsym_f64_wave<BR, BC, false>(a, (int)(lid % a.nm), lid / a.nm);
+}
+
+// The ONLY_DIAG model's plane sums: mode x alone, i.e. the contraction and epilogue
+// above for a one-mode structure whose table is the nodal PSDs X, with Psi_b W_x, FRF
+// row x and the moments of mode x.  grid (tiles * nm).  Cutting K into slices that
+// run side by side (the plane sums are linear in G) would fill the chip better at a few
+// hundred nodes, but the slices' sums cancel: 5e-15 of the moments against 1e-15.
+template <int BR, int BC>
+__global__ __launch_bounds__(256, 2) void k_gsym_diag(GsymArgs a, int nmodes)
+{
+   const long lid = blockIdx.x;
+   const int x = (int)(lid % nmodes);
+   GsymArgs b = a;
+   b.pb = a.pb + (size_t)x * a.K;
+   b.H = a.H + (size_t)x * a.nft;
+   b.m3f = a.m3f + x;
+   b.m3r = a.m3r + x;
+   gsym_f64_wave<BR, BC, true>(b, 0, lid / nmodes);
 }
 
 // ---------------------------------------------------------------------------
@@ -1140,15 +1208,15 @@ __device__ __forceinline__ void gsym_bf16x3_item(const GsymArgs &a, const GsymAr
    // last chunk's barrier
    uint4 *plane = w == 0 ? &Ah[0][0] : (w == 1 ? &Al[0][0] : (w == 2 ? &Bh[0][0] : &Bl[0][0]));
    double2 *win = reinterpret_cast<double2 *>(plane);
-   epi_wave<4, 4, true>(a, x, diag, R * T2 + wr * 64, Q * T2 + wc * 64, lane, false, sbase,
-                  [&](int b, double (&g)[4]) {
-                     f4v v;
-                     switch (b) {       // uniform branch: constant register indices
-#define CASE_(k) case k: v = acc[k / 4][k % 4]; break;
-                     CASE_(0) CASE_(1) CASE_(2) CASE_(3) CASE_(4) CASE_(5) CASE_(6) CASE_(7)
-                     CASE_(8) CASE_(9) CASE_(10) CASE_(11) CASE_(12) CASE_(13) CASE_(14)
-#undef CASE_
-                     default: v = acc[3][3]; break;
+   epi_wave<4, 4, false, false>(a, x, diag, R * T2 + wr * 64, Q * T2 + wc * 64, lane, sbase,
+                  [&](auto ic, int j, double (&g)[4]) {
+                     constexpr int I = decltype(ic)::value;
+                     f4v v = acc[I][3];
+                     switch (j) {       // uniform branch: constant register indices
+                     case 0: v = acc[I][0]; break;
+                     case 1: v = acc[I][1]; break;
+                     case 2: v = acc[I][2]; break;
+                     default: break;
                      }
 #pragma unroll
                      for (int t = 0; t < 4; ++t) g[t] = (double)v[t];
@@ -1260,15 +1328,15 @@ __device__ __forceinline__ void gsym_f32_item(const GsymArgs &a, const GsymArgs1
    // each wave's FRF window: 12 KB of the operand planes (2 x 32 KB), free after
    // the last chunk's barrier
    double2 *win = reinterpret_cast<double2 *>(w < 2 ? &As[0][0] : &Bs[0][0]) + (w & 1) * 768;
-   epi_wave<4, 4, true>(a, x, diag, R * T2 + wr * 64, Q * T2 + wc * 64, lane, false, sbase,
-                  [&](int bb, double (&gv)[4]) {
-                     f4v v;
-                     switch (bb) {      // uniform branch: constant register indices
-#define CASE_(k) case k: v = acc[k / 4][k % 4]; break;
-                     CASE_(0) CASE_(1) CASE_(2) CASE_(3) CASE_(4) CASE_(5) CASE_(6) CASE_(7)
-                     CASE_(8) CASE_(9) CASE_(10) CASE_(11) CASE_(12) CASE_(13) CASE_(14)
-#undef CASE_
-                     default: v = acc[3][3]; break;
+   epi_wave<4, 4, false, false>(a, x, diag, R * T2 + wr * 64, Q * T2 + wc * 64, lane, sbase,
+                  [&](auto ic, int j, double (&gv)[4]) {
+                     constexpr int I = decltype(ic)::value;
+                     f4v v = acc[I][3];
+                     switch (j) {       // uniform branch: constant register indices
+                     case 0: v = acc[I][0]; break;
+                     case 1: v = acc[I][1]; break;
+                     case 2: v = acc[I][2]; break;
+                     default: break;
                      }
 #pragma unroll
                      for (int t = 0; t < 4; ++t) gv[t] = (double)v[t];
@@ -1402,10 +1470,12 @@ struct M2Args {
    double d, om_step;
    double *m2f, *m2r, *m2o;
    double *m2part;            // NULL, or [frequency block][3][nm^2]
+   int diag;                  // ONLY_DIAG: n = 0, pa = Psi_l^2, entry p weighed by |H_p|^2
+   int kper;                  // K rows per slice (a multiple of 16; K: no slices)
 };
 
 template <int MT>
-__device__ __forceinline__ void m2_block(const M2Args &A, int n, int by, int p0)
+__device__ __forceinline__ void m2_block(const M2Args &A, int n, int by, int p0, int sl)
 {
    __shared__ double red[4][3][16 * MT];
    const int lane = threadIdx.x & 63;
@@ -1430,15 +1500,16 @@ __device__ __forceinline__ void m2_block(const M2Args &A, int n, int by, int p0)
 #pragma unroll
       for (int j = 0; j < MT; ++j) bv[j] = pb[j][k];
    };
-   load(0);
+   const int k0 = sl * A.kper, k1 = min(A.K, k0 + A.kper);
+   load(k0);
 #pragma unroll 2
-   for (int k = 0; k < A.K; k += 16) {
+   for (int k = k0; k < k1; k += 16) {
       double a[4], b[MT];
 #pragma unroll
       for (int i = 0; i < 4; ++i) a[i] = av[i];
 #pragma unroll
       for (int j = 0; j < MT; ++j) b[j] = bv[j];
-      if (k + 16 < A.K) load(k + 16);
+      if (k + 16 < k1) load(k + 16);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1457,7 +1528,7 @@ __device__ __forceinline__ void m2_block(const M2Args &A, int n, int by, int p0)
             if (u < A.nh) {
                double wt = (u == A.nh - 1) ? 0.5 * A.d : A.d;
                if (u > 0) wt *= 2.0;                                // +u and -u
-               const double2 hp = A.H[(size_t)p * A.nft + u], hn = A.H[(size_t)n * A.nft + u];
+               const double2 hp = A.H[(size_t)p * A.nft + u], hn = A.H[(size_t)(A.diag ? p : n) * A.nft + u];
                const double fr = hp.x * hn.x + hp.y * hn.y;         // Re[H_p conj(H_n)]
                const double om = A.om_step * u;
                const double v = wt * acc[i][j][t];
@@ -1481,7 +1552,7 @@ __device__ __forceinline__ void m2_block(const M2Args &A, int n, int by, int p0)
    __syncthreads();
    const int pl = threadIdx.x, p = p0 + pl;
    if (pl < 16 * MT && p < A.nm) {
-      const size_t nm2 = (size_t)A.nm * A.nm, id = n + (size_t)A.nm * p;
+      const size_t nm2 = (size_t)A.nm * A.nm, id = A.diag ? (size_t)p : n + (size_t)A.nm * p;
       double s[3];
 #pragma unroll
       for (int c = 0; c < 3; ++c) s[c] = (red[0][c][pl] + red[1][c][pl]) + (red[2][c][pl] + red[3][c][pl]);
@@ -1498,11 +1569,12 @@ __device__ __forceinline__ void m2_block(const M2Args &A, int n, int by, int p0)
    }
 }
 
-// grid (nm, ceil(nh/64), ceil(nm / (16 MT)))
+// grid (nm (diag: 1), ceil(nh/64), ceil(nm / (16 MT)) * K slices)
 template <int MT>
 __global__ __launch_bounds__(256, 2) void k_m2(M2Args A)
 {
-   m2_block<MT>(A, blockIdx.x, blockIdx.y, blockIdx.z * 16 * MT);
+   const int np = (A.nm + 16 * MT - 1) / (16 * MT);
+   m2_block<MT>(A, blockIdx.x, blockIdx.y, (int)blockIdx.z % np * 16 * MT, (int)blockIdx.z / np);
 }
 
 // Fixed-order compensated sums.  k_sum_lists: out[e] = sum over the slot list
