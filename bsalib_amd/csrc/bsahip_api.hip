@@ -519,6 +519,17 @@ int launch_frf(const Prob &D, int nft, double df, double2 *H)
    return 0;
 }
 
+// FP64 bispectra of nsel triples (device list sel; null: triple s of all) on the grid of
+// nf points per axis from the table U of nu rows per mode
+void bisp_grid_f64(const Prob &D, const double *U, long ldU, int nu, int nf, double df, long nsel,
+                   const int *sel, double *bfm, double *brm)
+{
+   const unsigned nt = (unsigned)((nf - 1) / 2 + 16) / 16;
+   const long ny = std::min(nsel, 65535L);
+   k_bisp_grid_f64<<<dim3(nt * nt, (unsigned)ny, (unsigned)((nsel + ny - 1) / ny)), 256, 0, g.s>>>(
+      U, ldU, nu, D.pb_k, D.K, D.nm, nf, df, nsel, sel, D.Mm, D.Km, D.Cm, bfm, brm);
+}
+
 int check_flags(int32_t flags, bool grid, bool allow_mixed)
 {
    const int prec = flags & BSAHIP_PREC_MASK;
@@ -1286,33 +1297,12 @@ int bsahip_classic_spectra(const bsahip_problem *p, int32_t nfh, double df, int3
    }
    if (bfm || brm) {
       const long npts = (long)nf * nf;
-      std::vector<int> i1(npts), i2(npts), i3(npts);
-      std::vector<double> f1(npts), f2(npts);
-      for (int q2 = 0; q2 < nf; ++q2)
-         for (int q1 = 0; q1 < nf; ++q1) {
-            const long pt = q1 + (long)nf * q2;
-            const int F1 = q1 - c, F2 = q2 - c, F3 = F1 + F2;
-            i1[pt] = std::abs(F1);
-            i2[pt] = std::abs(F2);
-            i3[pt] = (exact || std::abs(F3) <= c) ? std::abs(F3) : -1;
-            f1[pt] = F1 * df;
-            f2[pt] = F2 * df;
-         }
-      int *di1, *di2, *di3;
-      double *df1, *df2, *ob, *orr;
-      CHK(upload(B, "i1", i1, &di1));
-      CHK(upload(B, "i2", i2, &di2));
-      CHK(upload(B, "i3", i3, &di3));
-      CHK(upload(B, "f1", f1, &df1));
-      CHK(upload(B, "f2", f2, &df2));
+      double *ob, *orr;
       CHK(B.get("bfm_out", nm3 * npts, &ob));
       CHK(B.get("brm_out", nm3 * npts, &orr));
-      const long tot = (long)nm3 * npts;
-      if (tot > 0xffffff00L)
+      if ((long)nm3 * npts > 0xffffff00L)
          return fail(BSAHIP_EUNSUPPORTED, "NF^2 * NM^3 exceeds 2^32 bispectrum values in one call");
-      k_bfm_points<<<(unsigned)((tot + 255) / 256), 256, 0, g.s>>>(
-         U, ldU, nu, D.pb_k, D.K, D.nm, (int)npts, di1, di2, di3, df1, df2, D.Mm, D.Km, D.Cm,
-         ob, orr, 1, npts);
+      bisp_grid_f64(D, U, ldU, nu, nf, df, (long)nm3, nullptr, ob, orr);
       HIPC(hipGetLastError());
       if (bfm) HIPC(hipMemcpyAsync(bfm, ob, nm3 * npts * sizeof(double), hipMemcpyDeviceToHost, g.s));
       if (brm) HIPC(hipMemcpyAsync(brm, orr, nm3 * npts * sizeof(double), hipMemcpyDeviceToHost, g.s));
@@ -1376,7 +1366,7 @@ int bsahip_classic_bispectra_sel(const bsahip_problem *p, int32_t nfh, double df
                                             dsel, D.Mm, D.Km, D.Cm, ob, orr)
       if (prec == BSAHIP_PREC_FP32) LAUNCH_SEL(1);
       else if (prec == BSAHIP_PREC_BF16X3) LAUNCH_SEL(2);
-      else LAUNCH_SEL(0);
+      else bisp_grid_f64(D, U, ldU, nu, nf, df, nsel, dsel, ob, orr);
 #undef LAUNCH_SEL
    }
    HIPC(hipGetLastError());
@@ -1455,6 +1445,12 @@ int bsahip_diag_psd_points(const bsahip_problem *p, int32_t npts, const double *
 
 namespace {
 
+// the Mesher's point evaluation (mesher.hip)
+int point_table(Bufs &B, const Prob &D, const double *fl, int nu, int nmp, double **V);
+int point_psib(Bufs &B, const Prob &D, int nmp, double **PB);
+int bfm_batch(const Prob &D, const double *V, const double *PB, int nmp, int npts, const int *i1,
+              const int *i2, const int *i3, const long *slot, double *out);
+
 // sqrt-PSD table (ntc, nu, nnl) of the nodes at the distinct |f| uq; fmax > 0:
 // rows with |f| beyond fmax zero (the Classic grid's truncation)
 int diag_sq_table(Bufs &B, const Prob &D, const std::vector<double> &uq, double fmax, double **sq)
@@ -1525,38 +1521,51 @@ int bfm_points_impl(const bsahip_problem *p, int32_t npts, const double *fi, con
    }
    CHK(set_pod(p, D));
    const int nu = (int)uq.size();
-   const long ldU = (long)D.nm * nu;
-   double *dfl, *U;
-   CHK(upload(B, "fl", uq, &dfl));
-   CHK(B.get("U", (size_t)D.K * ldU, &U));
-   CHK(build_table(B, D, dfl, nu, nu, U, ldU));
-   if (fmax > 0.0) {
-      // uq is ascending: columns u0.. lie beyond the grid
-      const long u0 = std::upper_bound(uq.begin(), uq.end(), fmax * (1.0 + 1e-12)) - uq.begin();
-      if (u0 < nu) {
-         const long n = (long)D.K * D.nm * (nu - u0);
-         k_zero_cols<<<(unsigned)((n + 255) / 256), 256, 0, g.s>>>(U, ldU, nu, u0, D.nm, n);
-         HIPC(hipGetLastError());
-      }
-   }
+   const size_t nm3 = (size_t)D.nm * D.nm * D.nm;
+   const long tot = (long)nm3 * npts;
+   if (tot > 0xffffff00L)
+      return fail(BSAHIP_EUNSUPPORTED, "npts * NM^3 exceeds 2^32 bispectrum values in one call");
+   // uq is ascending: rows u0.. lie beyond the grid
+   const long u0 = fmax > 0.0 ? std::upper_bound(uq.begin(), uq.end(), fmax * (1.0 + 1e-12)) - uq.begin() : nu;
    std::vector<double> f1(fi, fi + npts), f2(fj, fj + npts);
    int *di1, *di2, *di3;
-   double *df1, *df2, *ob, *orr = nullptr;
+   double *dfl, *df1, *df2, *ob, *orr = nullptr;
+   CHK(upload(B, "fl", uq, &dfl));
    CHK(upload(B, "i1", i1, &di1));
    CHK(upload(B, "i2", i2, &di2));
    CHK(upload(B, "i3", i3, &di3));
    CHK(upload(B, "f1", f1, &df1));
    CHK(upload(B, "f2", f2, &df2));
-   const size_t nm3 = (size_t)D.nm * D.nm * D.nm;
    CHK(B.get("bfm_out", nm3 * npts, &ob));
    if (brm) CHK(B.get("brm_out", nm3 * npts, &orr));
-   const long tot = (long)nm3 * npts;
-   if (tot > 0xffffff00L)
-      return fail(BSAHIP_EUNSUPPORTED, "npts * NM^3 exceeds 2^32 bispectrum values in one call");
-   k_bfm_points<<<(unsigned)((tot + 255) / 256), 256, 0, g.s>>>(
-      U, ldU, nu, D.pb_k, D.K, D.nm, npts, di1, di2, di3, df1, df2, D.Mm, D.Km, D.Cm, ob, orr,
-      (long)nm3, 1);
-   HIPC(hipGetLastError());
+   const unsigned nblk = (unsigned)((tot + 255) / 256);
+   if (D.nm <= 32) {
+      // the Mesher's point kernel
+      const int nmp = (D.nm + 15) / 16 * 16;
+      const size_t slab = (size_t)D.K * nmp;
+      double *V, *PB;
+      CHK(point_table(B, D, dfl, nu, nmp, &V));
+      if (u0 < nu) CHK(fill(V + u0 * slab, (size_t)(nu - u0) * slab, 0.0));
+      CHK(point_psib(B, D, nmp, &PB));
+      CHK(bfm_batch(D, V, PB, nmp, npts, di1, di2, di3, nullptr, ob));
+      if (brm) {
+         k_brm_points<<<nblk, 256, 0, g.s>>>(ob, D.nm, tot, df1, df2, D.Mm, D.Km, D.Cm, orr);
+         HIPC(hipGetLastError());
+      }
+   } else {
+      const long ldU = (long)D.nm * nu;
+      double *U;
+      CHK(B.get("U", (size_t)D.K * ldU, &U));
+      CHK(build_table(B, D, dfl, nu, nu, U, ldU));
+      if (u0 < nu) {
+         const long n = (long)D.K * D.nm * (nu - u0);
+         k_zero_cols<<<(unsigned)((n + 255) / 256), 256, 0, g.s>>>(U, ldU, nu, u0, D.nm, n);
+         HIPC(hipGetLastError());
+      }
+      k_bfm_points<<<nblk, 256, 0, g.s>>>(U, ldU, nu, D.pb_k, D.K, D.nm, npts, di1, di2, di3, df1, df2,
+                                          D.Mm, D.Km, D.Cm, ob, orr, (long)nm3, 1);
+      HIPC(hipGetLastError());
+   }
    HIPC(hipMemcpyAsync(bfm, ob, nm3 * npts * sizeof(double), hipMemcpyDeviceToHost, g.s));
    if (brm) HIPC(hipMemcpyAsync(brm, orr, nm3 * npts * sizeof(double), hipMemcpyDeviceToHost, g.s));
    HIPC(hipStreamSynchronize(g.s));

@@ -1739,15 +1739,119 @@ __global__ __launch_bounds__(256) void k_bfm_points(
    if (brm) brm[pt * spt + mnp * smn] = s * brm_factor(f1s[pt], f2s[pt], m, n, p, Mm, Km, Cm);
 }
 
+// brm[e] = bfm[e] Re[H_m(f1) H_n(f2) conj H_p(f1+f2)] at points, e = pt nm^3 + mnp
+__global__ __launch_bounds__(256) void k_brm_points(const double *__restrict__ bfm, int nm, long total,
+                                                    const double *__restrict__ f1s,
+                                                    const double *__restrict__ f2s,
+                                                    const double *__restrict__ Mm,
+                                                    const double *__restrict__ Km,
+                                                    const double *__restrict__ Cm,
+                                                    double *__restrict__ brm)
+{
+   const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+   const long nm3 = (long)nm * nm * nm;
+   if (e >= total) return;
+   const long pt = e / nm3;
+   const int mnp = (int)(e % nm3);
+   brm[e] = bfm[e] * brm_factor(f1s[pt], f2s[pt], mnp % nm, (mnp / nm) % nm, mnp / (nm * nm), Mm, Km, Cm);
+}
+
 // ---------------------------------------------------------------------------
-// Bispectra of selected mode triples on the Classic grid f = (q - c) df,
-// q = 0 .. nf-1: out[q1 + nf*q2 + nf*nf*s] for triple sel[s] (linear index
-// m + n*nm + p*nm^2, m fastest), the reference's bisp(i, j, k) layout.
+// Bispectra of mode triples on the Classic grid f = (q - c) df, q = 0 .. nf-1:
+// out[q1 + nf*q2 + nf*nf*s] for triple sel[s] (linear index m + n*nm + p*nm^2,
+// m fastest; sel null: triple s), the reference's bisp(i, j, k) layout.
 // Rows of U: |F| for F within the grid; with exact, |f1+f2| up to 2c as well,
-// otherwise S(f1+f2) = 0 beyond the grid.  grid (ceil(nf*nf/256), nsel)
+// otherwise S(f1+f2) = 0 beyond the grid.
+//
+// FP64: one workgroup per 16x16 tile (|F1|, |F2|) and triple,
+//   B = 2 (G_m[(n,F1),(p,F2)] + G_n[(m,F3),(p,F2)] + G_p[(m,F3),(n,F1)]),
+// F3 = |F1 + F2| and |F1 - F2| in windows of 32 from |16 (a+b)| and 16 (a-b) - 16 on:
+// nine 16x16 blocks by MFMA.  A tile gives the four sign combinations of its points,
+// which are two values.  Its waves share the contraction (k = 16 i + 4 wave + 0..3) and
+// their parts are added in wave order, so a value does not depend on which launch formed
+// it.  One value per lane with a serial loop over k, five loads per term, took 286 us
+// for 3 triples, 300 nodes and 2 components, 257^2 points; now 33 us.
+// grid (tiles^2, min(nsel, 65535), ceil(nsel / 65535)), block 256
 // ---------------------------------------------------------------------------
-// PREC 0: FP64 (bfm_point); 1, 2: the G values of the FP32 / split-bf16x3
-// kernels (bfm_point_mixed).
+__global__ __launch_bounds__(256, 2) void k_bisp_grid_f64(
+   const double *__restrict__ U, long ldU, int rows, const double *__restrict__ pb, int K,
+   int nm, int nf, double df, long nsel, const int *__restrict__ sel,
+   const double *__restrict__ Mm, const double *__restrict__ Km, const double *__restrict__ Cm,
+   double *__restrict__ bfm, double *__restrict__ brm)
+{
+   __shared__ double part[4][9][256];
+   const long s = blockIdx.y + (long)gridDim.y * blockIdx.z;
+   if (s >= nsel) return;
+   const int c = (nf - 1) / 2, nt = (c + 16) / 16;
+   const int ta = (int)(blockIdx.x % nt), tb = (int)(blockIdx.x / nt);
+   const int mnp = sel ? sel[s] : (int)s;
+   const int m = mnp % nm, n = (mnp / nm) % nm, p = mnp / (nm * nm);
+   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 15, kk = 4 * wv + (lane >> 4);
+   // table rows of the lane's operands; those beyond the table are clamped and their
+   // products never used
+   const int last = rows - 1, d0 = 16 * (ta - tb) - 16 + l;
+   const double *An = U + (size_t)kk * ldU + (size_t)n * rows + min(16 * ta + l, last);
+   const double *Ap = U + (size_t)kk * ldU + (size_t)p * rows + min(16 * tb + l, last);
+   const double *Am = U + (size_t)kk * ldU + (size_t)m * rows;
+   const int r0 = min(16 * (ta + tb) + l, last), r1 = min(16 * (ta + tb) + 16 + l, last);
+   const int r2 = min(abs(d0), last), r3 = min(abs(d0 + 16), last);
+   const double *bm = pb + (size_t)m * K + kk, *bn = pb + (size_t)n * K + kk, *bp = pb + (size_t)p * K + kk;
+   d4 acc[9];
+#pragma unroll
+   for (int t = 0; t < 9; ++t) acc[t] = (d4){0.0, 0.0, 0.0, 0.0};
+   // K is a multiple of 32: every wave has K / 16 steps
+#pragma unroll 2
+   for (int k = 0; k < K; k += 16) {
+      const size_t o = (size_t)k * ldU;
+      const double an = An[o], ap = Ap[o], a0 = Am[o + r0], a1 = Am[o + r1], a2 = Am[o + r2], a3 = Am[o + r3];
+      const double x = bm[k] * an, y = bn[k] * ap, z = bp[k] * an;
+      acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, ap, acc[0], 0, 0, 0);
+      acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, y, acc[1], 0, 0, 0);
+      acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, y, acc[2], 0, 0, 0);
+      acc[3] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, z, acc[3], 0, 0, 0);
+      acc[4] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, z, acc[4], 0, 0, 0);
+      acc[5] = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, y, acc[5], 0, 0, 0);
+      acc[6] = __builtin_amdgcn_mfma_f64_16x16x4f64(a3, y, acc[6], 0, 0, 0);
+      acc[7] = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, z, acc[7], 0, 0, 0);
+      acc[8] = __builtin_amdgcn_mfma_f64_16x16x4f64(a3, z, acc[8], 0, 0, 0);
+   }
+#pragma unroll
+   for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) part[wv][t][16 * ((lane >> 4) + 4 * j) + l] = acc[t][j];
+   __syncthreads();
+   // F1 along the threads: it is the fastest index of the output
+   const int i = threadIdx.x & 15, j = threadIdx.x >> 4, u = 16 * ta + i, v = 16 * tb + j;
+   if (u > c || v > c) return;
+   const auto val = [&](int t, int row, int col) {
+      const int e = 16 * row + col;
+      return ((part[0][t][e] + part[1][t][e]) + part[2][t][e]) + part[3][t][e];
+   };
+   const double g = val(0, i, j);
+   const size_t o = (size_t)s * nf * nf;
+   const auto put = [&](int F1, int F2, double b, double fac) {
+      const size_t q = o + (size_t)(F1 + c) + (size_t)nf * (F2 + c);
+      if (bfm) bfm[q] = b;
+      if (brm) brm[q] = b * fac;
+   };
+#pragma unroll
+   for (int h = 0; h < 2; ++h) {                             // F1 + F2, then F1 - F2
+      const int w = h ? i - j + 16 : i + j, F2 = h ? -v : v;
+      double b = g;
+      if (abs(u + F2) <= last) {
+         b += val(1 + 4 * h + (w >> 4), w & 15, j);
+         b += val(3 + 4 * h + (w >> 4), w & 15, i);
+      }
+      b *= 2.0;
+      // both signs: H(-f) is the conjugate, the factor's real part the same
+      const double fac = brm ? brm_factor(u * df, F2 * df, m, n, p, Mm, Km, Cm) : 0.0;
+      put(u, F2, b, fac);
+      put(-u, -F2, b, fac);
+   }
+}
+
+// The same by the G values of the FP32 (PREC 1) and split-bf16x3 (2) kernels
+// (bfm_point_mixed).  grid (ceil(nf*nf/256), nsel)
 template <int PREC>
 __global__ __launch_bounds__(256) void k_bisp_grid_sel(
    const double *__restrict__ U, long ldU, int rows, const double *__restrict__ pb, int K,
@@ -1763,9 +1867,7 @@ __global__ __launch_bounds__(256) void k_bisp_grid_sel(
    const int m = mnp % nm, n = (mnp / nm) % nm, p = mnp / (nm * nm);
    const int F1 = (int)(pt % nf) - c, F2 = (int)(pt / nf) - c, F3 = F1 + F2;
    const int a3 = (exact || abs(F3) <= c) ? abs(F3) : -1;
-   const double s = PREC == 0 ? bfm_point(U, ldU, rows, pb, K, m, n, p, abs(F1), abs(F2), a3)
-                              : bfm_point_mixed<PREC>(U, ldU, rows, pb, K, m, n, p, abs(F1),
-                                                      abs(F2), a3);
+   const double s = bfm_point_mixed<PREC>(U, ldU, rows, pb, K, m, n, p, abs(F1), abs(F2), a3);
    const size_t o = (size_t)blockIdx.y * npts + pt;
    if (bfm) bfm[o] = s;
    if (brm) brm[o] = s * brm_factor(F1 * df, F2 * df, m, n, p, Mm, Km, Cm);

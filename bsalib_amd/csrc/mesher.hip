@@ -80,7 +80,9 @@ __global__ void k_pbt(const double *__restrict__ pb, int nm, int K, int nmp, dou
 // i.e. one NM x NM^2 product with a 2K-long contraction whose right operand
 // is formed on the fly.  Rows m are padded to MT*16, columns (n,p) (col =
 // n + p*nm) tiled by 16 and dealt to the 8 waves (TPW tiles each).
-// One workgroup per point; out[slot[pt]*nm3 + m + col*nm] = B.
+// One workgroup per point (point lists of the API too: 120 nodes, 2 components, 8 modes,
+// 301 points take 18 us where one value per lane took 209);
+// out[slot[pt]*nm3 + m + col*nm] = B (slot null: q0 + pt).
 // ---------------------------------------------------------------------------
 #define BKC 16   // K chunk staged in LDS
 
@@ -88,7 +90,7 @@ template <int MT, int TPW>
 __global__ __launch_bounds__(512) void k_bfm_batch(
    const double *__restrict__ V, const double *__restrict__ PB, int K, int nm, int npts,
    const int *__restrict__ ia1, const int *__restrict__ ia2, const int *__restrict__ ia3,
-   const long *__restrict__ slot, double *__restrict__ out)
+   const long *__restrict__ slot, long q0, double *__restrict__ out)
 {
    constexpr int NMP = MT * 16;
    __shared__ double s1[BKC][NMP], s2[BKC][NMP], s3[BKC][NMP], sp[BKC][NMP];
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(512) void k_bfm_batch(
       __syncthreads();
    }
    const long nm3 = (long)nm * ncol;
-   double *o = out + slot[pt] * nm3;
+   double *o = out + (slot ? slot[pt] : q0 + pt) * nm3;
 #pragma unroll
    for (int j = 0; j < TPW; ++j) {
       const int col = (wv + 8 * j) * 16 + (lane & 15);
@@ -936,6 +938,63 @@ size_t msh_lv0_at(const bsahip_mesher *M, const MshTile &t)
    return (size_t)t.g1 + (size_t)t.g2 * (size_t)M->nx;
 }
 
+// Point layout V of the table at the distinct |f| fl (k_vtable)
+int point_table(Bufs &B, const Prob &D, const double *fl, int nu, int nmp, double **V)
+{
+   CHK(B.get("m_V", (size_t)nu * D.K * nmp, V));
+   if (D.pod_nmodes > 0 || D.pod_lim > 0.0) {
+      const long ldU = (long)D.nm * nu;
+      double *U;
+      CHK(B.get("m_U", (size_t)D.K * ldU, &U));
+      CHK(build_table(B, D, fl, nu, nu, U, ldU));
+      dim3 gv((nu + 63) / 64, D.K);
+      k_vtable<<<gv, 256, 0, g.s>>>(U, ldU, nu, D.nm, D.K, nmp, *V);
+      HIPC(hipGetLastError());
+      return 0;
+   }
+   // the projection writes the point layout itself
+   double *sq;
+   CHK(psd_table(B, D, fl, nu, &sq));
+   return project(D, sq, fl, nu, nu, *V, nmp, true);
+}
+
+// Psi_b in the point layout
+int point_psib(Bufs &B, const Prob &D, int nmp, double **PB)
+{
+   CHK(B.get("m_PB", (size_t)D.K * nmp, PB));
+   k_pbt<<<(unsigned)(((long)D.K * nmp + 255) / 256), 256, 0, g.s>>>(D.pb_k, D.nm, D.K, nmp, *PB);
+   HIPC(hipGetLastError());
+   return 0;
+}
+
+// BFM at points: k_bfm_batch over V and PB; slot null: point q's values at q nm^3
+int bfm_batch(const Prob &D, const double *V, const double *PB, int nmp, int npts, const int *i1,
+              const int *i2, const int *i3, const long *slot, double *out)
+{
+   const int ncol = D.nm * D.nm, ct = (ncol + 15) / 16, tpw = (ct + 7) / 8;
+   // a grid holds fewer than 2^32 threads
+   constexpr int CHUNK = 1 << 22;
+   for (int q0 = 0; q0 < npts; q0 += CHUNK) {
+      const int n = std::min(CHUNK, npts - q0);
+#define LAUNCH_BATCH(MT, TPW)                                                                 \
+   k_bfm_batch<MT, TPW><<<n, 512, 0, g.s>>>(V, PB, D.K, D.nm, n, i1 + q0, i2 + q0, i3 + q0,   \
+                                            slot ? slot + q0 : nullptr, q0, out)
+      if (nmp == 16) {
+         if (tpw <= 1) LAUNCH_BATCH(1, 1);
+         else LAUNCH_BATCH(1, 2);
+      } else if (nmp == 32) {
+         if (tpw <= 2) LAUNCH_BATCH(2, 2);
+         else if (tpw <= 4) LAUNCH_BATCH(2, 4);
+         else LAUNCH_BATCH(2, 8);
+      } else {
+         return fail(BSAHIP_EUNSUPPORTED, "point evaluation supports at most 32 modes");
+      }
+#undef LAUNCH_BATCH
+      HIPC(hipGetLastError());
+   }
+   return 0;
+}
+
 // BFM at the points (f1[q], f2[q]) into out + slot[q]*nm3, in chunks of at
 // most MSH_CHUNK points so the A tables stay small (3 distinct |f| per point
 // at most).
@@ -983,44 +1042,16 @@ int msh_eval_chunk(bsahip_mesher *M, int npts, const double *f1p, const double *
       HIPC(hipGetLastError());
       return 0;
    }
-   const long ldU = (long)D.nm * nu;
-   double *fl, *U, *V;
+   double *fl, *V;
    CHK(upload(M->B, "m_fl", uq, &fl));
-   CHK(M->B.get("m_V", (size_t)nu * D.K * M->nmp, &V));
-   if (D.pod_nmodes > 0 || D.pod_lim > 0.0) {
-      CHK(M->B.get("m_U", (size_t)D.K * ldU, &U));
-      CHK(build_table(M->B, D, fl, nu, nu, U, ldU));
-      dim3 gv((nu + 63) / 64, D.K);
-      k_vtable<<<gv, 256, 0, g.s>>>(U, ldU, nu, D.nm, D.K, M->nmp, V);
-      HIPC(hipGetLastError());
-   } else {
-      // the projection writes the point layout itself
-      double *sq;
-      CHK(psd_table(M->B, D, fl, nu, &sq));
-      CHK(project(D, sq, fl, nu, nu, V, M->nmp, true));
-   }
+   CHK(point_table(M->B, D, fl, nu, M->nmp, &V));
    int *d1, *d2, *d3;
    long *ds;
    CHK(upload(M->B, "m_i1", i1, &d1));
    CHK(upload(M->B, "m_i2", i2, &d2));
    CHK(upload(M->B, "m_i3", i3, &d3));
    CHK(upload(M->B, "m_slot", slot, &ds));
-   const int ncol = D.nm * D.nm, ct = (ncol + 15) / 16, tpw = (ct + 7) / 8;
-#define LAUNCH_BATCH(MT, TPW)                                                                 \
-   k_bfm_batch<MT, TPW><<<npts, 512, 0, g.s>>>(V, M->PB, D.K, D.nm, npts, d1, d2, d3, ds, out)
-   if (M->nmp == 16) {
-      if (tpw <= 1) LAUNCH_BATCH(1, 1);
-      else LAUNCH_BATCH(1, 2);
-   } else if (M->nmp == 32) {
-      if (tpw <= 2) LAUNCH_BATCH(2, 2);
-      else if (tpw <= 4) LAUNCH_BATCH(2, 4);
-      else LAUNCH_BATCH(2, 8);
-   } else {
-      return fail(BSAHIP_EUNSUPPORTED, "point evaluation supports at most 32 modes");
-   }
-#undef LAUNCH_BATCH
-   HIPC(hipGetLastError());
-   return 0;
+   return bfm_batch(D, V, M->PB, M->nmp, npts, d1, d2, d3, ds, out);
 }
 
 // Points of a tile's BFM grid at level l (q = i + j*nb1).
@@ -1456,9 +1487,7 @@ int msh_setup(const bsahip_problem *p, const bsahip_mesher_cfg *cfg, int32_t fla
    CHK(msh_full_axis(cfg, D.nm, ax, M->dfref));
    msh_tiles(ax, cfg, D.nm, M->dfref, M->tiles);
    M->mirror = msh_mirror(M->tiles);
-   CHK(M->B.get("m_PB", (size_t)D.K * M->nmp, &M->PB));
-   k_pbt<<<(unsigned)((D.K * M->nmp + 255) / 256), 256, 0, g.s>>>(D.pb_k, D.nm, D.K, M->nmp, M->PB);
-   HIPC(hipGetLastError());
+   CHK(point_psib(M->B, D, M->nmp, &M->PB));
    M->diag = (flags & BSAHIP_ONLY_DIAG) != 0;
    M->nc = M->diag ? D.nm : D.nm * D.nm * D.nm;
    const size_t nm3 = (size_t)M->nc;
