@@ -51,6 +51,9 @@ int fail(int code, const std::string &msg)
       if (r_ != 0) return r_;                                                                \
    } while (0)
 
+struct Bufs;
+bool give_back(const Bufs *asking);
+
 // Named, grow-only device buffers.  With an arena (set_arena), get() carves
 // the buffers out of that fixed device region instead and never allocates.
 struct Bufs {
@@ -61,6 +64,8 @@ struct Bufs {
    std::map<std::string, Buf> m;
    char *arena = nullptr;
    size_t arena_cap = 0, arena_used = 0;
+   Bufs() = default;
+   Bufs(const Bufs &) = delete;                              // owns its buffers
    ~Bufs() { release(); }
    void release()
    {
@@ -75,6 +80,12 @@ struct Bufs {
       release();
       arena = static_cast<char *>(base);
       arena_cap = cap;
+   }
+   size_t total() const
+   {
+      size_t n = 0;
+      for (const auto &kv : m) n += kv.second.n;
+      return n;
    }
    template <class T>
    int get(const char *name, size_t count, T **out)
@@ -106,6 +117,10 @@ struct Bufs {
          b.p = nullptr;
          b.n = 0;
          hipError_t e = hipMalloc(&b.p, bytes);
+         if (e == hipErrorOutOfMemory && give_back(this)) {
+            (void)hipGetLastError();
+            e = hipMalloc(&b.p, bytes);
+         }
          if (e != hipSuccess)
             return fail(BSAHIP_ENOMEM, std::string("hipMalloc(") + name + ", " +
                                            std::to_string(bytes) + " B): " + hipGetErrorString(e));
@@ -134,6 +149,12 @@ struct Ctx {
    hipStream_t s2 = nullptr;             // side stream: modal PSD moments beside the G kernel
    hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr;
    Bufs *bufs = nullptr;                 // scratch of the one-shot entry points
+   char *stage = nullptr;                // pinned host memory of Pack, then of Pull
+   hipEvent_t es = nullptr;              // Pack's last copy out of it
+   // load_problem's host tables, kept up to HOST_KEPT values each: fresh ones cost a page
+   // fault every 4 KB
+   std::vector<double> pa_t, pa_k, pb_k;
+   std::vector<float> pb32;
    double last_ms = 0.0;
    int last_launches = 0;
    rocblas_handle blas = nullptr;        // created on first use (truncated POD)
@@ -141,6 +162,122 @@ struct Ctx {
 };
 
 Ctx g;
+
+// The one-shot scratch freed for another owner of buffers that found no memory.
+bool give_back(const Bufs *asking)
+{
+   if (!g.bufs || asking == g.bufs || g.bufs->m.empty()) return false;
+   (void)hipDeviceSynchronize();
+   g.bufs->release();
+   return true;
+}
+
+// Host arrays and device results of one call travel in few copies: a copy from or to
+// pageable memory costs about 5 us up and 20 us down however small it is (13 uploads of a
+// small problem 62 us, one of the same bytes out of pinned memory 12 us; 4 KB down 23 us,
+// by pinned memory 12 us).  From about a megabyte on there is nothing to win (1.6 MB down
+// 317 us either way: the page faults of the caller's array).
+constexpr size_t STAGE_UP = (size_t)4 << 20, STAGE_DOWN = (size_t)512 << 10, PART_UP = STAGE_UP / 4;
+
+// Uploads gathered into one device buffer (src null: room only).  The host arrays have to
+// live until send().
+struct Pack {
+   struct Part {
+      const void *src;
+      size_t bytes, off;
+      void **out;
+   };
+   std::vector<Part> parts;
+   size_t n = 0;
+   // every array starts where a buffer of its own would in an arena: at a multiple of 256
+   void add(const void *src, size_t bytes, void **out)
+   {
+      parts.push_back({src, bytes, n, out});
+      n += std::max<size_t>((bytes + 255) / 256 * 256, 256);
+   }
+   template <class T>
+   void add(const std::vector<T> &h, T **out)
+   {
+      add(h.data(), h.size() * sizeof(T), reinterpret_cast<void **>(out));
+   }
+   int send(Bufs &B, const char *name)
+   {
+      char *dev;
+      CHK(B.get(name, n, &dev));
+      size_t lo = 0, hi = 0;                                 // staged, not yet sent
+      const auto flush = [&]() -> int {
+         if (hi > lo) {
+            HIPC(hipMemcpyAsync(dev + lo, g.stage, hi - lo, hipMemcpyHostToDevice, g.s));
+            HIPC(hipEventRecord(g.es, g.s));
+         }
+         lo = hi;
+         return 0;
+      };
+      for (const Part &p : parts) {
+         if (p.out) *p.out = dev + p.off;
+         if (!p.bytes || !p.src) continue;
+         if (!g.stage || p.bytes > PART_UP) {
+            CHK(flush());
+            HIPC(hipMemcpyAsync(dev + p.off, p.src, p.bytes, hipMemcpyHostToDevice, g.s));
+            lo = hi = p.off + p.bytes;
+            continue;
+         }
+         if (p.off + p.bytes - lo > STAGE_UP) CHK(flush());
+         if (hi == lo) {
+            HIPC(hipEventSynchronize(g.es));                 // an earlier copy may still read it
+            lo = hi = p.off;
+         }
+         std::memcpy(g.stage + (p.off - lo), p.src, p.bytes);
+         hi = p.off + p.bytes;
+      }
+      CHK(flush());
+      parts.clear();
+      n = 0;
+      return 0;
+   }
+};
+
+// Results brought to the host: finish() waits for the stream.
+struct Pull {
+   struct Seg {
+      void *dst;
+      const char *src;
+      size_t bytes;
+   };
+   std::vector<Seg> segs;
+   size_t n = 0;
+   int add(void *dst, const void *src, size_t bytes)
+   {
+      if (!dst || !bytes) return 0;
+      if (!g.stage || n + bytes > STAGE_DOWN) {
+         HIPC(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g.s));
+         return 0;
+      }
+      segs.push_back({dst, static_cast<const char *>(src), bytes});
+      n += bytes;
+      return 0;
+   }
+   int finish()
+   {
+      char *stage = g.stage + STAGE_UP;
+      size_t at = 0;
+      for (size_t i = 0, j; i < segs.size(); i = j) {        // neighbours on the device in one copy
+         size_t len = segs[i].bytes;
+         for (j = i + 1; j < segs.size() && segs[j].src == segs[i].src + len; ++j) len += segs[j].bytes;
+         HIPC(hipMemcpyAsync(stage + at, segs[i].src, len, hipMemcpyDeviceToHost, g.s));
+         at += len;
+      }
+      HIPC(hipStreamSynchronize(g.s));
+      at = 0;
+      for (const Seg &q : segs) {
+         std::memcpy(q.dst, stage + at, q.bytes);
+         at += q.bytes;
+      }
+      segs.clear();
+      n = 0;
+      return 0;
+   }
+};
 
 template <class T>
 int upload(Bufs &B, const char *name, const std::vector<T> &h, T **out)
@@ -213,7 +350,12 @@ struct Prob {
 
 // psd_mode 0: reference Classic/Mesher semantics (evalPSD per component);
 // psd_mode 1: BsaCL semantics (u formula for every component, zone 1, rho clamped).
-int load_problem(const bsahip_problem *p, int psd_mode, Bufs &B, Prob &D)
+constexpr size_t HOST_KEPT = (size_t)1 << 18;
+
+// more: arrays of the caller that go up with the problem's; coh false: no coherence table
+// (D.lnr null), for callers that do not project.
+int load_problem(const bsahip_problem *p, int psd_mode, Bufs &B, Prob &D, Pack *more = nullptr,
+                 bool coh = true)
 {
    CHK(validate(p));
    D.nn = p->nn;
@@ -225,20 +367,26 @@ int load_problem(const bsahip_problem *p, int psd_mode, Bufs &B, Prob &D)
    D.K = round_up(D.kv, KC);
    D.pulsation = p->pulsation;
    const int nm = D.nm, nnl = D.nnl, K = D.K;
-   std::vector<double> pa_t((size_t)D.ntc * nm * nnl, 0.0), pa_k((size_t)nm * K, 0.0),
-      pb_k((size_t)nm * K, 0.0);
+   // only the truncated POD reads Psi_a by components
+   const bool pod = p->pod_nmodes != 0 || p->pod_trunc_lim != 0.0;
+   const size_t npt = (size_t)D.ntc * nm * nnl, npk = (size_t)nm * K;
+   std::vector<double> &pa_t = g.pa_t, &pa_k = g.pa_k, &pb_k = g.pb_k;
+   std::vector<float> &pb32 = g.pb32;
+   pa_t.resize(pod ? npt : 0);
+   pa_k.assign(npk, 0.0);
+   pb_k.assign(npk, 0.0);
    for (int c = 0; c < D.ntc; ++c) {
       const int t = p->tc[c];
       for (int i = 0; i < nnl; ++i)
          for (int m = 0; m < nm; ++m) {
             const double a = p->psi[m + (size_t)nm * (i + (size_t)nnl * (t - 1))];
             const double b = p->psi[m + (size_t)nm * (i + (size_t)nnl * (t + 2))];
-            pa_t[((size_t)c * nm + m) * nnl + i] = a;
+            if (pod) pa_t[((size_t)c * nm + m) * nnl + i] = a;
             pa_k[(size_t)m * K + (size_t)c * D.nnlp + i] = a;
             pb_k[(size_t)m * K + (size_t)c * D.nnlp + i] = b;
          }
    }
-   std::vector<float> pb32(pb_k.begin(), pb_k.end());
+   pb32.assign(pb_k.begin(), pb_k.end());
    // coherence columns actually read (nod_corr_(:, tc), or column 1 for all)
    std::vector<int> col(D.ntc);
    for (int c = 0; c < D.ntc; ++c)
@@ -249,10 +397,17 @@ int load_problem(const bsahip_problem *p, int psd_mode, Bufs &B, Prob &D)
    std::vector<int> colmap(D.ntc);
    for (int c = 0; c < D.ntc; ++c)
       colmap[c] = (int)(std::lower_bound(ucol.begin(), ucol.end(), col[c]) - ucol.begin());
-   std::vector<double> corr((size_t)ucol.size() * p->ncorr_rows);
-   for (size_t k = 0; k < ucol.size(); ++k)
-      std::memcpy(corr.data() + k * p->ncorr_rows, p->nod_corr + (size_t)ucol[k] * p->ncorr_rows,
-                  sizeof(double) * p->ncorr_rows);
+   // the table itself when they are its first ones, in order
+   std::vector<double> corr;
+   const double *corr_h = p->nod_corr;
+   const size_t ncorr = coh ? ucol.size() * (size_t)p->ncorr_rows : 0;
+   if (coh && ucol.back() != (int)ucol.size() - 1) {
+      corr.resize(ncorr);
+      for (size_t k = 0; k < ucol.size(); ++k)
+         std::memcpy(corr.data() + k * p->ncorr_rows, p->nod_corr + (size_t)ucol[k] * p->ncorr_rows,
+                     sizeof(double) * p->ncorr_rows);
+      corr_h = corr.data();
+   }
    std::vector<int> nl(p->n_load, p->n_load + nnl);
    std::vector<double> prm((size_t)D.ntc * nnl * 4, 0.0);
    std::vector<int> formula(D.ntc, 0);
@@ -279,18 +434,26 @@ int load_problem(const bsahip_problem *p, int psd_mode, Bufs &B, Prob &D)
    std::vector<double> Mm(p->Mm, p->Mm + nm), Km(p->Km, p->Km + nm), Cm(p->Cm, p->Cm + nm);
    double *dcorr;
    int *dcol, *dnl;
-   CHK(upload(B, "pa_t", pa_t, &D.pa_t));
-   CHK(upload(B, "pa_k", pa_k, &D.pa_k));
-   CHK(upload(B, "pb_k", pb_k, &D.pb_k));
-   CHK(upload(B, "pb32", pb32, &D.pb32));
-   CHK(upload(B, "corr", corr, &dcorr));
-   CHK(upload(B, "colmap", colmap, &dcol));
-   CHK(upload(B, "n_load", nl, &dnl));
-   CHK(upload(B, "prm", prm, &D.prm));
-   CHK(upload(B, "formula", formula, &D.formula));
-   CHK(upload(B, "Mm", Mm, &D.Mm));
-   CHK(upload(B, "Km", Km, &D.Km));
-   CHK(upload(B, "Cm", Cm, &D.Cm));
+   Pack own, &pk = more ? *more : own;
+   // room for Psi_a by components in any case: a problem needs the same scratch with a POD
+   pk.add(pod ? pa_t.data() : nullptr, npt * sizeof(double), reinterpret_cast<void **>(&D.pa_t));
+   pk.add(pa_k, &D.pa_k);
+   pk.add(pb_k, &D.pb_k);
+   pk.add(pb32, &D.pb32);
+   pk.add(colmap, &dcol);
+   pk.add(nl, &dnl);
+   pk.add(prm, &D.prm);
+   pk.add(formula, &D.formula);
+   pk.add(Mm, &D.Mm);
+   pk.add(Km, &D.Km);
+   pk.add(Cm, &D.Cm);
+   if (coh) pk.add(corr_h, ncorr * sizeof(double), reinterpret_cast<void **>(&dcorr));
+   CHK(pk.send(B, "problem"));
+   if (npk > HOST_KEPT) {
+      for (auto *v : {&pa_t, &pa_k, &pb_k}) std::vector<double>().swap(*v);
+      std::vector<float>().swap(pb32);
+   }
+   if (!coh) return 0;
    CHK(B.get("lnr", (size_t)D.ntc * nnl * nnl, &D.lnr));
    dim3 gl((nnl + 255) / 256, nnl, D.ntc);
    k_lnrho<<<gl, 256, 0, g.s>>>(dcorr, p->ncorr_rows, dcol, dnl, nnl, p->nn,
@@ -545,24 +708,51 @@ int check_flags(int32_t flags, bool grid, bool allow_mixed)
 void point_tables(int npts, const double *fi, const double *fj, std::vector<double> &uq,
                   std::vector<int> &i1, std::vector<int> &i2, std::vector<int> &i3)
 {
-   std::vector<double> all;
-   all.reserve(3 * (size_t)npts);
-   for (int q = 0; q < npts; ++q) {
-      all.push_back(std::fabs(fi[q]));
-      all.push_back(std::fabs(fj[q]));
-      all.push_back(std::fabs(fi[q] + fj[q]));
+   // distinct values by open addressing on their bits, then sorted: a sort of all 3 npts
+   // and a search for each took 3/5 of a Mesher's refinement (40 nodes, 3 modes: 10.4 ms of
+   // zones built, refined and integrated, now 4.3)
+   size_t cap = 16;
+   int shift = 60;
+   while (cap < 6 * (size_t)npts) {
+      cap *= 2;
+      --shift;
    }
-   uq = all;
-   std::sort(uq.begin(), uq.end());
-   uq.erase(std::unique(uq.begin(), uq.end()), uq.end());
-   auto idx = [&](double v) { return (int)(std::lower_bound(uq.begin(), uq.end(), v) - uq.begin()); };
+   std::vector<int> table(cap, -1), id(3 * (size_t)npts);
+   std::vector<double> keys;
+   const auto look = [&](double v) {
+      v = std::fabs(v);
+      uint64_t bits;
+      std::memcpy(&bits, &v, sizeof bits);
+      for (size_t h = (size_t)((bits * 0x9E3779B97F4A7C15ull) >> shift);; h = (h + 1) & (cap - 1)) {
+         const int k = table[h];
+         if (k < 0) {
+            table[h] = (int)keys.size();
+            keys.push_back(v);
+            return table[h];
+         }
+         if (std::memcmp(&keys[k], &bits, sizeof bits) == 0) return k;
+      }
+   };
+   for (int q = 0; q < npts; ++q) {
+      id[3 * (size_t)q] = look(fi[q]);
+      id[3 * (size_t)q + 1] = look(fj[q]);
+      id[3 * (size_t)q + 2] = look(fi[q] + fj[q]);
+   }
+   std::vector<int> order(keys.size()), rank(keys.size());
+   for (size_t k = 0; k < order.size(); ++k) order[k] = (int)k;
+   std::sort(order.begin(), order.end(), [&](int a, int b) { return keys[a] < keys[b]; });
+   uq.resize(keys.size());
+   for (size_t k = 0; k < order.size(); ++k) {
+      uq[k] = keys[order[k]];
+      rank[order[k]] = (int)k;
+   }
    i1.resize(npts);
    i2.resize(npts);
    i3.resize(npts);
    for (int q = 0; q < npts; ++q) {
-      i1[q] = idx(all[3 * q]);
-      i2[q] = idx(all[3 * q + 1]);
-      i3[q] = idx(all[3 * q + 2]);
+      i1[q] = rank[id[3 * (size_t)q]];
+      i2[q] = rank[id[3 * (size_t)q + 1]];
+      i3[q] = rank[id[3 * (size_t)q + 2]];
    }
 }
 
@@ -711,13 +901,18 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    if (nfh < 2 || !(df > 0.0)) return fail(BSAHIP_EINVAL, "need nfh >= 2 and df > 0");
    if (flags & BSAHIP_ONLY_DIAG)
       return fail(BSAHIP_EUNSUPPORTED, "the ONLY_DIAG model runs through bsahip_classic_run");
-   CHK(load_problem(p, psd_mode, P->B, P->D));
+   const int nu = (flags & BSAHIP_SUM_EXACT) ? 2 * nfh - 1 : nfh;
+   std::vector<double> fl(nu);
+   for (int u = 0; u < nu; ++u) fl[u] = (double)u * df;
+   Pack pk;
+   pk.add(fl, &P->fl);
+   CHK(load_problem(p, psd_mode, P->B, P->D, &pk));
    P->flags = flags;
    P->prec = flags & BSAHIP_PREC_MASK;
    P->df = df;
    P->nh = nfh;
    P->nf = 2 * nfh - 1;
-   P->nu = (flags & BSAHIP_SUM_EXACT) ? P->nf : P->nh;          // rows of A per mode
+   P->nu = nu;                                                  // rows of A per mode
    // rows of consecutive modes packed (no padding to 16 per mode): a 16-row
    // block may span two modes, and the epilogue masks the other mode's rows
    P->nhp = P->nu;
@@ -734,9 +929,6 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    if (npairs * P->D.nm * 256L > 0xffffffffL)
       return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: (tile pairs x modes) x 256 "
                                        "threads exceeds 2^32; use a coarser grid or fewer modes");
-   std::vector<double> fl(P->nu);
-   for (int u = 0; u < P->nu; ++u) fl[u] = (double)u * df;
-   CHK(upload(P->B, "fl", fl, &P->fl));
    CHK(P->B.get("U", (size_t)P->D.K * P->ldU, &P->U));
    CHK(zero_padding(P->D, P->nhp, P->U, P->ldU));      // the runs write the valid entries only
    CHK(P->B.get("H", (size_t)P->D.nm * P->nft, &P->H));
@@ -896,16 +1088,17 @@ int plan_copyout(bsahip_plan *P, double *m2mf, double *m2mr, double *m2o2mr, dou
 {
    const Prob &D = P->D;
    const size_t nm3 = (size_t)D.nm * D.nm * D.nm, nm2 = (size_t)D.nm * D.nm;
-   if (!(P->flags & BSAHIP_NO_BISP)) {
-      if (m3mf) HIPC(hipMemcpyAsync(m3mf, P->m3, nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
-      if (m3mr) HIPC(hipMemcpyAsync(m3mr, P->m3 + nm3, nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
-   }
+   Pull pl;
    if (!(P->flags & BSAHIP_NO_PSD)) {
-      if (m2mf) HIPC(hipMemcpyAsync(m2mf, P->m2, nm2 * sizeof(double), hipMemcpyDeviceToHost, g.s));
-      if (m2mr) HIPC(hipMemcpyAsync(m2mr, P->m2 + nm2, nm2 * sizeof(double), hipMemcpyDeviceToHost, g.s));
-      if (m2o2mr) HIPC(hipMemcpyAsync(m2o2mr, P->m2 + 2 * nm2, nm2 * sizeof(double), hipMemcpyDeviceToHost, g.s));
+      CHK(pl.add(m2mf, P->m2, nm2 * sizeof(double)));
+      CHK(pl.add(m2mr, P->m2 + nm2, nm2 * sizeof(double)));
+      CHK(pl.add(m2o2mr, P->m2 + 2 * nm2, nm2 * sizeof(double)));
    }
-   return 0;
+   if (!(P->flags & BSAHIP_NO_BISP)) {
+      CHK(pl.add(m3mf, P->m3, nm3 * sizeof(double)));
+      CHK(pl.add(m3mr, P->m3 + nm3, nm3 * sizeof(double)));
+   }
+   return pl.finish();
 }
 
 int plan_exec(bsahip_plan *P, double *m2mf, double *m2mr, double *m2o2mr, double *m3mf, double *m3mr)
@@ -935,7 +1128,6 @@ int plan_exec(bsahip_plan *P, double *m2mf, double *m2mr, double *m2o2mr, double
    if (want_psd && !side) CHK(plan_m2(P));
    if (side) HIPC(hipStreamWaitEvent(g.s, g.e3, 0));
    CHK(plan_copyout(P, m2mf, m2mr, m2o2mr, m3mf, m3mr));
-   HIPC(hipStreamSynchronize(g.s));
    g.last_ms = 0.0;
    g.last_launches = 0;
    if (want_bisp) {
@@ -953,6 +1145,20 @@ Bufs &oneshot_bufs()
    if (!g.bufs) g.bufs = new Bufs();
    return *g.bufs;
 }
+
+// A plan of one call works in the one-shot scratch: with buffers of its own, allocated and
+// freed by each call, 151 nodes, 9 modes, 101 frequencies took 296 us, so 248.  Scratch
+// beyond KEPT bytes is freed with the plan.
+struct PoolLoan {
+   static constexpr size_t KEPT = (size_t)256 << 20;
+   Bufs &B;
+   explicit PoolLoan(Bufs &b) : B(b) { B.m.swap(oneshot_bufs().m); }
+   ~PoolLoan()
+   {
+      if (B.total() > KEPT) B.release();
+      B.m.swap(oneshot_bufs().m);
+   }
+};
 
 }  // namespace
 
@@ -985,6 +1191,12 @@ int bsahip_init(int device)
    HIPC(hipEventCreate(&g.e1));
    HIPC(hipEventCreateWithFlags(&g.e2, hipEventDisableTiming));
    HIPC(hipEventCreateWithFlags(&g.e3, hipEventDisableTiming));
+   HIPC(hipEventCreateWithFlags(&g.es, hipEventDisableTiming));
+   if (hipHostMalloc(reinterpret_cast<void **>(&g.stage), STAGE_UP + STAGE_DOWN, hipHostMallocDefault) !=
+       hipSuccess) {
+      g.stage = nullptr;                                     // copies from pageable memory instead
+      (void)hipGetLastError();
+   }
    g.dev = device;
    g.ready = true;
    return 0;
@@ -1004,6 +1216,9 @@ int bsahip_finalise(void)
    (void)hipEventDestroy(g.e1);
    (void)hipEventDestroy(g.e2);
    (void)hipEventDestroy(g.e3);
+   (void)hipEventDestroy(g.es);
+   if (g.stage) (void)hipHostFree(g.stage);
+   g.stage = nullptr;
    (void)hipStreamDestroy(g.s2);
    (void)hipStreamDestroy(g.s);
    g.ready = false;
@@ -1085,14 +1300,10 @@ struct DiagTab {
    long ldX;
 };
 
-int diag_tables(Bufs &B, const Prob &D, int nh, double df, DiagTab &T)
+int diag_tables(Bufs &B, const Prob &D, const double *dfl, int nh, double df, DiagTab &T)
 {
    const int nft = 2 * nh - 1, nm = D.nm, K = D.K;
-   std::vector<double> fl(nh);
-   for (int u = 0; u < nh; ++u) fl[u] = (double)u * df;
-   double *dfl;
    T.ldX = round_up(nh, 128);
-   CHK(upload(B, "fl", fl, &dfl));
    CHK(B.get("dg_X", (size_t)K * T.ldX, &T.X));
    CHK(B.get("dg_W", (size_t)nm * K, &T.W));
    CHK(B.get("dg_A2", (size_t)nm * K, &T.A2));
@@ -1129,13 +1340,18 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
    if (nfh < 2 || !(df > 0.0)) return fail(BSAHIP_EINVAL, "need nfh >= 2 and df > 0");
    Bufs &B = oneshot_bufs();
    Prob D;
-   CHK(load_problem(p, 0, B, D));
+   Pack pk;
+   std::vector<double> fl(nfh);
+   for (int u = 0; u < nfh; ++u) fl[u] = (double)u * df;
+   double *dfl;
+   pk.add(fl, &dfl);
+   CHK(load_problem(p, 0, B, D, &pk, false));
    const int nh = nfh, nft = 2 * nh - 1, nm = D.nm, K = D.K;
    const double d = p->pulsation ? df * 2.0 * M_PI : df;
    const bool psd = !(flags & BSAHIP_NO_PSD), bisp = !(flags & BSAHIP_NO_BISP);
    DiagTab T;
    double *mom;
-   CHK(diag_tables(B, D, nh, df, T));
+   CHK(diag_tables(B, D, dfl, nh, df, T));
    CHK(B.get("dg_mom", 5 * (size_t)nm, &mom));
    CHK(fill(mom, 5 * (size_t)nm, 0.0));
    double *m2f = mom, *m2r = mom + nm, *m2o = mom + 2 * nm, *m3f = mom + 3 * nm, *m3r = mom + 4 * nm;
@@ -1178,18 +1394,18 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
       HIPC(hipGetLastError());
    }
    if (psd) HIPC(hipStreamWaitEvent(g.s, g.e3, 0));
-   std::vector<double> h(5 * (size_t)nm);
-   HIPC(hipMemcpyAsync(h.data(), mom, h.size() * sizeof(double), hipMemcpyDeviceToHost, g.s));
-   HIPC(hipStreamSynchronize(g.s));
-   auto put = [&](double *dst, int slot, bool on) {
-      if (dst && on) std::memcpy(dst, h.data() + (size_t)slot * nm, nm * sizeof(double));
-   };
-   put(m2mf, 0, psd);
-   put(m2mr, 1, psd);
-   put(m2o2mr, 2, psd);
-   put(m3mf, 3, bisp);
-   put(m3mr, 4, bisp);
-   return 0;
+   Pull pl;
+   const size_t nb = nm * sizeof(double);
+   if (psd) {
+      CHK(pl.add(m2mf, m2f, nb));
+      CHK(pl.add(m2mr, m2r, nb));
+      CHK(pl.add(m2o2mr, m2o, nb));
+   }
+   if (bisp) {
+      CHK(pl.add(m3mf, m3f, nb));
+      CHK(pl.add(m3mr, m3r, nb));
+   }
+   return pl.finish();
 }
 
 }  // namespace
@@ -1209,8 +1425,11 @@ int bsahip__classic_moments(const bsahip_problem *p, int32_t nfh, double df, int
       return classic_diag(p, nfh, df, flags, m2mf, m2mr, m2o2mr, m3mf, m3mr);
    }
    bsahip_plan P;
-   CHK(plan_setup(&P, p, nfh, df, flags, psd_mode));
-   return plan_exec(&P, m2mf, m2mr, m2o2mr, m3mf, m3mr);
+   PoolLoan loan(P.B);
+   int rc = plan_setup(&P, p, nfh, df, flags, psd_mode);
+   if (rc == 0) rc = plan_exec(&P, m2mf, m2mr, m2o2mr, m3mf, m3mr);
+   if (rc != 0) (void)hipDeviceSynchronize();                // nothing in flight on kept buffers
+   return rc;
 }
 
 int bsahip__points_sum(const bsahip_problem *p, int32_t npts, const double *fi, const double *fj,
@@ -1330,35 +1549,36 @@ int bsahip_classic_bispectra_sel(const bsahip_problem *p, int32_t nfh, double df
    if (nfh > 46341) return fail(BSAHIP_EINVAL, "nfh too large for one selected bispectrum");
    Bufs &B = oneshot_bufs();
    Prob D;
-   CHK(load_problem(p, 0, B, D));
-   const long ncol = diag ? D.nm : (long)D.nm * D.nm * D.nm;
+   CHK(validate(p));
+   const long ncol = diag ? p->nm : (long)p->nm * p->nm * p->nm;
+   const int nh = nfh, nf = 2 * nh - 1, nu = exact ? nf : nh;
    std::vector<int> s0(nsel);
+   std::vector<double> fl(nu);
+   for (int u = 0; u < nu; ++u) fl[u] = (double)u * df;
    for (int s = 0; s < nsel; ++s) {
       if (sel[s] < 1 || sel[s] > ncol)
          return fail(BSAHIP_EINVAL, "selection index out of 1..NM^3 (1..NM with ONLY_DIAG)");
       s0[s] = sel[s] - 1;
    }
-   const int nh = nfh, nf = 2 * nh - 1;
    const size_t npts = (size_t)nf * nf, nout = npts * (size_t)nsel;
    int *dsel;
-   double *ob = nullptr, *orr = nullptr;
-   CHK(upload(B, "sel", s0, &dsel));
+   double *dfl, *ob = nullptr, *orr = nullptr;
+   Pack pk;
+   pk.add(s0, &dsel);
+   pk.add(fl, &dfl);
+   CHK(load_problem(p, 0, B, D, &pk, !diag));
    if (bfm) CHK(B.get("bisp_sel_f", nout, &ob));
    if (brm) CHK(B.get("bisp_sel_r", nout, &orr));
    const dim3 gs((unsigned)((npts + 255) / 256), (unsigned)nsel);
    if (diag) {
       DiagTab X;
       double *T;
-      CHK(diag_tables(B, D, nh, df, X));
+      CHK(diag_tables(B, D, dfl, nh, df, X));
       CHK(diag_products(B, D, nh, X, &T));
       k_diag_bisp_sel<<<gs, 256, 0, g.s>>>(T, nh, X.H, 2 * nh - 1, dsel, ob, orr);
    } else {
-      const int nu = exact ? nf : nh;
       const long ldU = (long)D.nm * nu;
-      std::vector<double> fl(nu);
-      for (int u = 0; u < nu; ++u) fl[u] = (double)u * df;
-      double *dfl, *U;
-      CHK(upload(B, "fl", fl, &dfl));
+      double *U;
       CHK(B.get("U", (size_t)D.K * ldU, &U));
       CHK(build_table(B, D, dfl, nu, nu, U, ldU));
 #define LAUNCH_SEL(PR)                                                                        \
@@ -1418,7 +1638,7 @@ int bsahip_diag_psd_points(const bsahip_problem *p, int32_t npts, const double *
    if (npts == 0) return 0;
    Bufs &B = oneshot_bufs();
    Prob D;
-   CHK(load_problem(p, 0, B, D));
+   CHK(load_problem(p, 0, B, D, nullptr, false));
    std::vector<double> af(npts);
    for (int q = 0; q < npts; ++q) af[q] = std::fabs(f[q]);
    std::vector<double> uq(af);
@@ -1482,33 +1702,36 @@ int bfm_points_impl(const bsahip_problem *p, int32_t npts, const double *fi, con
    if (npts == 0) return 0;
    Bufs &B = oneshot_bufs();
    Prob D;
-   CHK(load_problem(p, 0, B, D));
+   CHK(validate(p));
    std::vector<double> uq;
    std::vector<int> i1, i2, i3;
    point_tables(npts, fi, fj, uq, i1, i2, i3);
+   int *di1, *di2, *di3;
+   double *dfl, *df1, *df2;
+   Pack pk;
+   pk.add(uq, &dfl);
+   pk.add(i1, &di1);
+   pk.add(i2, &di2);
+   pk.add(i3, &di3);
+   pk.add(fi, npts * sizeof(double), reinterpret_cast<void **>(&df1));
+   pk.add(fj, npts * sizeof(double), reinterpret_cast<void **>(&df2));
+   CHK(load_problem(p, 0, B, D, &pk, !diag));
    if (diag) {
       const long tot = (long)npts * D.nm;
       if (tot > 0xffffff00L) return fail(BSAHIP_EUNSUPPORTED, "npts * NM exceeds 2^32 values");
-      double *sq, *ob, *df1, *df2;
-      int *d1, *d2, *d3;
+      double *sq, *ob;
       long *ds;
       std::vector<long> slot(npts);
       for (int q = 0; q < npts; ++q) slot[q] = q;
       CHK(diag_sq_table(B, D, uq, fmax, &sq));
-      CHK(upload(B, "i1", i1, &d1));
-      CHK(upload(B, "i2", i2, &d2));
-      CHK(upload(B, "i3", i3, &d3));
       CHK(upload(B, "dg_slot", slot, &ds));
       CHK(B.get("bfm_out", (size_t)tot, &ob));
       k_diag_points<<<(unsigned)((tot + 255) / 256), 256, 0, g.s>>>(
-         sq, (int)uq.size(), D.nnl, D.kv, D.pa_k, D.pb_k, D.K, D.nm, npts, d1, d2, d3, ds, ob);
+         sq, (int)uq.size(), D.nnl, D.kv, D.pa_k, D.pb_k, D.K, D.nm, npts, di1, di2, di3, ds, ob);
       HIPC(hipGetLastError());
       HIPC(hipMemcpyAsync(bfm, ob, (size_t)tot * sizeof(double), hipMemcpyDeviceToHost, g.s));
       if (brm) {
-         std::vector<double> f1(fi, fi + npts), f2(fj, fj + npts);
          double *orr;
-         CHK(upload(B, "f1", f1, &df1));
-         CHK(upload(B, "f2", f2, &df2));
          CHK(B.get("brm_out", (size_t)tot, &orr));
          HIPC(hipMemcpyAsync(orr, ob, (size_t)tot * sizeof(double), hipMemcpyDeviceToDevice, g.s));
          k_frf_apply<<<(unsigned)((tot + 255) / 256), 256, 0, g.s>>>(
@@ -1527,15 +1750,7 @@ int bfm_points_impl(const bsahip_problem *p, int32_t npts, const double *fi, con
       return fail(BSAHIP_EUNSUPPORTED, "npts * NM^3 exceeds 2^32 bispectrum values in one call");
    // uq is ascending: rows u0.. lie beyond the grid
    const long u0 = fmax > 0.0 ? std::upper_bound(uq.begin(), uq.end(), fmax * (1.0 + 1e-12)) - uq.begin() : nu;
-   std::vector<double> f1(fi, fi + npts), f2(fj, fj + npts);
-   int *di1, *di2, *di3;
-   double *dfl, *df1, *df2, *ob, *orr = nullptr;
-   CHK(upload(B, "fl", uq, &dfl));
-   CHK(upload(B, "i1", i1, &di1));
-   CHK(upload(B, "i2", i2, &di2));
-   CHK(upload(B, "i3", i3, &di3));
-   CHK(upload(B, "f1", f1, &df1));
-   CHK(upload(B, "f2", f2, &df2));
+   double *ob, *orr = nullptr;
    CHK(B.get("bfm_out", nm3 * npts, &ob));
    if (brm) CHK(B.get("brm_out", nm3 * npts, &orr));
    const unsigned nblk = (unsigned)((tot + 255) / 256);
@@ -1592,7 +1807,7 @@ int bsahip_frf_apply(const bsahip_problem *p, int32_t flags, int32_t kind, int64
       return fail(BSAHIP_EINVAL, "NULL frequencies or data");
    Bufs &B = oneshot_bufs();
    Prob D;
-   CHK(load_problem(p, 0, B, D));
+   CHK(load_problem(p, 0, B, D, nullptr, false));
    const long nm = D.nm, nm2 = diag ? nm : nm * nm, nm3 = diag ? nm : nm * nm * nm;
    const long nf2 = kind == BSAHIP_FRF_GRID ? n2 : (kind == BSAHIP_FRF_POINTS ? n1 : 0);
    const double tot_d = kind == BSAHIP_FRF_PSD ? (double)n1 * nm2

@@ -1,0 +1,74 @@
+"""One-shot calls share scratch and staging memory: calls of growing and shrinking
+sizes through different entry points, in any order, from several threads and after a
+refused call, give what each gives by itself; results above the staged size and inputs
+above the staged part size too.  Ordered sums make equal calls equal bit for bit."""
+import threading
+
+import numpy as np
+import pytest
+
+from bsalib_amd import abi, synth
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _tower(nn, nm, nfh, comps=(1, 3)):
+    return synth.tower(nn=nn, nm=nm, comps=comps, natf=np.linspace(0.2, 3.0, nm), nfreqs=nfh,
+                       df=4.0 / nfh, seed=nn + nm)
+
+
+def _calls():
+    """One-shot calls; 42 modes and 530 nodes pass the staged sizes, 300 nodes with 513
+    frequencies the scratch that is kept."""
+    big, mid, small, many = _tower(530, 3, 9), _tower(120, 17, 40), _tower(7, 2, 17), _tower(30, 42, 5)
+    wide = _tower(300, 15, 513, (1, 2, 3))
+    pts = np.linspace(-3.0, 3.0, 23), np.linspace(2.5, -1.5, 23)
+
+    def run(p, **kw):
+        return lambda: {k: v for k, v in abi.classic_run(p, deterministic=True, **kw).items()}
+
+    return [run(mid), run(small), run(big), run(many), run(small, exact=True), run(mid, bisp=False),
+            run(mid, psd=False, prec="bf16x3"), run(wide, bisp=False, prec="bf16x3"),
+            lambda: abi.classic_bispectra_sel(small, [1, 8]),
+            lambda: abi.classic_bispectra_sel(mid, [5], exact=True),
+            lambda: abi.classic_bispectra_sel(mid, [5], only_diag=True),
+            lambda: dict(zip("fr", abi.bfm_points(mid, *pts))),
+            lambda: dict(zip("fr", abi.bfm_points(small, *pts, only_diag=True)))]
+
+
+def _same(a, b):
+    return all(np.array_equal(a[k], b[k]) for k in a)
+
+
+def test_order_and_threads(gpu_lib):
+    calls = _calls()
+    want = [c() for c in calls]
+    rng = np.random.default_rng(1)
+    for i in np.concatenate([rng.permutation(len(calls)) for _ in range(3)]):
+        if i % 4 == 0:
+            with pytest.raises(abi.BsaHipError):
+                abi.classic_bispectra_sel(_tower(7, 2, 17), [0])
+        assert _same(want[i], calls[i]()), i
+    bad = []
+
+    def work(seed):
+        for i in np.random.default_rng(seed).permutation(len(calls)):
+            if not _same(want[i], calls[i]()):
+                bad.append(i)
+
+    ts = [threading.Thread(target=work, args=(s,)) for s in (2, 3, 4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
+
+
+def test_second_moments_above_the_staged_sizes(gpu_lib):
+    """Tolerance 1e-12 of the largest entry, sums of at most 2 * 530 * 17 products."""
+    for p in (_tower(530, 3, 9), _tower(30, 42, 5)):
+        o = O.modal_psd(p)
+        r = abi.classic_run(p)
+        for k in ("m2mf", "m2mr", "m2o2mr"):
+            assert np.abs(r[k] - o[k]).max() < 1e-12 * np.abs(o[k]).max()
