@@ -84,7 +84,9 @@ __global__ void k_pbt(const double *__restrict__ pb, int nm, int K, int nmp, dou
 // 301 points take 18 us where one value per lane took 209);
 // out[slot[pt]*nm3 + m + col*nm] = B (slot null: q0 + pt).
 // ---------------------------------------------------------------------------
-#define BKC 16   // K chunk staged in LDS
+// K chunk staged in LDS: K is a multiple of 32; 16 took 17.5 us where 32 takes 15.2 at 301
+// points, 8 modes, and 2.20 where 2.14 ms at 35000 points, 10 modes
+#define BKC 32
 
 template <int MT, int TPW>
 __global__ __launch_bounds__(512) void k_bfm_batch(
@@ -995,10 +997,19 @@ int bfm_batch(const Prob &D, const double *V, const double *PB, int nmp, int npt
    return 0;
 }
 
-// BFM at the points (f1[q], f2[q]) into out + slot[q]*nm3, in chunks of at
-// most MSH_CHUNK points so the A tables stay small (3 distinct |f| per point
-// at most).
-constexpr int MSH_CHUNK = 8192;
+// BFM at the points (f1[q], f2[q]) into out + slot[q]*nm3, in chunks so the A tables stay
+// small (3 distinct |f| per point at most): 16384 points where their table takes at most
+// 8 GB, never fewer than 8192.  Points of one chunk share the rows of equal |f|: 8192
+// points projected 3.7 ms of tables for 200 nodes, 2 components, 10 modes, 16384 3.1,
+// 21845 (65535 frequencies, the most of one table) no less in the sum.
+constexpr size_t MSH_CHUNK = 8192, MSH_CHUNK_MAX = 16384;
+
+size_t msh_chunk(const bsahip_mesher *M)
+{
+   const size_t row = (size_t)M->D.K * M->nmp * sizeof(double);
+   return std::max(MSH_CHUNK, std::min(MSH_CHUNK_MAX, ((size_t)8 << 30) / (3 * row)));
+}
+
 
 int msh_eval_chunk(bsahip_mesher *M, int npts, const double *f1, const double *f2,
                    const long *slot_p, double *out);
@@ -1006,8 +1017,9 @@ int msh_eval_chunk(bsahip_mesher *M, int npts, const double *f1, const double *f
 int msh_eval(bsahip_mesher *M, const std::vector<double> &f1, const std::vector<double> &f2,
              const std::vector<long> &slot, double *out)
 {
-   for (size_t q0 = 0; q0 < f1.size(); q0 += MSH_CHUNK) {
-      const int n = (int)std::min<size_t>(MSH_CHUNK, f1.size() - q0);
+   const size_t chunk = msh_chunk(M);
+   for (size_t q0 = 0; q0 < f1.size(); q0 += chunk) {
+      const int n = (int)std::min(chunk, f1.size() - q0);
       CHK(msh_eval_chunk(M, n, f1.data() + q0, f2.data() + q0, slot.data() + q0, out));
    }
    return 0;
