@@ -14,8 +14,8 @@
 // epilogue (k_gsym_diag), each T value formed once and never stored, and the second
 // moments its modal PSD kernel (k_m2 with diag).  Bound by launches and latency at
 // these sizes: T stored by a GEMM per mode, read back over the whole plane and a
-// serial loop over k per PSD value took 530 us for 20 modes, 1000 nodes and
-// components, 257 frequencies; now 89 us, with the 15 us of k_m2 beside.  Selected bispectra
+// serial loop over k per PSD value took 530 us for 500 nodes with 2 components, 20
+// modes, 257 frequencies; now 80 us, with the 15 us of k_m2 beside.  Selected bispectra
 // still store their T_m (one GEMM per mode).
 
 // X[k*ldX + u] = S_k(u df), zero for u >= nh and in the padding rows k >= kv; from the
