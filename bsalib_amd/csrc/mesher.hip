@@ -1677,14 +1677,18 @@ int bsahip_mesher_run_tiles(bsahip_mesher *m, const int32_t *levels, double *til
    }
    if (m3mf) HIPC(hipMemcpyAsync(m3mf, acc, nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
    HIPC(hipStreamSynchronize(g.s));
+   if (tile_m3mr)
+      // a mirror image has the slot of its first tile, integrated for both
+      for (size_t k = 0; k < nt; ++k) {
+         const long j = msh_image(m, levels, k);
+         if (j >= 0 && j < (long)k)
+            std::copy(tile_m3mr + j * nm3, tile_m3mr + (j + 1) * nm3, tile_m3mr + k * nm3);
+      }
    if (m3mr) {
       if (tile_m3mr) {
          // tile by tile, so that each pass reads one contiguous slot
          std::fill(m3mr, m3mr + nm3, 0.0);
          for (size_t k = 0; k < nt; ++k) {
-            const long j = msh_image(m, levels, k);      // an image: the slot of its first tile
-            if (j >= 0 && j < (long)k)
-               std::copy(tile_m3mr + j * nm3, tile_m3mr + (j + 1) * nm3, tile_m3mr + k * nm3);
             const double *c = tile_m3mr + k * nm3;
             for (size_t q = 0; q < nm3; ++q) m3mr[q] += c[q];
          }

@@ -6,6 +6,7 @@ the exported integrand (bsahip_mesher_export, another kernel), taken with math.f
 Tolerance 1e-12 of the largest entry: a tile's sum holds at most 257^2 terms, each
 correct to a few ulp (1e-15 relative), accumulated over at most 257 + 257 / 4 chained
 roundings, with terms that may cancel by some two digits."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -94,4 +95,33 @@ def test_mirrored_tiles_at_unequal_levels(gpu_lib, only_diag):
         assert r["evals_post"] == int(n.sum())
         assert r["brm_points"] == int(np.sum(np.prod(M.export(levels=lv)["dims"].astype(np.int64),
                                                      axis=1)))
+    M.close()
+
+
+@pytest.mark.parametrize("only_diag", [False, True])
+def test_tiles_alone(gpu_lib, only_diag):
+    """bsahip_mesher_run_tiles asked for the tiles' moments only, with each of the other
+    outputs left out in turn: every slot is the one of the call that takes them all, the
+    slots of mirror images among them (1e-13: the order of the atomic sums varies)."""
+    M = _mesher(3, 5, 2, 8) if not only_diag else abi.Mesher(
+        synth.tower(nn=4, nm=3, comps=(1, 3), natf=np.linspace(0.2, 3.0, 3),
+                    xi=np.linspace(0.02, 0.05, 3), nfreqs=9, df=0.5, seed=3),
+        bkg_base_rfmnt=5, tile_cells=2, bkg_peakw=8.0, brm_cells=8, only_diag=True)
+    geom, rule = M.tiles()
+    twin = {tuple(np.round(g[:4], 9)) for g in geom}
+    assert any(tuple(np.round([-g[1], -g[0], -g[3], -g[2]], 9)) in twin for g in geom)
+    want = M.run(per_tile=True)
+    assert np.abs(want["tile_m3mr"]).max(axis=1).min() > 0.0
+    ptr = lambda a: None if a is None else a.ctypes.data_as(C.POINTER(C.c_double))  # noqa: E731
+    for with_f, with_r in ((False, False), (True, False), (False, True)):
+        tiles = np.full((M.ntiles, M.nc), np.nan)
+        f = np.zeros(M.nc) if with_f else None
+        r = np.zeros(M.nc) if with_r else None
+        assert abi.lib().bsahip_mesher_run_tiles(M.h, None, ptr(tiles), ptr(f), ptr(r), None) == 0
+        for k in range(M.ntiles):
+            w = want["tile_m3mr"][k]
+            assert np.abs(tiles[k] - w).max() <= 1e-13 * np.abs(w).max(), (k, with_f, with_r)
+        for got, key in ((f, "m3mf"), (r, "m3mr")):
+            if got is not None:
+                assert np.abs(got - want[key]).max() <= 1e-13 * np.abs(want[key]).max()
     M.close()
