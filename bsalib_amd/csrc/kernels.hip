@@ -161,14 +161,14 @@ __global__ void k_frf_table(const double *__restrict__ Mm, const double *__restr
 // VLAY: the point layout U[(q*K + k)*ldU + y] of the Mesher (ldU modes, zero from nm
 // on, K rows) instead of U[k*ldU + y*row_stride + q]; its padding rows k are cleared.
 // ---------------------------------------------------------------------------
-// exp(x) of the projection's inner loop: x = n ln 2 + r, |r| <= ln 2 / 2 (Cody-Waite,
-// the high part of ln 2 cut to 33 bits so that n times it is exact), a degree-11
-// polynomial on r whose coefficients interpolate (e^r - 1 - r) / r^2 at the Chebyshev
-// nodes (relative error 2e-17), and a power of two.  0.85 ulp at most (5000 arguments
-// from -690 to 0 against 60 digits), within the 1 ulp of the library's exp, whose
-// steps these are; here the coefficients stay in scalar registers, where the library
-// call reloads eighteen vector registers with them for every value.  As there, results
-// below the subnormals are 0, those above the largest double infinite, NaN stays.
+// exp(x) of the projection's inner loop by Cody-Waite reduction: x = n ln 2 + r,
+// |r| <= ln 2 / 2 (the high part of ln 2 cut to 33 bits so that n times it is exact), a
+// degree-11 polynomial on r whose coefficients interpolate (e^r - 1 - r) / r^2 at the
+// Chebyshev nodes (relative error 2e-17), and a power of two.  0.85 ulp at most (5000
+// arguments from -690 to 0 against 60 digits), within the 1 ulp of the library's exp;
+// here the coefficients stay in scalar registers, where the library call reloads eighteen
+// vector registers with them for every value.  Results below the subnormals are 0, those
+// above the largest double infinite.
 struct ExpC {
    double magic, inv, hi, lo, c3, c4, c5, c6, c7, c8, c9, c10, c11;
 };
@@ -186,8 +186,8 @@ __device__ __forceinline__ ExpC exp_consts()
    return e;
 }
 
-// `one`: 1, or NaN where x is to give NaN (the clamps drop it)
-__device__ __forceinline__ double exp_fast(double x, double one, const ExpC &e)
+// NaN is left to the caller: the clamps drop it
+__device__ __forceinline__ double exp_fast(double x, const ExpC &e)
 {
    x = __builtin_fmin(__builtin_fmax(x, -800.0), 720.0);
    const double t = __builtin_fma(x, e.inv, e.magic);
@@ -205,7 +205,7 @@ __device__ __forceinline__ double exp_fast(double x, double one, const ExpC &e)
    p = __builtin_fma(p, r, e.c3);
    p = __builtin_fma(p, r, 0.5);
    p = __builtin_fma(p, r, 1.0);
-   p = __builtin_fma(p, r, one);
+   p = __builtin_fma(p, r, 1.0);
    return __builtin_amdgcn_ldexp(p, n);
 }
 
@@ -264,14 +264,16 @@ __device__ __forceinline__ void project_wave(const ProjArgs &P, long wid, int tc
 #pragma unroll
       for (int r = 0; r < MT; ++r) acc[f][r] = (d4){0.0, 0.0, 0.0, 0.0};
    const ExpC ec = exp_consts();
+   unsigned long long nan = 0;                // lanes that met a NaN of ln rho
    // one MFMA step: ln rho l of the lane's (j, i), Psi_a a of its (y, j), s_j
    auto step = [&](double l, const double (&a)[MT], const double (&sj)[F]) {
-      // |f| = 0 gives 1 even for rho == 0: the infinity becomes a finite number
-      const double one = l == l ? 1.0 : l;
+      // |f| = 0 gives 1 for any rho: the infinity of rho == 0 becomes a finite number, the
+      // NaN of rho < 0 is noted and joins its column at the end where |f| is another
+      nan |= __ballot(l != l);
       const double lc = __builtin_fmin(__builtin_fmax(l, -0x1.fffffffffffffp1023), 0x1.fffffffffffffp1023);
 #pragma unroll
       for (int f = 0; f < F; ++f) {
-         const double e = exp_fast(af[f] * lc, one, ec) * sj[f];
+         const double e = exp_fast(af[f] * lc, ec) * sj[f];
 #pragma unroll
          for (int r = 0; r < MT; ++r)
             acc[f][r] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], e, acc[f][r], 0, 0, 0);
@@ -325,6 +327,11 @@ __device__ __forceinline__ void project_wave(const ProjArgs &P, long wid, int tc
       for (int f = 0; f < F; ++f) x[f] = j < nnl ? sqq[f][jc] : 0.0;
       step(lnt[(size_t)jc * nnl], a, x);
    }
+   nan |= nan >> 32;
+   nan |= nan >> 16;
+   const double bad = (nan >> lr) & 1 ? __builtin_nan("") : 0.0;      // the lane's column
+   // s_i; a frequency that is not a number, or infinite (rho_ii = 1), gives NaN as well
+   auto row = [&](int f) { return sqq[f][i] + (af[f] - af[f]) + (af[f] == 0.0 ? 0.0 : bad); };
    const int k = tc * nnlp + i;
    const bool ok = i < nnl;
    if constexpr (VLAY) {
@@ -332,7 +339,7 @@ __device__ __forceinline__ void project_wave(const ProjArgs &P, long wid, int tc
 #pragma unroll
       for (int f = 0; f < F; ++f) {
          if (q0 + f >= nfl) break;
-         const double si = ok ? sqq[f][i] : 0.0;
+         const double si = ok ? row(f) : 0.0;
          double *d = U + ((size_t)(q0 + f) * K + k) * ldU + y0 + lk;
 #pragma unroll
          for (int r = 0; r < MT; ++r)
@@ -344,7 +351,7 @@ __device__ __forceinline__ void project_wave(const ProjArgs &P, long wid, int tc
       if (!ok) return;
       double si[F];
 #pragma unroll
-      for (int f = 0; f < F; ++f) si[f] = sqq[f][i];
+      for (int f = 0; f < F; ++f) si[f] = row(f);
 #pragma unroll
       for (int r = 0; r < MT; ++r)
 #pragma unroll

@@ -74,3 +74,36 @@ def test_limits_of_the_coherence(gpu_lib):
     _check(p, np.array([0.0, 0.5, 1.0, 1.05, 2.0, 3.9]))
     p.nod_corr[at[45], :] = -1.0      # no real power: NaN stays NaN
     assert np.isnan(abi.modal_psd_points(p, np.array([0.5]))).any()
+
+
+@pytest.mark.parametrize("nm", [3, 20, 40, 60])
+@pytest.mark.parametrize("bad", [-1.0, float("nan")])
+def test_zero_frequency_with_no_real_power(gpu_lib, nm, bad):
+    """rho < 0 or NaN: rho^0 is 1 all the same, in every place of a group of frequencies
+    and in both table layouts; every other power is NaN."""
+    p = synth.tower(nn=13, nm=nm, comps=(1, 3), natf=np.linspace(0.2, 3.0, nm), seed=5)
+    one = synth.tower(nn=13, nm=nm, comps=(1, 3), natf=np.linspace(0.2, 3.0, nm), seed=5)
+    at = [3, 20, 77]                       # pairs of different nodes
+    p.nod_corr, one.nod_corr = p.nod_corr.copy(), one.nod_corr.copy()
+    p.nod_corr[at], one.nod_corr[at] = bad, 1.0
+    for f in (np.zeros(1), np.array([0.5, 0.0, 1.0, 0.0, 0.0, 2.0, 0.25, 3.0, 0.0])):
+        r, ref = abi.modal_psd_points(p, f), _ref(one, f)
+        z = f == 0.0
+        assert np.isnan(r[:, :, ~z]).all()
+        assert np.abs(r[:, :, z] - ref[:, :, z]).max() < 1e-12 * np.abs(ref[:, :, z]).max()
+    if nm <= 32:
+        bfm, _ = abi.bfm_points(p, np.zeros(2), np.zeros(2))
+        want = O.msh_points(one, np.zeros(2), np.zeros(2))
+        assert np.abs(bfm - want).max() < 1e-12 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("psd_id", [1, 2, 3, 5])
+def test_frequencies_that_are_not_finite(gpu_lib, psd_id):
+    """NaN and infinite frequencies give NaN and leave their neighbours alone."""
+    p = synth.tower(nn=9, nm=3, comps=(1, 3), natf=np.linspace(0.2, 3.0, 3), seed=5)
+    b = abi.Bound(p, psd_id=psd_id)
+    f = np.array([0.0, np.nan, 1.0, np.inf, 2.0, -np.inf, 0.5, 3.0, np.nan])
+    ok = np.isfinite(f)
+    r = abi.modal_psd_points(p, f, bound=b)
+    assert np.isnan(r[:, :, ~ok]).all()
+    assert np.array_equal(r[:, :, ok], abi.modal_psd_points(p, f[ok], bound=b))
