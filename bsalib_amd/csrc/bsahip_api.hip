@@ -1398,6 +1398,11 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
    const int nh = nfh, nft = 2 * nh - 1, nm = D.nm, K = D.K;
    const double d = p->pulsation ? df * 2.0 * M_PI : df;
    const bool psd = !(flags & BSAHIP_NO_PSD), bisp = !(flags & BSAHIP_NO_BISP);
+   int br, bc;
+   f64_shape(nh, nm, F64_LEAST_DIAG, br, bc);
+   const long items = f64_tiles(nh, br, bc) * nm;
+   if (bisp && items > 0xffffffL)
+      return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: use a coarser grid or fewer modes");
    DiagTab T;
    double *mom;
    CHK(diag_tables(B, D, dfl, nh, df, T));
@@ -1432,11 +1437,6 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
       a.epi_plain = (flags & BSAHIP_EPI_GENERIC) ? 1 : 0;
       a.m3f = m3f;
       a.m3r = m3r;
-      int br, bc;
-      f64_shape(nh, nm, F64_LEAST_DIAG, br, bc);
-      const long items = f64_tiles(nh, br, bc) * nm;
-      if (items > 0xffffffL)
-         return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: use a coarser grid or fewer modes");
       if (br == 4) k_gsym_diag<4, 2><<<(unsigned)items, 256, 0, g.s>>>(a, nm);
       else if (br == 2) k_gsym_diag<2, 2><<<(unsigned)items, 256, 0, g.s>>>(a, nm);
       else k_gsym_diag<1, 1><<<(unsigned)items, 256, 0, g.s>>>(a, nm);
@@ -1471,7 +1471,9 @@ int bsahip__classic_moments(const bsahip_problem *p, int32_t nfh, double df, int
       if (psd_mode != 0) return fail(BSAHIP_EUNSUPPORTED, "the ONLY_DIAG model has no BsaCL form");
       if (flags & BSAHIP_DETERMINISTIC)
          return fail(BSAHIP_EUNSUPPORTED, "the ONLY_DIAG model has no fixed-order mode");
-      return classic_diag(p, nfh, df, flags, m2mf, m2mr, m2o2mr, m3mf, m3mr);
+      const int rc = classic_diag(p, nfh, df, flags, m2mf, m2mr, m2o2mr, m3mf, m3mr);
+      if (rc != 0) (void)hipDeviceSynchronize();             // nothing in flight on the one-shot scratch
+      return rc;
    }
    bsahip_plan P;
    PoolLoan loan(P.B);

@@ -72,3 +72,19 @@ def test_second_moments_above_the_staged_sizes(gpu_lib):
         r = abi.classic_run(p)
         for k in ("m2mf", "m2mr", "m2o2mr"):
             assert np.abs(r[k] - o[k]).max() < 1e-12 * np.abs(o[k]).max()
+
+
+def test_refused_diagonal_grid(gpu_lib):
+    """A diagonal run whose plane is too large for one launch is refused before anything
+    starts on the side stream; the calls after it have the scratch to themselves."""
+    p = _tower(9, 4, 33)
+    o = O.classic_diag(p)
+    want = abi.classic_run(p, only_diag=True)
+    huge = _tower(1, 256, 33100, (1,))
+    for _ in range(3):
+        with pytest.raises(abi.BsaHipError, match="too large"):
+            abi.classic_run(huge, only_diag=True)
+        r = abi.classic_run(p, only_diag=True)
+        for k in ("m2mf", "m2mr", "m3mf", "m3mr"):
+            assert np.abs(r[k] - want[k]).max() <= 1e-14 * np.abs(want[k]).max()
+            assert np.abs(r[k] - o[k]).max() < 1e-12 * np.abs(o[k]).max()
