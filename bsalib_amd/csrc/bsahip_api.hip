@@ -183,7 +183,7 @@ constexpr size_t STAGE_UP = (size_t)4 << 20, STAGE_DOWN = (size_t)512 << 10, PAR
                  SUMS_DOWN = (size_t)64 << 10;
 
 // Uploads gathered into one device buffer (src null: room only).  The host arrays have to
-// live until send().
+// live until send(), which has read them when it returns.
 struct Pack {
    struct Part {
       const void *src;
@@ -208,6 +208,7 @@ struct Pack {
       char *dev;
       CHK(B.get(name, n, &dev));
       size_t lo = 0, hi = 0;                                 // staged, not yet sent
+      bool direct = false;                                   // the caller's memory is read
       const auto flush = [&]() -> int {
          if (hi > lo) {
             HIPC(hipMemcpyAsync(dev + lo, g.stage, hi - lo, hipMemcpyHostToDevice, g.s));
@@ -223,6 +224,7 @@ struct Pack {
             CHK(flush());
             HIPC(hipMemcpyAsync(dev + p.off, p.src, p.bytes, hipMemcpyHostToDevice, g.s));
             lo = hi = p.off + p.bytes;
+            direct = true;
             continue;
          }
          if (p.off + p.bytes - lo > STAGE_UP) CHK(flush());
@@ -234,6 +236,9 @@ struct Pack {
          hi = p.off + p.bytes;
       }
       CHK(flush());
+      // a copy out of pageable memory is over when it returns, one out of the caller's
+      // pinned memory is not
+      if (direct) HIPC(hipStreamSynchronize(g.s));
       parts.clear();
       n = 0;
       return 0;

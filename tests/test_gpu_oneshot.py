@@ -2,6 +2,7 @@
 sizes through different entry points, in any order, from several threads and after a
 refused call, give what each gives by itself; results above the staged size and inputs
 above the staged part size too.  Ordered sums make equal calls equal bit for bit."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -88,3 +89,36 @@ def test_refused_diagonal_grid(gpu_lib):
         for k in ("m2mf", "m2mr", "m3mf", "m3mr"):
             assert np.abs(r[k] - want[k]).max() <= 1e-14 * np.abs(want[k]).max()
             assert np.abs(r[k] - o[k]).max() < 1e-12 * np.abs(o[k]).max()
+
+
+def test_pinned_coherence_table(gpu_lib, tmp_path):
+    """A coherence table in pinned memory, larger than the staged parts, is read when the
+    call returns, also by the calls that do not wait for their results (a Mesher loaded
+    from its checkpoint): the caller may overwrite it."""
+    def deck():
+        return synth.tower(nn=800, nm=2, comps=(1, 2), natf=np.array([0.3, 0.8]),
+                           xi=np.array([0.02, 0.03]), nfreqs=9, df=0.5, seed=3)
+
+    kw = dict(bkg_base_rfmnt=4, tile_cells=2, bkg_peakw=2.0)
+    m = abi.Mesher(deck(), **kw)
+    want = m.run(levels=2)
+    m.save(tmp_path / "zones")
+    m.close()
+    p = deck()
+    table = p.nod_corr
+    at = C.c_void_p()                   # of the HIP runtime that the library is linked to
+    assert gpu_lib.lib().hipHostMalloc(C.byref(at), C.c_size_t(8 * table.size), C.c_uint(0)) == 0
+    pinned = np.ctypeslib.as_array(C.cast(at, C.POINTER(C.c_double)), (table.size,))
+    for _ in range(3):
+        p.nod_corr = pinned.reshape(table.shape, order="F")
+        p.nod_corr[:] = table
+        b = abi.Bound(p)
+        assert np.shares_memory(b.keep["nod_corr"], pinned)
+        m = abi.Mesher(p, bound=b, load=tmp_path / "zones", **kw)
+        pinned[::-1] = 0.5
+        r = m.run(levels=2)
+        m.close()
+        for k in ("m3mf", "m3mr"):
+            assert np.abs(r[k] - want[k]).max() <= 1e-12 * np.abs(want[k]).max()
+    del b, p
+    assert gpu_lib.lib().hipHostFree(at) == 0
