@@ -944,7 +944,16 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    if (nfh < 2 || !(df > 0.0)) return fail(BSAHIP_EINVAL, "need nfh >= 2 and df > 0");
    if (flags & BSAHIP_ONLY_DIAG)
       return fail(BSAHIP_EUNSUPPORTED, "the ONLY_DIAG model runs through bsahip_classic_run");
-   const int nu = (flags & BSAHIP_SUM_EXACT) ? 2 * nfh - 1 : nfh;
+   CHK(validate(p));
+   const long nul = (flags & BSAHIP_SUM_EXACT) ? 2L * nfh - 1 : nfh;
+   const int tile = (flags & BSAHIP_PREC_MASK) == BSAHIP_PREC_FP64 ? 64 : T2;
+   const long nt = (p->nm * nul + tile - 1) / tile;
+   // one workgroup of 256 threads per (tile pair, mode): the launch's global
+   // size must fit 32 bits.  Before any table of that size is made.
+   if ((double)nt * (nt + 1) / 2 * p->nm * 256.0 > 4294967295.0)
+      return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: (tile pairs x modes) x 256 "
+                                       "threads exceeds 2^32; use a coarser grid or fewer modes");
+   const int nu = (int)nul;
    std::vector<double> fl(nu);
    for (int u = 0; u < nu; ++u) fl[u] = (double)u * df;
    Pack pk;
@@ -960,18 +969,11 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    // block may span two modes, and the epilogue masks the other mode's rows
    P->nhp = P->nu;
    P->rows = P->D.nm * P->nhp;
-   const int tile = (P->prec == BSAHIP_PREC_FP64) ? 64 : T2;
-   P->ntile = (P->rows + tile - 1) / tile;
+   P->ntile = (int)nt;
    if (P->f64_br == 0) f64_shape(P->rows, P->D.nm, F64_LEAST, P->f64_br, P->f64_bc);
    P->ldU = (long)round_up(P->rows, T2);
    P->nft = 2 * P->nu - 1;
    P->d = p->pulsation ? df * 2.0 * M_PI : df;
-   const long npairs = (long)P->ntile * (P->ntile + 1) / 2;
-   // one workgroup of 256 threads per (tile pair, mode): the launch's global
-   // size must fit 32 bits
-   if (npairs * P->D.nm * 256L > 0xffffffffL)
-      return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: (tile pairs x modes) x 256 "
-                                       "threads exceeds 2^32; use a coarser grid or fewer modes");
    CHK(P->B.get("U", (size_t)P->D.K * P->ldU, &P->U));
    CHK(zero_padding(P->D, P->nhp, P->U, P->ldU));      // the runs write the valid entries only
    CHK(P->B.get("H", (size_t)P->D.nm * P->nft, &P->H));
@@ -1392,6 +1394,13 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
    if ((flags & BSAHIP_PREC_MASK) != BSAHIP_PREC_FP64)
       return fail(BSAHIP_EUNSUPPORTED, "the ONLY_DIAG model runs in FP64");
    if (nfh < 2 || !(df > 0.0)) return fail(BSAHIP_EINVAL, "need nfh >= 2 and df > 0");
+   CHK(validate(p));
+   const bool psd = !(flags & BSAHIP_NO_PSD), bisp = !(flags & BSAHIP_NO_BISP);
+   int br, bc;
+   f64_shape(nfh, p->nm, F64_LEAST_DIAG, br, bc);
+   const long items = f64_tiles(nfh, br, bc) * p->nm;
+   if (bisp && items > 0xffffffL)
+      return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: use a coarser grid or fewer modes");
    Bufs &B = oneshot_bufs();
    Prob D;
    Pack pk;
@@ -1402,12 +1411,6 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
    CHK(load_problem(p, 0, B, D, &pk, false));
    const int nh = nfh, nft = 2 * nh - 1, nm = D.nm, K = D.K;
    const double d = p->pulsation ? df * 2.0 * M_PI : df;
-   const bool psd = !(flags & BSAHIP_NO_PSD), bisp = !(flags & BSAHIP_NO_BISP);
-   int br, bc;
-   f64_shape(nh, nm, F64_LEAST_DIAG, br, bc);
-   const long items = f64_tiles(nh, br, bc) * nm;
-   if (bisp && items > 0xffffffL)
-      return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: use a coarser grid or fewer modes");
    DiagTab T;
    double *mom;
    CHK(diag_tables(B, D, dfl, nh, df, T));

@@ -965,7 +965,7 @@ __host__ __device__ inline void f64_tile(long t, int rho, int &Q2, int &R)
    R = (int)(t - rho * q * (q + 1) / 2);
 }
 
-__host__ __device__ inline long f64_tiles(int rows, int BR, int BC)
+__host__ __device__ inline long f64_tiles(long rows, int BR, int BC)
 {
    const long n = (rows + 64 * BC - 1) / (64 * BC);
    return 4 * BC / BR * n * (n + 1) / 2;

@@ -3,6 +3,7 @@ sizes through different entry points, in any order, from several threads and aft
 refused call, give what each gives by itself; results above the staged size and inputs
 above the staged part size too.  Ordered sums make equal calls equal bit for bit."""
 import ctypes as C
+import resource
 import threading
 
 import numpy as np
@@ -122,3 +123,22 @@ def test_pinned_coherence_table(gpu_lib, tmp_path):
             assert np.abs(r[k] - want[k]).max() <= 1e-12 * np.abs(want[k]).max()
     del b, p
     assert gpu_lib.lib().hipHostFree(at) == 0
+
+
+def test_refused_grids_make_no_tables(gpu_lib):
+    """A grid that no launch can hold is refused before a list of its frequencies (2 GB
+    and more here) is made or sent: the process does not grow, and an allocation that
+    fails cannot leave the C entry by an exception."""
+    p = _tower(3, 1, 9, (1,))
+    p.nfreqs = 1 << 28
+    before = resource.getrusage(resource.RUSAGE_SELF).ru_maxrss
+    for make in (lambda: abi.classic_run(p), lambda: abi.classic_run(p, exact=True, prec="bf16x3"),
+                 lambda: abi.classic_run(p, only_diag=True), lambda: abi.Plan(p, prec="fp32"),
+                 lambda: abi.Batch([p])):
+        with pytest.raises(abi.BsaHipError, match="too large"):
+            make()
+    p.nfreqs = 2 ** 31 - 1                               # the list would hold 2^32 - 3
+    for kw in ({"exact": True}, {}, {"only_diag": True}):
+        with pytest.raises(abi.BsaHipError, match="too large"):
+            abi.classic_run(p, **kw)
+    assert resource.getrusage(resource.RUSAGE_SELF).ru_maxrss - before < 256 << 10
