@@ -17,6 +17,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -803,8 +804,7 @@ struct bsahip_plan {
    // fixed-order summation (BSAHIP_DETERMINISTIC): per-flush slots of the G
    // epilogue, the slot list of every m3 entry, per-block m2 partials
    double *slots = nullptr, *m2part = nullptr;
-   long *det_off = nullptr, *det_idx = nullptr;
-   int mflush = 0;
+   long *det_off = nullptr, *det_idx = nullptr, *det_slot0 = nullptr;
 };
 
 namespace {
@@ -820,18 +820,23 @@ void host_pair(long t, int &R, int &Q)
    R = (int)(t - q * (q + 1) / 2);
 }
 
-// FP64 wave tile (blocks of 16 rows x columns) for `rows` table rows and nm modes x: the
-// larger tiles load and scale less per MFMA, the smaller ones give more waves.  Measured
-// in us at (rows, nm, K), tiles 1x1 / 2x2 / 4x2: full model (17, 1, 32) 9 / 11 / -,
-// (66, 2, 32) 14 / 20 / -, (195, 3, 32) 22 / 20 / 30, (606, 6, 128) 53 / 34 / 39,
-// (909, 9, 320) 173 / 110 / 116, (1300, 20, 96) 400 / 227 / 224, (2570, 10, 608)
-// 1911 / 987 / 890; diagonal model, no accumulators shared between modes,
-// (257, 4, 608) 33 / 39 / -, (65, 60, 128) 11 / 14 / -, (257, 20, 3008) 297 / 243 / -.
-// `least` is the count of waves from which 2x2 is the faster.
-void f64_shape(long rows, int nm, double least, int &br, int &bc)
+// FP64 wave tile (blocks of 16 rows x columns) for nm modes x and nm (diagonal model: one)
+// runs of `per` table rows: the larger tiles load and scale less per MFMA, the smaller ones
+// give more waves.  Measured in us at (rows, nm, K), tiles 1x1 / 2x2 / 4x2: full model
+// (193, 1, 608) 27 / 40 / 62, (195, 3, 32) 22 / 23 / 33, (771, 3, 608) 137 / 69 / 81,
+// (780, 12, 608) 260 / 144 / 170, (3084, 12, 608) 3195 / 1537 / 1432, (2910, 30, 608)
+// 7254 / 3418 / 3264; diagonal model, no accumulators shared between modes, (257, 4, 608)
+// 33 / 39 / -, (65, 60, 128) 11 / 14 / -, (257, 20, 3008) 297 / 243 / -.  `least` is the
+// count of waves from which 2x2 is the faster.  A wave sums for each pair of modes it
+// meets, one after the other: tiles that would meet more than some four keep to 2x2, (270,
+// 30, 608) 156 / 157 / 241, (990, 30, 608) 918 / 518 / 539, (900, 100, 32)
+// 2388 / 2068 / 2538.
+constexpr long F64_LARGE = 48;
+
+void f64_shape(long rows, long per, int nm, double least, int &br, int &bc)
 {
    const auto waves = [&](int r, int c) { return (double)rows * (double)rows / (512.0 * r * c) * nm; };
-   if (waves(4, 2) >= 4096.0) {
+   if (per >= F64_LARGE && waves(4, 2) >= 4096.0) {
       br = 4;
       bc = 2;
    } else if (waves(2, 2) >= least) {
@@ -843,17 +848,20 @@ void f64_shape(long rows, int nm, double least, int &br, int &bc)
 
 // Doubles of the moments (forces, then responses) whose additions keep their errors, or 0.
 // FP64 only (the other precisions' own error is 1e-7), and from 48 rows per mode on: below,
-// an entry gets a few additions, at most two waves' tiles across a mode pair, and with many
-// modes the atomics are what such a launch waits for.  REST_MAX bounds the memory; a fixed
-// arena keeps the scratch it always had.
-constexpr int REST_ROWS = 48;
+// an entry gets a few additions, at most two waves' tiles across a mode pair.  Not beyond
+// 16 modes unless the contraction is long: the rate of the atomics, some 2.3e9 a second,
+// bounds such a launch, and they double (2910 rows, 30 modes, K 32 905 -> 1024 us, K 608
+// 3264 as without).  REST_MAX bounds the memory; a fixed arena keeps the scratch it had.
+constexpr int REST_ROWS = 48, REST_MODES = 16, REST_K = 256;
 constexpr long REST_MAX = 1L << 21;
 
 long rest_sums(const bsahip_plan *P)
 {
    const long n = 2L * P->D.nm * P->D.nm * P->D.nm;
    const bool atomics = !(P->flags & (BSAHIP_NO_BISP | BSAHIP_DETERMINISTIC));
-   return P->prec == BSAHIP_PREC_FP64 && atomics && P->nhp >= REST_ROWS && n <= REST_MAX && !P->B.arena ? n : 0;
+   const bool few = P->D.nm <= REST_MODES || P->D.K >= REST_K;
+   return P->prec == BSAHIP_PREC_FP64 && atomics && few && P->nhp >= REST_ROWS && n <= REST_MAX && !P->B.arena
+             ? n : 0;
 }
 
 constexpr double F64_LEAST = 32.0, F64_LEAST_DIAG = 384.0;
@@ -867,74 +875,69 @@ long plan_items(const bsahip_plan *P)
 }
 
 // Slot lists of the fixed-order mode: the flushes of every wave of every G
-// item in the order epi_wave makes them (kernels.hip), each with the twelve m3
-// entries of epi_flush (m3f entries 0 .. NM^3-1, m3r entries NM^3 .. 2 NM^3-1).
-// off (2 NM^3 + 1) and idx list, per entry, its slots in ascending order;
-// mflush is the largest flush count of a wave.
+// item in the order epi_wave makes them (kernels.hip), each with its m3 entries
+// in the order of epi_flush (m3f entries 0 .. NM^3-1, m3r entries NM^3 ..
+// 2 NM^3-1).  off (2 NM^3 + 1) and idx list, per entry, its slots in ascending
+// order, slot0 the first slot of each wave.
 void det_slot_lists(const bsahip_plan *P, std::vector<long> &off, std::vector<long> &idx,
-                    int &mflush)
+                    std::vector<long> &slot0)
 {
    const int nm = P->D.nm, nhp = P->nhp;
    const bool f64 = (P->prec == BSAHIP_PREC_FP64);
    const int BR = f64 ? P->f64_br : 4, BC = f64 ? P->f64_bc : 4;
    const long nm3 = (long)nm * nm * nm, nent = 2 * nm3, nitems = plan_items(P);
-   auto walk = [&](auto emit) {
+   auto walk = [&](auto wave, auto flush) {
       for (long lid = 0; lid < nitems; ++lid) {
          const int x = (int)(lid % nm);
-         int R, Q;
-         if (f64) f64_tile(lid / nm, 4 * BC / BR, Q, R);
-         else host_pair(lid / nm, R, Q);
+         int R = 0, Q = 0;
+         if (!f64) host_pair(lid / nm, R, Q);
          for (int w = 0; w < 4; ++w) {
             int rw0 = R * T2 + (w >> 1) * 64, cw0 = Q * T2 + (w & 1) * 64;
             bool diag = (R == Q);
             if (f64) {                     // gsym_f64_wave
-               const int c = 4 * Q + w, q = c * BC / BR;
-               if (R > q || c * 16 * BC >= P->rows) continue;
+               const long i = 4 * (lid / nm) + w;
+               if (i >= f64_waves(P->rows, BR, BC)) continue;
+               int c;
+               f64_tile(i, (P->rows + 16 * BC - 1) / (16 * BC), BR / BC, R, c);
                rw0 = R * 16 * BR;
                cw0 = c * 16 * BC;
-               diag = (R == q);
+               diag = c < (R + 1) * (BR / BC);
             }
-            const int y0 = rw0 / nhp, y1 = (rw0 + 16 * BR - 1) / nhp;
-            const int z0 = cw0 / nhp, z1 = (cw0 + 16 * BC - 1) / nhp;
-            int f = 0;
-            if (y0 == y1 && z0 == z1) {
-               if (y0 < nm && z0 < nm) emit(lid, w, f++, x, y0, z0, diag);
-            } else {
-               for (int y = y0; y <= y1; ++y)
-                  for (int z = z0; z <= z1; ++z)
-                     if (y < nm && z < nm) emit(lid, w, f++, x, y, z, diag);
-            }
+            const int y0 = rw0 / nhp, y1 = std::min((rw0 + 16 * BR - 1) / nhp, nm - 1);
+            const int z0 = cw0 / nhp, z1 = std::min((cw0 + 16 * BC - 1) / nhp, nm - 1);
+            wave(lid * 4 + w);
+            for (int y = y0; y <= y1; ++y)
+               for (int z = z0; z <= z1; ++z) flush(x, y, z, diag);
          }
       }
    };
-   auto entries = [&](int x, int y, int z, bool diag, long (&e)[12]) {
+   auto entries = [&](int x, int y, int z, bool diag, auto entry) {
       const long xyz = x + (long)nm * y + (long)nm * nm * z, yxz = y + (long)nm * x + (long)nm * nm * z,
                  yzx = y + (long)nm * z + (long)nm * nm * x, xzy = x + (long)nm * z + (long)nm * nm * y,
                  zxy = z + (long)nm * x + (long)nm * nm * y, zyx = z + (long)nm * y + (long)nm * nm * x;
       const long v[12] = {xyz, nm3 + xyz, yxz, nm3 + yxz, yzx, nm3 + yzx,
                           xzy, nm3 + xzy, zxy, nm3 + zxy, zyx, nm3 + zyx};
-      for (int t = 0; t < 12; ++t) e[t] = (diag && t >= 6) ? -1 : v[t];
+      const int n = epi_count(f64, x, y, z, diag);
+      for (int t = 0; t < n; ++t) entry(v[t]);
    };
-   std::vector<long> cnt(nent + 1, 0);
-   mflush = 1;
-   walk([&](long, int, int f, int x, int y, int z, bool diag) {
-      mflush = std::max(mflush, f + 1);
-      long e[12];
-      entries(x, y, z, diag, e);
-      for (int t = 0; t < 12; ++t)
-         if (e[t] >= 0) ++cnt[e[t] + 1];
-   });
    off.assign(nent + 1, 0);
-   for (long e = 0; e < nent; ++e) off[e + 1] = off[e] + cnt[e + 1];
-   idx.assign(off[nent], 0);
+   slot0.assign(nitems * 4, 0);
+   long slot = 0;
+   walk([&](long w) { slot0[w] = slot; },
+        [&](int x, int y, int z, bool diag) {
+           entries(x, y, z, diag, [&](long e) {
+              ++off[e + 1];
+              ++slot;
+           });
+        });
+   for (long e = 0; e < nent; ++e) off[e + 1] += off[e];
+   idx.assign(slot, 0);
    std::vector<long> pos(off.begin(), off.end() - 1);
-   walk([&](long lid, int w, int f, int x, int y, int z, bool diag) {
-      long e[12];
-      entries(x, y, z, diag, e);
-      const long base = ((lid * 4 + w) * (long)mflush + f) * 12;
-      for (int t = 0; t < 12; ++t)
-         if (e[t] >= 0) idx[pos[e[t]]++] = base + t;
-   });
+   slot = 0;
+   walk([](long) {},
+        [&](int x, int y, int z, bool diag) {
+           entries(x, y, z, diag, [&](long e) { idx[pos[e]++] = slot++; });
+        });
 }
 
 int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
@@ -970,7 +973,7 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    P->nhp = P->nu;
    P->rows = P->D.nm * P->nhp;
    P->ntile = (int)nt;
-   if (P->f64_br == 0) f64_shape(P->rows, P->D.nm, F64_LEAST, P->f64_br, P->f64_bc);
+   if (P->f64_br == 0) f64_shape(P->rows, P->nhp, P->D.nm, F64_LEAST, P->f64_br, P->f64_bc);
    P->ldU = (long)round_up(P->rows, T2);
    P->nft = 2 * P->nu - 1;
    P->d = p->pulsation ? df * 2.0 * M_PI : df;
@@ -983,11 +986,12 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    CHK(P->B.get("moments", 3 * nm2 + 2 * nm3 + P->rest, &P->m2));
    P->m3 = P->m2 + 3 * nm2;
    if ((flags & BSAHIP_DETERMINISTIC) && !(flags & BSAHIP_NO_BISP)) {
-      std::vector<long> off, idx;
-      det_slot_lists(P, off, idx, P->mflush);
+      std::vector<long> off, idx, slot0;
+      det_slot_lists(P, off, idx, slot0);
       CHK(upload(P->B, "det_off", off, &P->det_off));
       CHK(upload(P->B, "det_idx", idx, &P->det_idx));
-      CHK(P->B.get("det_slots", (size_t)plan_items(P) * 4 * P->mflush * 12, &P->slots));
+      CHK(upload(P->B, "det_slot0", slot0, &P->det_slot0));
+      CHK(P->B.get("det_slots", idx.size(), &P->slots));
    }
    if ((flags & BSAHIP_DETERMINISTIC) && !(flags & BSAHIP_NO_PSD))
       CHK(P->B.get("m2part", (size_t)((P->nh + 63) / 64) * 3 * nm2, &P->m2part));
@@ -1042,7 +1046,7 @@ void plan_args(const bsahip_plan *P, GsymArgs &a, GsymArgs16 &b16)
    a.m3f = P->m3;
    a.m3r = P->m3 + nm3;
    a.slots = P->slots;
-   a.mflush = P->mflush;
+   a.slot0 = P->det_slot0;
    a.rest = P->rest;
    b16.UR = P->UR;
    b16.UCh = reinterpret_cast<const uint4 *>(P->Ch);
@@ -1397,8 +1401,9 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
    CHK(validate(p));
    const bool psd = !(flags & BSAHIP_NO_PSD), bisp = !(flags & BSAHIP_NO_BISP);
    int br, bc;
-   f64_shape(nfh, p->nm, F64_LEAST_DIAG, br, bc);
-   const long items = f64_tiles(nfh, br, bc) * p->nm;
+   f64_shape(nfh, nfh, p->nm, F64_LEAST_DIAG, br, bc);
+   // (2^20 frequencies: past any accepted plane, within the 32 bits of f64_waves)
+   const long items = nfh > 1 << 20 ? LONG_MAX : f64_tiles(nfh, br, bc) * p->nm;
    if (bisp && items > 0xffffffL)
       return fail(BSAHIP_EUNSUPPORTED, "grid too large for one launch: use a coarser grid or fewer modes");
    Bufs &B = oneshot_bufs();

@@ -437,10 +437,10 @@ struct GsymArgs {
    int rule;
    int epi_plain;         // 1: every 16x16 block through the generic epilogue
    double *m3f, *m3r;     // [nm^3] accumulated (atomic)
-   double *slots;         // NULL, or fixed-order mode: each flush of a wave writes
-                          // its 12 m3 contributions to slots + ((item*4 + wave)
-                          // * mflush + flush) * 12 instead of the atomics
-   int mflush;            // flushes per wave at most (fixed-order mode)
+   double *slots;         // NULL, or fixed-order mode: the flushes of a wave write
+                          // their m3 contributions one after the other to slots +
+                          // slot0[item*4 + wave] instead of the atomics
+   const long *slot0;
    long rest;             // not 0: the rounding errors of the additions to a moment are
                           // added up `rest` doubles behind it
 };
@@ -770,7 +770,7 @@ __device__ __forceinline__ void epi_halve(double (&v)[9], int lane)
 }
 
 // Reduce the nine sums over the wave and add them (times 4 d^2) to the m3 entries, or
-// in the fixed-order mode store them in the wave's slot `f` (det_slot_lists of
+// in the fixed-order mode store them from the wave's slot on (det_slot_lists of
 // bsahip_api.hip builds the matching lists).  The exchanges halve the values a lane
 // holds as they halve the lanes that share one, 13 instead of 54, and leave sum k on
 // the lanes of one 4-lane group, so that the contributions (slot t: permutation t / 2 of
@@ -781,21 +781,58 @@ __device__ __forceinline__ void epi_halve(double (&v)[9], int lane)
 // error over ten decks and towers of 1000 nodes and 30 modes 9.6e-15 -> 6e-16 of the
 // largest moment, 151 nodes and 9 modes 1.4e-15 -> 7e-16, 20 nodes and 3 modes
 // 6.5e-16 -> 3e-16.
-// ONE: a structure of one mode, whose twelve contributions meet in two entries.
-template <bool ONE>
+// F64 (the FP64 kernels; the others' tiles of 64 x 64 make a quarter of the flushes, and the
+// longer code costs them 0.8 %): contributions that meet in one entry leave as one.  With
+// y == z, off the tile diagonal, the second six are those of the first again, with x == y ==
+// z two of them are left.  An atomic to one address takes some 40 ns however many waves
+// wait, and the entries of one mode are the ones that most waves share: 300 nodes, 1 mode,
+// 193 frequencies 42 -> 27 us.
+// ONE: a structure of one mode.
+__host__ __device__ inline int epi_count(bool f64, int x, int y, int z, bool diag)
+{
+   if (f64 && y == z) return x == y ? 2 : 6;
+   return diag ? 6 : 12;
+}
+
+template <bool F64>
+__device__ __forceinline__ void epi_put(const GsymArgs &a, int t, size_t e, double q, unsigned wave, int f)
+{
+   if (a.slots) {
+      a.slots[a.slot0[wave] + f + t] = q;
+      return;
+   }
+   double *o = (t & 1 ? a.m3r : a.m3f) + e;
+   if (F64 && a.rest) {
+      // two-sum of the addition as it was made
+      const double old = atomicAdd(o, q), sum = old + q, part = sum - old;
+      const double err = (old - (sum - part)) + (q - part);
+      if (err != 0.0 && err == err) atomicAdd(o + a.rest, err);
+   } else {
+      atomicAdd(o, q);
+   }
+}
+
+template <bool ONE, bool F64>
 __device__ __forceinline__ void epi_flush(const GsymArgs &a, int x, int y, int z, bool diag,
-                                          int lane, double (&s)[9], long sbase, int f)
+                                          int lane, double (&s)[9], unsigned wave, int f)
 {
    const double d2 = 4.0 * a.d2;
-   if constexpr (ONE) {
-      s[0] = diag ? s[0] + 2.0 * s[2] : 2.0 * (s[0] + s[2] + s[6]);
-      s[1] = diag ? s[1] + s[3] + s[4] : (s[1] + s[3] + s[4]) + (s[5] + s[7] + s[8]);
+   if (F64 && y == z && !diag) {
+      s[0] *= 2.0;
+      s[1] += s[5];
+      s[2] += s[6];
+      s[3] += s[7];
+      s[4] += s[8];
+   }
+   const int n = ONE ? 2 : epi_count(F64, x, y, z, diag);
+   if (n == 2) {
+      s[0] += 2.0 * s[2];
+      s[1] = (s[1] + s[3]) + s[4];
       epi_halve<2, 32>(s, lane);
-      const double r = s[0];
-      double q = r;
+      double q = s[0];
 #pragma unroll
       for (int o = 16; o >= 1; o >>= 1) q += __shfl_xor(q, o, 64);
-      if ((lane & 31) == 0) atomicAdd(lane ? a.m3r : a.m3f, q * d2);
+      if ((lane & 31) == 0) epi_put<F64>(a, lane >> 5, (size_t)x * (1 + a.nm + (size_t)a.nm * a.nm), q * d2, wave, f);
    } else {
       epi_halve<9, 32>(s, lane);
       epi_halve<5, 16>(s, lane);
@@ -814,25 +851,12 @@ __device__ __forceinline__ void epi_flush(const GsymArgs &a, int x, int y, int z
       int t = -1;
       if (!pad && second == 0) t = k == 0 ? 0 : (k <= 3 ? k : (k == 4 ? 5 : (k == 5 ? 7 : (k == 6 ? 8 : (k == 7 ? 9 : 11)))));
       if (!pad && second == 1) t = k == 0 ? 6 : (k == 2 ? 4 : (k == 6 ? 10 : -1));
-      if (t >= 0 && !(diag && t >= 6)) {
-         if (a.slots) {
-            a.slots[sbase + (long)f * 12 + t] = q;
-         } else {
-            const int p = t >> 1;
-            const int i0 = p == 0 || p == 3 ? x : (p == 1 || p == 2 ? y : z);
-            const int i1 = p == 0 || p == 5 ? y : (p == 1 || p == 4 ? x : z);
-            const int i2 = p == 0 || p == 1 ? z : (p == 2 || p == 5 ? x : y);
-            const size_t e = i0 + (size_t)a.nm * (i1 + (size_t)a.nm * i2);
-            double *o = (t & 1 ? a.m3r : a.m3f) + e;
-            if (a.rest) {
-               // two-sum of the addition as it was made
-               const double old = atomicAdd(o, q), sum = old + q, part = sum - old;
-               const double err = (old - (sum - part)) + (q - part);
-               if (err != 0.0 && err == err) atomicAdd(o + a.rest, err);
-            } else {
-               atomicAdd(o, q);
-            }
-         }
+      if (t >= 0 && t < n) {
+         const int p = t >> 1;
+         const int i0 = p == 0 || p == 3 ? x : (p == 1 || p == 2 ? y : z);
+         const int i1 = p == 0 || p == 5 ? y : (p == 1 || p == 4 ? x : z);
+         const int i2 = p == 0 || p == 1 ? z : (p == 2 || p == 5 ? x : y);
+         epi_put<F64>(a, t, i0 + (size_t)a.nm * (i1 + (size_t)a.nm * i2), q, wave, f);
       }
    }
 #pragma unroll
@@ -846,11 +870,11 @@ __device__ __forceinline__ void epi_flush(const GsymArgs &a, int x, int y, int z
 // wave.  getv<i>(j, g): values of block (i, j).
 template <int BR, int BC, bool IL, bool ONE, class GetVal>
 __device__ __forceinline__ void epi_wave(const GsymArgs &a, int x, bool diag, int rw0, int cw0,
-                                         int lane, long sbase, GetVal getv, double2 *win)
+                                         int lane, unsigned wave, GetVal getv, double2 *win)
 {
    constexpr int ST = IL ? 4 : 1;
    const int nm = a.nm;
-   int f = 0;                                         // flushes of this wave so far
+   int f = 0;                                         // slots of this wave so far
    const int y0 = rw0 / a.nhp, y1 = min((rw0 + 16 * BR - 1) / a.nhp, nm - 1);
    const int z0 = cw0 / a.nhp, z1 = min((cw0 + 16 * BC - 1) / a.nhp, nm - 1);
    const int lr = lane & 15, lk = lane >> 4;
@@ -926,7 +950,8 @@ __device__ __forceinline__ void epi_wave(const GsymArgs &a, int x, bool diag, in
             const int u0 = ub + 16 * i, v0 = vb + 16 * j;
             epi_rule<ST>(a, u0, v0, lane, g, s, win, ub, vb, wdb);
          }
-         epi_flush<ONE>(a, x, y, z, diag, lane, s, sbase, f++);
+         epi_flush<ONE, IL>(a, x, y, z, diag, lane, s, wave, f);
+         f += epi_count(IL, x, y, z, diag);
       }
 }
 
@@ -951,24 +976,39 @@ __device__ __forceinline__ long xcd_lid()
    return lid;
 }
 
-// Tiles of the FP64 G kernel: waves of 16 BR table rows x 16 BC table columns (BC <= BR),
-// four waves of a workgroup on consecutive column tiles c = 4 Q2 + w and the same rows.
-// With column tiles grouped to the row tile's size, Q = c BC / BR, a wave works when
-// R <= Q (G is symmetric) and treats its block as a diagonal one when R == Q.
-// Item t of a mode: column group Q2, row tile R < rho (Q2 + 1), rho = 4 BC / BR.
-__host__ __device__ inline void f64_tile(long t, int rho, int &Q2, int &R)
+// Tiles of the FP64 G kernel: a wave takes 16 BR table rows x 16 BC table columns
+// (r = BR / BC, 1 or 2).  G is symmetric: row tile R goes with the column tiles c from r R
+// on, the first r of them diagonal.  The waves of a mode are numbered row by row; a
+// workgroup takes four that follow one another, as a rule neighbours of one row, and none
+// of them idles (with four column tiles and a row tile per workgroup, those below the
+// diagonal and beyond the last column did, on the same SIMDs throughout: 270 rows, 30
+// modes, 700 nodes 394 us where 64 x 64 tiles take 297).
+// Counts fit 32 bits: a plan's grid has at most 2^24 tile pairs of 64.
+__host__ __device__ inline unsigned f64_row(unsigned R, unsigned nc, unsigned r)
 {
-   long q = (long)((sqrt(8.0 * (double)(t / rho) + 1.0) - 1.0) * 0.5);
-   while (rho * (q + 1) * (q + 2) / 2 <= t) ++q;
-   while (rho * q * (q + 1) / 2 > t) --q;
-   Q2 = (int)q;
-   R = (int)(t - rho * q * (q + 1) / 2);
+   return R * nc - r * (R * (R - 1) / 2);
+}
+
+__host__ __device__ inline void f64_tile(unsigned i, unsigned nc, unsigned r, int &R, int &c)
+{
+   const float b = (float)nc + 0.5f * r, d = b * b - 2.0f * r * (float)i;
+   unsigned q = (unsigned)((b - sqrtf(d > 0.0f ? d : 0.0f)) / r);      // the loops make it exact
+   while (q > 0 && f64_row(q, nc, r) > i) --q;
+   while (i - f64_row(q, nc, r) >= nc - r * q) ++q;
+   R = (int)q;
+   c = (int)(r * q + i - f64_row(q, nc, r));
+}
+
+// waves of a mode, workgroups of a mode
+__host__ __device__ inline unsigned f64_waves(long rows, int BR, int BC)
+{
+   const unsigned nc = (unsigned)((rows + 16 * BC - 1) / (16 * BC)), r = BR / BC;
+   return f64_row((nc + r - 1) / r, nc, r);
 }
 
 __host__ __device__ inline long f64_tiles(long rows, int BR, int BC)
 {
-   const long n = (rows + 64 * BC - 1) / (64 * BC);
-   return 4 * BC / BR * n * (n + 1) / 2;
+   return (f64_waves(rows, BR, BC) + 3L) / 4;
 }
 
 // One wave item of the FP64 G contraction: mode x, tile t.  The operands go from L1 / L2
@@ -986,12 +1026,15 @@ __device__ __forceinline__ void gsym_f64_wave(const GsymArgs &a, int x, long t)
 {
    constexpr int D = 4;                                      // K is a multiple of 32 = 8 D
    __shared__ double2 wins[4 * 768];
-   int Q2, R;
-   f64_tile(t, 4 * BC / BR, Q2, R);
    const int lane = threadIdx.x & 63;
    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-   const int c = 4 * Q2 + w, Q = c * BC / BR;
-   if (R > Q || c * 16 * BC >= a.nm * a.nhp) return;         // uniform per wave
+   const int rows = a.nm * a.nhp, nc = (rows + 16 * BC - 1) / (16 * BC);
+   const unsigned i = 4 * (unsigned)t + w;
+   if (i >= f64_waves(rows, BR, BC)) return;                 // uniform per wave
+   int R, c;
+   f64_tile(i, nc, BR / BC, R, c);
+   R = __builtin_amdgcn_readfirstlane(R);
+   c = __builtin_amdgcn_readfirstlane(c);
    const int lr = lane & 15, lk = lane >> 4;
    const double *pA = a.U + (size_t)lk * a.ldU + R * 16 * BR + lr;
    const double *pB = a.U + (size_t)lk * a.ldU + c * 16 * BC + lr;
@@ -1032,8 +1075,8 @@ __device__ __forceinline__ void gsym_f64_wave(const GsymArgs &a, int x, long t)
 
    // ---- epilogue: for v_mfma_f64_16x16x4f64, register t of lane l holds
    // D[(l/16) + 4t][l%16] of its 16x16 block (rows interleaved by 4).
-   const long sbase = ((t * a.nm + x) * 4 + w) * (long)a.mflush * 12;
-   epi_wave<BR, BC, true, ONE>(a, x, R == Q, R * 16 * BR, c * 16 * BC, lane, sbase,
+   const unsigned wave = (unsigned)((t * a.nm + x) * 4 + w);
+   epi_wave<BR, BC, true, ONE>(a, x, c < (R + 1) * (BR / BC), R * 16 * BR, c * 16 * BC, lane, wave,
                   [&](auto ic, int j, double (&g)[4]) {
                      constexpr int I = decltype(ic)::value;
 #pragma unroll
@@ -1051,10 +1094,10 @@ __device__ __forceinline__ void gsym_f64_wave(const GsymArgs &a, int x, long t)
 // 2x2 makes the compiler keep the accumulators in AGPRs, without copies: 121.9 -> 116.5 us
 // at 151 nodes, 9 modes, 101 frequencies, 59.0 -> 57.7 at 60, 8, 129, diagonal model 88 -> 80
 // at 500 nodes, 20 modes, 257 frequencies; three waves per SIMD spill, 140.7, 78.5 and 89.
-constexpr int f64_waves(int blocks) { return blocks > 4 ? 2 : 4; }
+constexpr int f64_bound(int blocks) { return blocks > 4 ? 2 : 4; }
 
 template <int BR, int BC>
-__global__ __launch_bounds__(256, f64_waves(BR * BC)) void k_gsym_f64(GsymArgs a)
+__global__ __launch_bounds__(256, f64_bound(BR * BC)) void k_gsym_f64(GsymArgs a)
 {
    const long lid = xcd_lid();
    gsym_f64_wave<BR, BC, false>(a, (int)(lid % a.nm), lid / a.nm);
@@ -1066,7 +1109,7 @@ __global__ __launch_bounds__(256, f64_waves(BR * BC)) void k_gsym_f64(GsymArgs a
 // run side by side (the plane sums are linear in G) would fill the chip better at a few
 // hundred nodes, but the slices' sums cancel: 5e-15 of the moments against 1e-15.
 template <int BR, int BC>
-__global__ __launch_bounds__(256, f64_waves(BR * BC)) void k_gsym_diag(GsymArgs a, int nmodes)
+__global__ __launch_bounds__(256, f64_bound(BR * BC)) void k_gsym_diag(GsymArgs a, int nmodes)
 {
    const long lid = blockIdx.x;
    const int x = (int)(lid % nmodes);
@@ -1239,12 +1282,12 @@ __device__ __forceinline__ void gsym_bf16x3_item(const GsymArgs &a, const GsymAr
 
    __builtin_amdgcn_s_setprio(0);
    // epilogue: f32-output 16x16 MFMAs hold D[4(l/16)+t][l%16]
-   const long sbase = ((tp * a.nm + x) * 4 + w) * (long)a.mflush * 12;
+   const unsigned wave = (unsigned)((tp * a.nm + x) * 4 + w);
    // each wave's FRF window: 12 KB of one operand plane (16 KB), free after the
    // last chunk's barrier
    uint4 *plane = w == 0 ? &Ah[0][0] : (w == 1 ? &Al[0][0] : (w == 2 ? &Bh[0][0] : &Bl[0][0]));
    double2 *win = reinterpret_cast<double2 *>(plane);
-   epi_wave<4, 4, false, false>(a, x, diag, R * T2 + wr * 64, Q * T2 + wc * 64, lane, sbase,
+   epi_wave<4, 4, false, false>(a, x, diag, R * T2 + wr * 64, Q * T2 + wc * 64, lane, wave,
                   [&](auto ic, int j, double (&g)[4]) {
                      constexpr int I = decltype(ic)::value;
                      f4v v = acc[I][3];
@@ -1359,12 +1402,12 @@ __device__ __forceinline__ void gsym_f32_item(const GsymArgs &a, const GsymArgs1
    }
 
    // epilogue: f32-output 16x16 MFMAs hold D[4(l/16)+t][l%16]
-   const long sbase = ((tp * a.nm + x) * 4 + w) * (long)a.mflush * 12;
+   const unsigned wave = (unsigned)((tp * a.nm + x) * 4 + w);
    __builtin_amdgcn_s_setprio(0);
    // each wave's FRF window: 12 KB of the operand planes (2 x 32 KB), free after
    // the last chunk's barrier
    double2 *win = reinterpret_cast<double2 *>(w < 2 ? &As[0][0] : &Bs[0][0]) + (w & 1) * 768;
-   epi_wave<4, 4, false, false>(a, x, diag, R * T2 + wr * 64, Q * T2 + wc * 64, lane, sbase,
+   epi_wave<4, 4, false, false>(a, x, diag, R * T2 + wr * 64, Q * T2 + wc * 64, lane, wave,
                   [&](auto ic, int j, double (&gv)[4]) {
                      constexpr int I = decltype(ic)::value;
                      f4v v = acc[I][3];

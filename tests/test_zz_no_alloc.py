@@ -50,3 +50,23 @@ def test_noalloc_refuses_a_problem_beyond_the_scratch(gpu_lib):
     assert rc == 0
     ref = gpu_lib.classic_run(synth.config1())
     assert rel_err(r["m3mr"], ref["m3mr"]) < 1e-12
+
+
+@pytest.mark.parametrize("nn,nm,nfh", [(600, 64, 3), (1000, 64, 3), (600, 64, 5), (600, 64, 7),
+                                       (10, 70, 9), (20, 30, 40), (40, 12, 129)])
+def test_noalloc_fixed_order(gpu_lib, nn, nm, nfh):
+    """Fixed-order runs with many modes and few frequencies fit the static array: a wave's
+    slots hold its contributions and no more (48 to 64 MB were needed by slots sized for
+    the largest wave), and the sums are those of the allocating run, bit for bit."""
+    p = synth.tower(nn=nn, nm=nm, comps=(1,), natf=np.linspace(0.2, 3.0, nm), nfreqs=nfh,
+                    df=4.0 / nfh, seed=nn)
+    b = abi.Bound(p)
+    out = {k: np.zeros(nm ** 2 if k[1] == "2" else nm ** 3)
+           for k in ("m2mf", "m2mr", "m2o2mr", "m3mf", "m3mr")}
+    rc = abi.lib().bsahip_classic_run_noalloc(
+        C.byref(b.struct), C.c_int32(nfh), C.c_double(p.df), C.c_int32(abi.DETERMINISTIC),
+        *[abi._ptr(out[k], C.c_double) for k in out])
+    assert rc == 0, abi.lib().bsahip_last_error().decode()
+    ref = gpu_lib.classic_run(p, deterministic=True, bound=b)
+    for k in out:
+        assert np.array_equal(out[k], ref[k]), k
