@@ -150,6 +150,7 @@ struct Ctx {
    hipStream_t s2 = nullptr;             // side stream: modal PSD moments beside the G kernel
    hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, e3 = nullptr;
    Bufs *bufs = nullptr;                 // scratch of the one-shot entry points
+   Bufs *plan_bufs = nullptr;            // buffers kept for the plans of one call (PlanLoan)
    char *stage = nullptr;                // pinned host memory of Pack, then of Pull
    hipEvent_t es = nullptr;              // Pack's last copy out of it
    // load_problem's host tables, kept up to HOST_KEPT values each: fresh ones cost a page
@@ -164,13 +165,18 @@ struct Ctx {
 
 Ctx g;
 
-// The one-shot scratch freed for another owner of buffers that found no memory.
+// Kept scratch freed for an owner of buffers that found no memory.  No call uses the
+// one-shot scratch beside other buffers, and a plan on loan has taken its own out.
 bool give_back(const Bufs *asking)
 {
-   if (!g.bufs || asking == g.bufs || g.bufs->m.empty()) return false;
-   (void)hipDeviceSynchronize();
-   g.bufs->release();
-   return true;
+   bool any = false;
+   for (Bufs *b : {g.bufs, g.plan_bufs}) {
+      if (!b || b == asking || b->m.empty()) continue;
+      if (!any) (void)hipDeviceSynchronize();
+      b->release();
+      any = true;
+   }
+   return any;
 }
 
 // Host arrays and device results of one call travel in few copies: a copy from or to
@@ -1206,17 +1212,21 @@ Bufs &oneshot_bufs()
    return *g.bufs;
 }
 
-// A plan of one call works in the one-shot scratch: with buffers of its own, allocated and
-// freed by each call, 151 nodes, 9 modes, 101 frequencies took 296 us, so 248.  Scratch
-// beyond KEPT bytes is freed with the plan.
-struct PoolLoan {
+// A plan of one call works in buffers kept for the next one: allocated and freed by each
+// call, 151 nodes, 9 modes, 101 frequencies took 296 us, so 248.  Beyond KEPT bytes they are
+// freed with the plan; the other entry points' scratch is not touched.
+struct PlanLoan {
    static constexpr size_t KEPT = (size_t)256 << 20;
    Bufs &B;
-   explicit PoolLoan(Bufs &b) : B(b) { B.m.swap(oneshot_bufs().m); }
-   ~PoolLoan()
+   explicit PlanLoan(Bufs &b) : B(b)
+   {
+      if (!g.plan_bufs) g.plan_bufs = new Bufs();
+      B.m.swap(g.plan_bufs->m);
+   }
+   ~PlanLoan()
    {
       if (B.total() > KEPT) B.release();
-      B.m.swap(oneshot_bufs().m);
+      B.m.swap(g.plan_bufs->m);
    }
 };
 
@@ -1268,7 +1278,8 @@ int bsahip_finalise(void)
    if (!g.ready) return 0;
    (void)hipStreamSynchronize(g.s);
    delete g.bufs;
-   g.bufs = nullptr;
+   delete g.plan_bufs;
+   g.bufs = g.plan_bufs = nullptr;
    if (g.blas) (void)rocblas_destroy_handle(g.blas);
    g.blas = nullptr;
    (void)hipStreamSynchronize(g.s2);
@@ -1489,7 +1500,7 @@ int bsahip__classic_moments(const bsahip_problem *p, int32_t nfh, double df, int
       return rc;
    }
    bsahip_plan P;
-   PoolLoan loan(P.B);
+   PlanLoan loan(P.B);
    int rc = plan_setup(&P, p, nfh, df, flags, psd_mode);
    if (rc == 0) rc = plan_exec(&P, m2mf, m2mr, m2o2mr, m3mf, m3mr);
    if (rc != 0) (void)hipDeviceSynchronize();                // nothing in flight on kept buffers
