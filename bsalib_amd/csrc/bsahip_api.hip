@@ -22,6 +22,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -82,6 +83,18 @@ struct Bufs {
       arena = static_cast<char *>(base);
       arena_cap = cap;
    }
+   // gives single buffers back; nothing may be using them
+   void drop(std::initializer_list<const char *> names)
+   {
+      if (arena) return;
+      (void)hipDeviceSynchronize();
+      for (const char *name : names) {
+         const auto it = m.find(name);
+         if (it == m.end()) continue;
+         if (it->second.p) (void)hipFree(it->second.p);
+         m.erase(it);
+      }
+   }
    size_t total() const
    {
       size_t n = 0;
@@ -122,9 +135,12 @@ struct Bufs {
             (void)hipGetLastError();
             e = hipMalloc(&b.p, bytes);
          }
-         if (e != hipSuccess)
+         if (e != hipSuccess) {
+            (void)hipGetLastError();             // or the next launch's check reports it
+            b.p = nullptr;
             return fail(BSAHIP_ENOMEM, std::string("hipMalloc(") + name + ", " +
                                            std::to_string(bytes) + " B): " + hipGetErrorString(e));
+         }
          b.n = bytes;
       }
       *out = static_cast<T *>(b.p);
@@ -1829,20 +1845,23 @@ int bfm_points_impl(const bsahip_problem *p, int32_t npts, const double *fi, con
    CHK(B.get("bfm_out", nm3 * npts, &ob));
    if (brm) CHK(B.get("brm_out", nm3 * npts, &orr));
    const unsigned nblk = (unsigned)((tot + 255) / 256);
-   if (D.nm <= 32) {
-      // the Mesher's point kernel
-      const int nmp = (D.nm + 15) / 16 * 16;
+   // the Mesher's point kernel up to 32 modes; where its table, 16 or 32 columns for any
+   // count of modes, finds no memory, the general one with its own of nm columns
+   const int nmp = (D.nm + 15) / 16 * 16;
+   double *V = nullptr, *PB = nullptr;
+   int rc = D.nm <= 32 ? point_table(B, D, dfl, nu, nmp, &V) : BSAHIP_ENOMEM;
+   if (rc == 0) rc = point_psib(B, D, nmp, &PB);
+   if (rc != 0 && rc != BSAHIP_ENOMEM) return rc;
+   if (rc == 0) {
       const size_t slab = (size_t)D.K * nmp;
-      double *V, *PB;
-      CHK(point_table(B, D, dfl, nu, nmp, &V));
       if (u0 < nu) CHK(fill(V + u0 * slab, (size_t)(nu - u0) * slab, 0.0));
-      CHK(point_psib(B, D, nmp, &PB));
       CHK(bfm_batch(D, V, PB, nmp, npts, di1, di2, di3, nullptr, ob));
       if (brm) {
          k_brm_points<<<nblk, 256, 0, g.s>>>(ob, D.nm, tot, df1, df2, D.Mm, D.Km, D.Cm, orr);
          HIPC(hipGetLastError());
       }
    } else {
+      if (D.nm <= 32) B.drop({"m_V", "m_PB", "m_U"});
       const long ldU = (long)D.nm * nu;
       double *U;
       CHK(B.get("U", (size_t)D.K * ldU, &U));
