@@ -1872,7 +1872,7 @@ int bfm_points_impl(const bsahip_problem *p, int32_t npts, const double *fi, con
          HIPC(hipGetLastError());
       }
       k_bfm_points<<<nblk, 256, 0, g.s>>>(U, ldU, nu, D.pb_k, D.K, D.nm, npts, di1, di2, di3, df1, df2,
-                                          D.Mm, D.Km, D.Cm, ob, orr, (long)nm3, 1);
+                                          D.Mm, D.Km, D.Cm, ob, orr);
       HIPC(hipGetLastError());
    }
    HIPC(hipMemcpyAsync(bfm, ob, nm3 * npts * sizeof(double), hipMemcpyDeviceToHost, g.s));

@@ -383,20 +383,8 @@ __global__ __launch_bounds__(256, 2) void k_project(ProjArgs P)
 }
 
 // ---------------------------------------------------------------------------
-// quadrature weight and FRF helpers (FP64)
+// FRF helpers and quadrature weights (FP64)
 // ---------------------------------------------------------------------------
-// rule 0: intgSpectraVect_ (BsaClassicImpl.F90:604-631): interior 1, edge 1/2,
-// corner 1 - 3/2;  rule 1: plain Riemann (:331,341);  rule 2: tensor trapezoid.
-__device__ __forceinline__ double qweight(int F1, int F2, int nh1, int rule, double d2)
-{
-   const int a1 = abs(F1), a2 = abs(F2);
-   if (a1 > nh1 || a2 > nh1) return 0.0;
-   const bool e1 = (a1 == nh1), e2 = (a2 == nh1);
-   if (rule == 1) return d2;
-   if (rule == 0) return (e1 && e2) ? (1.0 - 1.5) * d2 : ((e1 || e2) ? 0.5 * d2 : d2);
-   return d2 * (e1 ? 0.5 : 1.0) * (e2 ? 0.5 : 1.0);
-}
-
 __device__ __forceinline__ double2 hget(const double2 *__restrict__ H, int nft, int m, int F)
 {
    double2 h = H[(size_t)m * nft + abs(F)];
@@ -683,23 +671,6 @@ __device__ __forceinline__ void epi_rows(const GsymArgs &a, int cls, int ur0, in
       epi_value<3, I, 2, ST>(ps, pd, h[2], w[2], rx, rz, Z);
       epi_value<3, I, 3, ST>(ps, pd, h[3], w[3], rx, rz, Z);
    }
-}
-
-// Adds the nine contributions of one value: gas, gao weigh the (u, +-v) places, gbs, gdo
-// those at |u-v|, u+v with v, ges, gfo with u (units of 4 g).
-__device__ __forceinline__ void epi_nine(double (&s)[9], double gas, double gao, double gbs, double gdo,
-                                         double ges, double gfo, double F1s, double F1o, double F2s,
-                                         double F2o)
-{
-   s[0] += gas + gao;
-   s[1] += gas * F1s + gao * F1o;
-   s[2] += gbs + gdo;
-   s[3] += gbs * F2s + gdo * F2o;
-   s[4] += gbs * F1o + gdo * F1s;
-   s[5] += gas * F2o + gao * F2s;
-   s[6] += ges + gfo;
-   s[7] += ges * F1o + gfo * F1s;
-   s[8] += ges * F2s + gfo * F2o;
 }
 
 // Block of class 4: every weight of every point by the rule, FRF values from the window.
@@ -1146,13 +1117,6 @@ __device__ __forceinline__ uint32_t bf16_rne_bits(float f)
    return (b + 0x7FFFu + ((b >> 16) & 1u)) >> 16;
 }
 
-__device__ __forceinline__ void split_bf16(float v, uint32_t &hi, uint32_t &lo)
-{
-   hi = bf16_rne_bits(v);
-   const float r = v - __uint_as_float(hi << 16);     // exact in FP32
-   lo = bf16_rne_bits(r);
-}
-
 __device__ __forceinline__ int swz(int row, int g) { return row * 4 + (g ^ ((row >> 1) & 3)); }
 
 struct GsymArgs16 {
@@ -1485,14 +1449,6 @@ __global__ void k_split_table(const double *__restrict__ U, long ldU, int K, int
    split_tile(blockIdx.x * 32, blockIdx.y * 32, U, ldU, K, rows, ldk, UR, Ch, Cl);
 }
 
-// FP64 -> FP32 copy of the A table
-__global__ void k_to_f32(const double *__restrict__ src, float *__restrict__ dst, size_t n)
-{
-   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-   const size_t st = (size_t)gridDim.x * blockDim.x;
-   for (; i < n; i += st) dst[i] = (float)src[i];
-}
-
 // Lane-layout self test of v_mfma_f32_16x16x32_bf16 (one wave, 768 floats):
 // three products with known answers, see bsahip_selftest_mfma_layout.
 __global__ void k_mfma_bf16_layout(float *__restrict__ out)
@@ -1798,14 +1754,14 @@ __device__ __forceinline__ double brm_factor(double f1, double f2, int m, int n,
 // ---------------------------------------------------------------------------
 // Per-point bispectrum: B(m,n,p) at points given by row indices into U
 // (i1 -> f1, i2 -> f2, i3 -> f1+f2, i3 < 0 means S(f1+f2) = 0) and the
-// signed frequencies for the FRF.  out index = pt*spt + mnp*smn.
+// signed frequencies for the FRF.  out index = pt*nm^3 + mnp.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_bfm_points(
    const double *__restrict__ U, long ldU, int rows, const double *__restrict__ pb, int K,
    int nm, int npts, const int *__restrict__ i1, const int *__restrict__ i2,
    const int *__restrict__ i3, const double *__restrict__ f1s, const double *__restrict__ f2s,
    const double *__restrict__ Mm, const double *__restrict__ Km, const double *__restrict__ Cm,
-   double *__restrict__ bfm, double *__restrict__ brm, long spt, long smn)
+   double *__restrict__ bfm, double *__restrict__ brm)
 {
    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
    const long nm3 = (long)nm * nm * nm;
@@ -1814,8 +1770,8 @@ __global__ __launch_bounds__(256) void k_bfm_points(
    const int mnp = (int)(gid % nm3);
    const int m = mnp % nm, n = (mnp / nm) % nm, p = mnp / (nm * nm);
    const double s = bfm_point(U, ldU, rows, pb, K, m, n, p, i1[pt], i2[pt], i3[pt]);
-   if (bfm) bfm[pt * spt + mnp * smn] = s;
-   if (brm) brm[pt * spt + mnp * smn] = s * brm_factor(f1s[pt], f2s[pt], m, n, p, Mm, Km, Cm);
+   bfm[gid] = s;
+   if (brm) brm[gid] = s * brm_factor(f1s[pt], f2s[pt], m, n, p, Mm, Km, Cm);
 }
 
 // brm[e] = bfm[e] Re[H_m(f1) H_n(f2) conj H_p(f1+f2)] at points, e = pt nm^3 + mnp

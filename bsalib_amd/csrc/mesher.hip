@@ -267,44 +267,41 @@ struct MshTileRun {
    double wf;                  // weight of the force sums
 };
 
-// Tile quadrature: bilinear BFM on the BRM grid, exact FRF, trapezoid
-// weights.  A tile's BFM grid is nb1 x nb2 (point q = i + j*ldq, values
-// bf[q*nm3 + mnp]); each BFM cell holds s1 x s2 BRM cells.  BRM point (a, b):
+// Tile quadrature of the ONLY_DIAG model (nm entries): bilinear BFM on the BRM grid,
+// exact FRF, trapezoid weights.  A tile's BFM grid is nb1 x nb2 (point q = i + j*ldq,
+// values bf[q*nm + m]); each BFM cell holds s1 x s2 BRM cells.  BRM point (a, b):
 // f1 = f1a + a*dh1, f2 = f2a + b*dh2.  Adds sum w*B into m3f and
-// sum w*B*Re[H_m(f1)H_n(f2)H_p*(f1+f2)] into the tile's m3r.
-// grid (nitems * bx), block 256: block -> (item blockIdx.x / bx, entries
+// sum w*B*Re[H_m(f1)H_m(f2)H_m*(f1+f2)] into the tile's m3r.
+// grid (nitems * bx), block 256: block -> (item blockIdx.x / bx, modes
 // (blockIdx.x % bx) * 256 ..); item q covers cells [c0, c1) of tile it[q]
 __global__ __launch_bounds__(256) void k_msh_integrate(
    const MshTileRun *__restrict__ tr, const int *__restrict__ it, const int2 *__restrict__ cr,
-   int bx, int diag, const double2 *__restrict__ H)
+   int bx, const double2 *__restrict__ H)
 {
    const long q = blockIdx.x / bx;
    const MshTileRun T = tr[it[q]];
    const int nm = T.nm;
-   const int nm3 = diag ? nm : nm * nm * nm;
-   const int mnp = (int)(blockIdx.x % bx) * blockDim.x + threadIdx.x;
-   if (mnp >= nm3) return;
+   const int m = (int)(blockIdx.x % bx) * blockDim.x + threadIdx.x;
+   if (m >= nm) return;
    const int c0 = cr[q].x, c1 = cr[q].y;
-   int m, n, p;
-   msh_entry(mnp, nm, diag, m, n, p);
    const int nc1 = T.nb1 - 1, nc2 = T.nb2 - 1;
    const int NA = nc1 * T.s1, NB = nc2 * T.s2;
-   const double Mp = T.Mm[p], Kp = T.Km[p], Cp = T.Cm[p];
+   const double Mm = T.Mm[m], Km = T.Km[m], Cm = T.Cm[m];
    const double inv1 = 1.0 / T.s1, inv2 = 1.0 / T.s2;
    const double2 *H1 = H + T.h1, *H2 = H + T.h2, *H3 = T.h3 >= 0 ? H + T.h3 : nullptr;
    double sf = 0.0, sr = 0.0;
    for (int c = c0; c < c1; ++c) {
       const int ci = c % nc1, cj = c / nc1;
       const size_t q00 = (size_t)ci + (size_t)cj * T.ldq;
-      const double b00 = T.bf[q00 * nm3 + mnp], b10 = T.bf[(q00 + 1) * nm3 + mnp];
-      const double b01 = T.bf[(q00 + T.ldq) * nm3 + mnp], b11 = T.bf[(q00 + T.ldq + 1) * nm3 + mnp];
+      const double b00 = T.bf[q00 * nm + m], b10 = T.bf[(q00 + 1) * nm + m];
+      const double b01 = T.bf[(q00 + T.ldq) * nm + m], b11 = T.bf[(q00 + T.ldq + 1) * nm + m];
       const int ea = (ci == nc1 - 1) ? T.s1 : T.s1 - 1;   // owned BRM points per axis
       const int eb = (cj == nc2 - 1) ? T.s2 : T.s2 - 1;
       for (int bb = 0; bb <= eb; ++bb) {
          const int b = cj * T.s2 + bb;
          const double wb = (b == 0 || b == NB) ? 0.5 : 1.0;
          const double sv = bb * inv2;
-         const double2 h2v = H2[(size_t)b * nm + n];
+         const double2 h2v = H2[(size_t)b * nm + m];
          const double e0 = (1.0 - sv) * b00 + sv * b01, e1 = (1.0 - sv) * b10 + sv * b11;
          for (int aa = 0; aa <= ea; ++aa) {
             const int a = ci * T.s1 + aa;
@@ -314,10 +311,10 @@ __global__ __launch_bounds__(256) void k_msh_integrate(
             const double2 h1v = H1[(size_t)a * nm + m];
             double2 h3v;
             if (H3) {
-               h3v = H3[(size_t)(a + b) * nm + p];
+               h3v = H3[(size_t)(a + b) * nm + m];
             } else {
                const double w3 = 2.0 * M_PI * (T.f3a + a * T.dh1 + b * T.dh2);
-               const double r = Kp - w3 * w3 * Mp, im = w3 * Cp, d = r * r + im * im;
+               const double r = Km - w3 * w3 * Mm, im = w3 * Cm, d = r * r + im * im;
                h3v = make_double2(r / d, -im / d);
             }
             const double w = wa * wb;
@@ -326,8 +323,8 @@ __global__ __launch_bounds__(256) void k_msh_integrate(
          }
       }
    }
-   atomicAdd(T.m3f + mnp, sf * T.wf);
-   atomicAdd(T.m3r + mnp, sr * T.ws);
+   atomicAdd(T.m3f + m, sf * T.wf);
+   atomicAdd(T.m3r + m, sr * T.ws);
 }
 
 // The same quadrature for the full model (nm^3 entries) as two chained products
@@ -1305,7 +1302,7 @@ int msh_integrate_jobs(const std::vector<MshJob *> &jobs)
       CHK(upload(B, "m_ranges", cr, &dcr));
       k_frf_segs<<<(unsigned)((eoff.back() + 255) / 256), 256, 0, g.s>>>(dseg, doff, (int)seg.size(), H);
       HIPC(hipGetLastError());
-      k_msh_integrate<<<(unsigned)(it.size() * bx), 256, 0, g.s>>>(dtr, dit, dcr, bx, 1, H);
+      k_msh_integrate<<<(unsigned)(it.size() * bx), 256, 0, g.s>>>(dtr, dit, dcr, bx, H);
       HIPC(hipGetLastError());
    } else {
       // items of about equal cost, some 4096 of them: runs of cells of one tile, or,
