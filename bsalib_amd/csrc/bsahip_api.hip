@@ -1387,10 +1387,10 @@ struct DiagTab {
    long ldX;
 };
 
-int diag_tables(Bufs &B, const Prob &D, const double *dfl, int nh, double df, DiagTab &T)
+int diag_tables(Bufs &B, const Prob &D, const double *dfl, int nh, double df, long ldX, DiagTab &T)
 {
    const int nft = 2 * nh - 1, nm = D.nm, K = D.K;
-   T.ldX = round_up(nh, 128);
+   T.ldX = ldX;
    CHK(B.get("dg_X", (size_t)K * T.ldX, &T.X));
    CHK(B.get("dg_W", (size_t)nm * K, &T.W));
    CHK(B.get("dg_A2", (size_t)nm * K, &T.A2));
@@ -1445,7 +1445,7 @@ int classic_diag(const bsahip_problem *p, int32_t nfh, double df, int32_t flags,
    const double d = p->pulsation ? df * 2.0 * M_PI : df;
    DiagTab T;
    double *mom;
-   CHK(diag_tables(B, D, dfl, nh, df, T));
+   CHK(diag_tables(B, D, dfl, nh, df, (nh + 127L) / 128 * 128, T));      // whole tiles
    CHK(B.get("dg_mom", 5 * (size_t)nm, &mom));
    CHK(fill(mom, 5 * (size_t)nm, 0.0));
    double *m2f = mom, *m2r = mom + nm, *m2o = mom + 2 * nm, *m3f = mom + 3 * nm, *m3r = mom + 4 * nm;
@@ -1664,7 +1664,7 @@ int bsahip_classic_bispectra_sel(const bsahip_problem *p, int32_t nfh, double df
    if (diag) {
       DiagTab X;
       double *T;
-      CHK(diag_tables(B, D, dfl, nh, df, X));
+      CHK(diag_tables(B, D, dfl, nh, df, nh, X));
       CHK(diag_products(B, D, nh, X, &T));
       k_diag_bisp_sel<<<gs, 256, 0, g.s>>>(T, nh, X.H, 2 * nh - 1, dsel, ob, orr);
    } else {
