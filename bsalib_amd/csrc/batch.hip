@@ -64,6 +64,9 @@ __device__ __forceinline__ void batch_drain(const long *__restrict__ offs, int n
    }
 }
 
+// 2x2 blocks for every structure: the launch has one tile shape, and small structures, which
+// batches are for, need the smaller one.  The launch bound of the single form's 2x2 (4)
+// changes nothing here (-1 to +2 % over batches of 4 to 64 structures).
 __global__ __launch_bounds__(256, 2) void k_gsym_f64_batch(const GsymArgs *__restrict__ args,
                                                         const long *__restrict__ offs, int ns,
                                                         const long *__restrict__ qbeg,

@@ -15,7 +15,7 @@
 // moments its modal PSD kernel (k_m2 with diag).  Bound by launches and latency at
 // these sizes: T stored by a GEMM per mode, read back over the whole plane and a
 // serial loop over k per PSD value took 530 us for 500 nodes with 2 components, 20
-// modes, 257 frequencies; now 80 us, with the 15 us of k_m2 beside.  Selected bispectra
+// modes, 257 frequencies; now 64 us, with the 15 us of k_m2 beside.  Selected bispectra
 // still store their T_m (one GEMM per mode).
 
 // X[k*ldX + u] = S_k(u df), zero for u >= nh and in the padding rows k >= kv; from the

@@ -990,8 +990,9 @@ __host__ __device__ inline long f64_tiles(long rows, int BR, int BC)
 // top of its 64), so what is left to win is the vector work: the scaling by Psi_b
 // (BR multiplies per 4 BR BC MFMAs) and the epilogue.  Staged through LDS with two
 // barriers per chunk of 32 K rows it took 254 ms at 1000 nodes, 30 modes, 513
-// frequencies (61 TFLOP/s where bare MFMA reaches 76.9) and 2686 / 259 us at 333, 17,
-// 193 / 40, 20, 65; now 236 ms, of which the epilogue 15, and 2466 / 222 us.
+// frequencies (61 TFLOP/s where bare MFMA reaches 76.9) and 2690 / 262 us at 333, 17,
+// 193 / 40, 20, 65; now 232.7 ms, of which the epilogue 24, and 2415 / 200 us, of which
+// 520 / 139.
 template <int BR, int BC, bool ONE>
 __device__ __forceinline__ void gsym_f64_wave(const GsymArgs &a, int x, long t)
 {
@@ -1062,9 +1063,10 @@ __device__ __forceinline__ void gsym_f64_wave(const GsymArgs &a, int x, long t)
 }
 
 // Two waves per SIMD (registers; LDS allows three).  The bound of 4 for the tiles up to
-// 2x2 makes the compiler keep the accumulators in AGPRs, without copies: 121.9 -> 116.5 us
-// at 151 nodes, 9 modes, 101 frequencies, 59.0 -> 57.7 at 60, 8, 129, diagonal model 88 -> 80
-// at 500 nodes, 20 modes, 257 frequencies; three waves per SIMD spill, 140.7, 78.5 and 89.
+// 2x2 makes the compiler keep the accumulators in AGPRs, without copies: with 2 it takes
+// 100 us where 4 takes 95 at 151 nodes, 9 modes, 101 frequencies, 68 / 66 at 60, 8, 129,
+// 33 / 28 at 300, 1, 193, and a call of the diagonal model 248 / 244 at 500, 20, 257.
+// A bound of 3 spills: 20 to 35 % slower.
 constexpr int f64_bound(int blocks) { return blocks > 4 ? 2 : 4; }
 
 template <int BR, int BC>

@@ -81,7 +81,7 @@ __global__ void k_pbt(const double *__restrict__ pb, int nm, int K, int nmp, dou
 // is formed on the fly.  Rows m are padded to MT*16, columns (n,p) (col =
 // n + p*nm) tiled by 16 and dealt to the 8 waves (TPW tiles each).
 // One workgroup per point (point lists of the API too: 120 nodes, 2 components, 8 modes,
-// 301 points take 18 us where one value per lane took 209);
+// 301 points take 15 us where one value per lane took 209);
 // out[slot[pt]*nm3 + m + col*nm] = B (slot null: q0 + pt).
 // ---------------------------------------------------------------------------
 // K chunk staged in LDS: K is a multiple of 32; 16 took 17.5 us where 32 takes 15.2 at 301

@@ -74,8 +74,8 @@ extern "C" {
  * atomically, then each entry sums its partials in one fixed order with
  * Kahan compensation (the wave reductions already run in a fixed tree), so
  * repeated runs give bitwise-equal moments.  Costs an extra buffer of
- * 12 doubles per wave flush of the G epilogue (0.36 GB at NN=1000, NM=30,
- * 1025^2 in split-bf16x3) and a reduction pass.  Without it the moments are
+ * up to 12 doubles per wave flush of the G epilogue (0.10 GB at NN=1000,
+ * NM=30, 1025^2 in split-bf16x3) and a reduction pass.  Without it the moments are
  * FP64 atomic sums whose order, and last bits, vary between runs.  No
  * reference counterpart (the reference's sums are sequential). */
 #define BSAHIP_DETERMINISTIC (1 << 13)
