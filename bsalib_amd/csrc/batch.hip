@@ -181,17 +181,16 @@ __global__ __launch_bounds__(256, 2) void k_m2_batch(const M2Args *__restrict__ 
 }
 
 // results of every structure into one contiguous buffer: array j = srcs[j]
-// (lens[j] doubles) to dst + offs[j], the errors of its additions rest[j] doubles behind
-// (0: none) added; one block per array
+// (lens[j] doubles) to dst + offs[j], its copies[j] copies summed; grid (arrays, any)
 __global__ void k_pack(const double *const *__restrict__ srcs, const long *__restrict__ lens,
-                       const long *__restrict__ rest, const long *__restrict__ offs,
+                       const int *__restrict__ copies, const long *__restrict__ offs,
                        double *__restrict__ dst)
 {
    const int j = blockIdx.x;
    const double *src = srcs[j];
    double *d = dst + offs[j];
-   const long r = rest[j];
-   for (long t = threadIdx.x; t < lens[j]; t += blockDim.x) d[t] = r ? src[t] + src[t + r] : src[t];
+   for (long t = blockIdx.y * blockDim.x + threadIdx.x; t < lens[j]; t += gridDim.y * blockDim.x)
+      d[t] = sum_all(copies[j], [&](int c) { return src[c * lens[j] + t]; });
 }
 
 struct bsahip_batch {
@@ -233,7 +232,9 @@ struct bsahip_batch {
    bool joint = true;            // one table launch per kind (batch_descriptors)
    // packed results: per structure m3 (m3f, m3r) then m2 (f, r, o)
    const double **psrc = nullptr;
-   long *plen = nullptr, *poff = nullptr, *prest = nullptr;
+   long *plen = nullptr, *poff = nullptr;
+   int *pcopies = nullptr;
+   long longest = 0;                        // doubles of the longest result
    double *pack = nullptr, *hpack = nullptr;   // device buffer, pinned host copy
    std::vector<long> m3off, m2off;
    long npack = 0;
@@ -278,6 +279,15 @@ int batch_launch(bsahip_batch *b)
    return 0;
 }
 
+// results of every structure into `pack`
+int batch_pack(bsahip_batch *b)
+{
+   const dim3 grid((unsigned)(2 * b->plans.size()), (unsigned)std::min<long>((b->longest + 255) / 256, 64));
+   k_pack<<<grid, 256, 0, g.s>>>(b->psrc, b->plen, b->pcopies, b->poff, b->pack);
+   HIPC(hipGetLastError());
+   return 0;
+}
+
 // descriptors of the launches over every structure, on the device
 int batch_descriptors(bsahip_batch *b)
 {
@@ -308,7 +318,7 @@ int batch_descriptors(bsahip_batch *b)
       T.pulsation = D.pulsation;
       T.npsd = (long)D.ntc * P->nu * D.nnl;
       T.nfrf = (long)D.nm * P->nft;
-      T.nm3 = bisp ? 2L * D.nm * D.nm * D.nm + P->rest : 0;
+      T.nm3 = bisp ? 2L * D.nm * D.nm * D.nm * P->copies : 0;
       T.nm2 = psd ? 3L * D.nm * D.nm : 0;
       tab.push_back(T);
       toff.push_back(toff.back() + (T.npsd + T.nfrf + T.nm3 + T.nm2 + 255) / 256);
@@ -423,9 +433,7 @@ int batch_step(bsahip_batch *b, int mode)
          for (int s : b->order) CHK(plan_gsym(b->plans[s].get()));
       if (psd)
          for (auto &P : b->plans) CHK(plan_m2(P.get()));
-      k_pack<<<(unsigned)(2 * b->plans.size()), 256, 0, g.s>>>(b->psrc, b->plen, b->prest, b->poff, b->pack);
-      HIPC(hipGetLastError());
-      return 0;
+      return batch_pack(b);
    }
    CHK(batch_tables(b));
    if (psd) {
@@ -449,9 +457,7 @@ int batch_step(bsahip_batch *b, int mode)
    }
    if (bisp) CHK(batch_launch(b));
    if (psd) HIPC(hipStreamWaitEvent(g.s, b->ev_m2, 0));
-   k_pack<<<(unsigned)(2 * b->plans.size()), 256, 0, g.s>>>(b->psrc, b->plen, b->prest, b->poff, b->pack);
-   HIPC(hipGetLastError());
-   return 0;
+   return batch_pack(b);
 }
 
 void batch_drop_graph(bsahip_batch *b)
@@ -548,20 +554,22 @@ int bsahip_batch_create(const bsahip_problem *const *probs, const int32_t *nfh, 
    HIPC(hipEventCreateWithFlags(&B->ev_fork, hipEventDisableTiming));
    {
       std::vector<const double *> src;
-      std::vector<long> len, off, rest;
+      std::vector<long> len, off;
+      std::vector<int> copies;
       long o = 0;
       for (auto &P : B->plans) {
          const long nm = P->D.nm;
          B->m3off.push_back(o);
          src.push_back(P->m3);
          len.push_back(2 * nm * nm * nm);
-         rest.push_back(P->rest);
+         copies.push_back(P->copies);
          off.push_back(o);
          o += 2 * nm * nm * nm;
+         B->longest = std::max({B->longest, len.back(), 3 * nm * nm});
          B->m2off.push_back(o);
          src.push_back(P->m2);
          len.push_back(3 * nm * nm);
-         rest.push_back(0);
+         copies.push_back(1);
          off.push_back(o);
          o += 3 * nm * nm;
       }
@@ -570,7 +578,7 @@ int bsahip_batch_create(const bsahip_problem *const *probs, const int32_t *nfh, 
       CHK(B->B.get("plen", len.size(), &B->plen));
       CHK(B->B.get("poff", off.size(), &B->poff));
       CHK(B->B.get("pack", (size_t)o, &B->pack));
-      CHK(upload(B->B, "prest", rest, &B->prest));
+      CHK(upload(B->B, "pcopies", copies, &B->pcopies));
       HIPC(hipMemcpyAsync(B->psrc, src.data(), src.size() * sizeof(double *), hipMemcpyHostToDevice, g.s));
       HIPC(hipMemcpyAsync(B->plen, len.data(), len.size() * sizeof(long), hipMemcpyHostToDevice, g.s));
       HIPC(hipMemcpyAsync(B->poff, off.data(), off.size() * sizeof(long), hipMemcpyHostToDevice, g.s));

@@ -199,11 +199,8 @@ bool give_back(const Bufs *asking)
 // pageable memory costs about 5 us up and 20 us down however small it is (13 uploads of a
 // small problem 62 us, one of the same bytes out of pinned memory 12 us; 4 KB down 23 us,
 // by pinned memory 12 us).  From about a megabyte on there is nothing to win (1.6 MB down
-// 317 us either way: the page faults of the caller's array).  Moments with their errors
-// behind them come whole up to SUMS_DOWN (32 KB: 1.021 ms a run, 1.027 with the sums formed
-// by a launch before the copy).
-constexpr size_t STAGE_UP = (size_t)4 << 20, STAGE_DOWN = (size_t)512 << 10, PART_UP = STAGE_UP / 4,
-                 SUMS_DOWN = (size_t)64 << 10;
+// 317 us either way: the page faults of the caller's array).
+constexpr size_t STAGE_UP = (size_t)4 << 20, STAGE_DOWN = (size_t)512 << 10, PART_UP = STAGE_UP / 4;
 
 // Uploads gathered into one device buffer (src null: room only).  The host arrays have to
 // live until send(), which has read them when it returns.
@@ -274,20 +271,9 @@ struct Pull {
       void *dst;
       const char *src;
       size_t bytes;
-      double *next;            // add_sums: dst and next receive sums
    };
    std::vector<Seg> segs;
    size_t n = 0;
-   // a and b (either null) = the first and the second m of 4 m doubles src, each with the
-   // value 2 m behind it added; false: not staged, for the device to add
-   bool add_sums(double *a, double *b, const double *src, size_t m)
-   {
-      const size_t bytes = 4 * m * sizeof(double);
-      if (!g.stage || bytes > SUMS_DOWN || n + bytes > STAGE_DOWN) return false;
-      segs.push_back({a, reinterpret_cast<const char *>(src), bytes, b});
-      n += bytes;
-      return true;
-   }
    int add(void *dst, const void *src, size_t bytes)
    {
       if (!dst || !bytes) return 0;
@@ -295,7 +281,7 @@ struct Pull {
          HIPC(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g.s));
          return 0;
       }
-      segs.push_back({dst, static_cast<const char *>(src), bytes, static_cast<double *>(dst)});
+      segs.push_back({dst, static_cast<const char *>(src), bytes});
       n += bytes;
       return 0;
    }
@@ -312,15 +298,7 @@ struct Pull {
       HIPC(hipStreamSynchronize(g.s));
       at = 0;
       for (const Seg &q : segs) {
-         if (q.next == q.dst) {
-            std::memcpy(q.dst, stage + at, q.bytes);
-         } else {
-            const double *v = reinterpret_cast<const double *>(stage + at);
-            const size_t m = q.bytes / (4 * sizeof(double));
-            double *a = static_cast<double *>(q.dst), *b = q.next;
-            for (size_t k = 0; a && k < m; ++k) a[k] = v[k] + v[2 * m + k];
-            for (size_t k = 0; b && k < m; ++k) b[k] = v[m + k] + v[3 * m + k];
-         }
+         std::memcpy(q.dst, stage + at, q.bytes);
          at += q.bytes;
       }
       segs.clear();
@@ -818,7 +796,7 @@ struct bsahip_plan {
    long ldU = 0;
    double df = 0.0, d = 0.0;
    double *fl = nullptr, *U = nullptr, *m3 = nullptr, *m2 = nullptr;
-   long rest = 0;                        // doubles of m3 with errors behind them (rest_sums)
+   int copies = 1;                       // of m3 (gsym_copies)
    double2 *H = nullptr;
    float *UR = nullptr;
    uint16_t *Ch = nullptr, *Cl = nullptr;
@@ -868,22 +846,19 @@ void f64_shape(long rows, long per, int nm, double least, int &br, int &bc)
    }
 }
 
-// Doubles of the moments (forces, then responses) whose additions keep their errors, or 0.
-// FP64 only (the other precisions' own error is 1e-7), and from 48 rows per mode on: below,
-// an entry gets a few additions, at most two waves' tiles across a mode pair.  Not beyond
-// 16 modes unless the contraction is long: the rate of the atomics, some 2.3e9 a second,
-// bounds such a launch, and they double (2910 rows, 30 modes, K 32 905 -> 1024 us, K 608
-// 3264 as without).  REST_MAX bounds the memory; a fixed arena keeps the scratch it had.
-constexpr int REST_ROWS = 48, REST_MODES = 16, REST_K = 256;
-constexpr long REST_MAX = 1L << 21;
+// Copies of the third moments that the FP64 contraction adds into (gsym_f64_wave): about one
+// for every COPY_ADDS additions to an entry, three for each tile of a mode pair, while all of
+// them stay within COPY_MAX doubles and the last sum, serial per entry, within COPY_MOST.
+// One where a fixed arena keeps the scratch it had or the sums have an order of their own,
+// and for the other precisions, whose own error is 1e-7.
+constexpr long COPY_ADDS = 4, COPY_MAX = 1L << 20, COPY_MOST = 256;
 
-long rest_sums(const bsahip_plan *P)
+int gsym_copies(const bsahip_plan *P)
 {
+   if (P->prec != BSAHIP_PREC_FP64 || (P->flags & (BSAHIP_NO_BISP | BSAHIP_DETERMINISTIC)) || P->B.arena) return 1;
    const long n = 2L * P->D.nm * P->D.nm * P->D.nm;
-   const bool atomics = !(P->flags & (BSAHIP_NO_BISP | BSAHIP_DETERMINISTIC));
-   const bool few = P->D.nm <= REST_MODES || P->D.K >= REST_K;
-   return P->prec == BSAHIP_PREC_FP64 && atomics && few && P->nhp >= REST_ROWS && n <= REST_MAX && !P->B.arena
-             ? n : 0;
+   const long adds = 3L * (P->nhp / (16 * P->f64_br) + 1) * (P->nhp / (16 * P->f64_bc) + 1);
+   return (int)std::max(1L, std::min({adds / COPY_ADDS, COPY_MAX / n, COPY_MOST}));
 }
 
 constexpr double F64_LEAST = 32.0, F64_LEAST_DIAG = 384.0;
@@ -1003,9 +978,9 @@ int plan_setup(bsahip_plan *P, const bsahip_problem *p, int32_t nfh, double df, 
    CHK(zero_padding(P->D, P->nhp, P->U, P->ldU));      // the runs write the valid entries only
    CHK(P->B.get("H", (size_t)P->D.nm * P->nft, &P->H));
    const size_t nm3 = (size_t)P->D.nm * P->D.nm * P->D.nm, nm2 = (size_t)P->D.nm * P->D.nm;
-   P->rest = rest_sums(P);
+   P->copies = gsym_copies(P);
    // one buffer: the results come back in one copy
-   CHK(P->B.get("moments", 3 * nm2 + 2 * nm3 + P->rest, &P->m2));
+   CHK(P->B.get("moments", 3 * nm2 + 2 * nm3 * P->copies, &P->m2));
    P->m3 = P->m2 + 3 * nm2;
    if ((flags & BSAHIP_DETERMINISTIC) && !(flags & BSAHIP_NO_BISP)) {
       std::vector<long> off, idx, slot0;
@@ -1038,7 +1013,7 @@ int plan_prepare(bsahip_plan *P)
    CHK(build_table(P->B, D, P->fl, P->nu, P->nhp, P->U, P->ldU, true));
    CHK(launch_frf(D, P->nft, P->df, P->H));
    if (!(P->flags & BSAHIP_NO_BISP)) {
-      CHK(fill(P->m3, 2 * nm3 + P->rest, 0.0));
+      CHK(fill(P->m3, 2 * nm3 * P->copies, 0.0));
       if (P->prec != BSAHIP_PREC_FP64) {
          dim3 gs((unsigned)(P->ldU / 32), (unsigned)((D.K + 31) / 32));
          k_split_table<<<gs, 256, 0, g.s>>>(P->U, P->ldU, D.K, (int)P->ldU, D.K, P->UR, P->Ch, P->Cl);
@@ -1069,7 +1044,7 @@ void plan_args(const bsahip_plan *P, GsymArgs &a, GsymArgs16 &b16)
    a.m3r = P->m3 + nm3;
    a.slots = P->slots;
    a.slot0 = P->det_slot0;
-   a.rest = P->rest;
+   a.copies = P->copies;
    b16.UR = P->UR;
    b16.UCh = reinterpret_cast<const uint4 *>(P->Ch);
    b16.UCl = reinterpret_cast<const uint4 *>(P->Cl);
@@ -1168,12 +1143,8 @@ int plan_copyout(bsahip_plan *P, double *m2mf, double *m2mr, double *m2o2mr, dou
       CHK(pl.add(m2mr, P->m2 + nm2, nm2 * sizeof(double)));
       CHK(pl.add(m2o2mr, P->m2 + 2 * nm2, nm2 * sizeof(double)));
    }
-   // the errors of the additions join the moments on the way, or on the device where
-   // fetching them costs more than a launch
-   const bool sums = P->rest && (m3mf || m3mr);
-   if (sums && m3mf != m3mr && pl.add_sums(m3mf, m3mr, P->m3, nm3)) return pl.finish();
-   if (sums) {
-      k_add_rest<<<(unsigned)((P->rest + 255) / 256), 256, 0, g.s>>>(P->m3, P->rest);
+   if (P->copies > 1 && (m3mf || m3mr)) {
+      k_sum_copies<<<(unsigned)((2 * nm3 + 63) / 64), 64, 0, g.s>>>(P->m3, (long)(2 * nm3), P->copies);
       HIPC(hipGetLastError());
    }
    if (!(P->flags & BSAHIP_NO_BISP)) {

@@ -35,13 +35,6 @@ __global__ void k_fill(double *__restrict__ p, size_t n, double v)
    for (; i < n; i += st) p[i] = v;
 }
 
-// p[i] += p[n + i]
-__global__ void k_add_rest(double *__restrict__ p, long n)
-{
-   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-   if (i < n) p[i] += p[n + i];
-}
-
 // U[k*ld + c] = 0 for c >= c0, the first n / (ld - c0) rows
 __global__ void k_zero_tail(double *__restrict__ U, long ld, long c0, long n)
 {
@@ -429,8 +422,7 @@ struct GsymArgs {
                           // their m3 contributions one after the other to slots +
                           // slot0[item*4 + wave] instead of the atomics
    const long *slot0;
-   long rest;             // not 0: the rounding errors of the additions to a moment are
-                          // added up `rest` doubles behind it
+   int copies;            // of m3f and m3r, 2 nm^3 doubles apart (gsym_f64_wave)
 };
 
 // Quadrature weight / d^2 from edge flags of |F1| (p) and |F2| (q) on the
@@ -746,12 +738,6 @@ __device__ __forceinline__ void epi_halve(double (&v)[9], int lane)
 // holds as they halve the lanes that share one, 13 instead of 54, and leave sum k on
 // the lanes of one 4-lane group, so that the contributions (slot t: permutation t / 2 of
 // xyz, yxz, yzx, xzy, zxy, zyx; even force, odd response) leave as one atomic.
-// The blocks near the origin and the resonances hold most of a moment, and with hundreds
-// of small additions after them the order alone costs ten roundings and more: with `rest`
-// the errors are kept (Knuth's two-sum on the value that the atomic returns).  Largest
-// error over ten decks and towers of 1000 nodes and 30 modes 9.6e-15 -> 6e-16 of the
-// largest moment, 151 nodes and 9 modes 1.4e-15 -> 7e-16, 20 nodes and 3 modes
-// 6.5e-16 -> 3e-16.
 // F64 (the FP64 kernels; the others' tiles of 64 x 64 make a quarter of the flushes, and the
 // longer code costs them 0.8 %): contributions that meet in one entry leave as one.  With
 // y == z, off the tile diagonal, the second six are those of the first again, with x == y ==
@@ -765,22 +751,13 @@ __host__ __device__ inline int epi_count(bool f64, int x, int y, int z, bool dia
    return diag ? 6 : 12;
 }
 
-template <bool F64>
 __device__ __forceinline__ void epi_put(const GsymArgs &a, int t, size_t e, double q, unsigned wave, int f)
 {
    if (a.slots) {
       a.slots[a.slot0[wave] + f + t] = q;
       return;
    }
-   double *o = (t & 1 ? a.m3r : a.m3f) + e;
-   if (F64 && a.rest) {
-      // two-sum of the addition as it was made
-      const double old = atomicAdd(o, q), sum = old + q, part = sum - old;
-      const double err = (old - (sum - part)) + (q - part);
-      if (err != 0.0 && err == err) atomicAdd(o + a.rest, err);
-   } else {
-      atomicAdd(o, q);
-   }
+   atomicAdd((t & 1 ? a.m3r : a.m3f) + e, q);
 }
 
 template <bool ONE, bool F64>
@@ -803,7 +780,7 @@ __device__ __forceinline__ void epi_flush(const GsymArgs &a, int x, int y, int z
       double q = s[0];
 #pragma unroll
       for (int o = 16; o >= 1; o >>= 1) q += __shfl_xor(q, o, 64);
-      if ((lane & 31) == 0) epi_put<F64>(a, lane >> 5, (size_t)x * (1 + a.nm + (size_t)a.nm * a.nm), q * d2, wave, f);
+      if ((lane & 31) == 0) epi_put(a, lane >> 5, (size_t)x * (1 + a.nm + (size_t)a.nm * a.nm), q * d2, wave, f);
    } else {
       epi_halve<9, 32>(s, lane);
       epi_halve<5, 16>(s, lane);
@@ -827,7 +804,7 @@ __device__ __forceinline__ void epi_flush(const GsymArgs &a, int x, int y, int z
          const int i0 = p == 0 || p == 3 ? x : (p == 1 || p == 2 ? y : z);
          const int i1 = p == 0 || p == 5 ? y : (p == 1 || p == 4 ? x : z);
          const int i2 = p == 0 || p == 1 ? z : (p == 2 || p == 5 ? x : y);
-         epi_put<F64>(a, t, i0 + (size_t)a.nm * (i1 + (size_t)a.nm * i2), q, wave, f);
+         epi_put(a, t, i0 + (size_t)a.nm * (i1 + (size_t)a.nm * i2), q, wave, f);
       }
    }
 #pragma unroll
@@ -993,9 +970,24 @@ __host__ __device__ inline long f64_tiles(long rows, int BR, int BC)
 // frequencies (61 TFLOP/s where bare MFMA reaches 76.9) and 2690 / 262 us at 333, 17,
 // 193 / 40, 20, 65; now 232.7 ms, of which the epilogue 24, and 2415 / 200 us, of which
 // 520 / 139.
+// The blocks near the origin and the resonances hold most of a moment, and with hundreds
+// of small additions after them the order alone costs ten roundings and more; waves that
+// add to one address wait for each other, too (some 40 ns each).  The workgroups of a mode
+// therefore take the copies of the moments in turn, summed up at the end (k_sum_copies).
+// Largest difference from the compensated sums of the same contributions over the largest
+// moment, one copy -> gsym_copies of them: 30 nodes, 2 modes, 1025 frequencies 5.7e-15 ->
+// 2.1e-16, 60, 16, 257 1.3e-15 -> 2.0e-16, 200, 24, 513 3.0e-15 -> 1.6e-16, 40, 9, 101
+// 8.4e-16 -> 2.2e-16; times 18 nodes, 3 modes, 405 frequencies 92 -> 34 us, 132, 3, 504
+// 136 -> 69, 27, 2, 254 30 -> 22.
 template <int BR, int BC, bool ONE>
-__device__ __forceinline__ void gsym_f64_wave(const GsymArgs &a, int x, long t)
+__device__ __forceinline__ void gsym_f64_wave(const GsymArgs &args, int x, long t)
 {
+   GsymArgs a = args;
+   if (!ONE) {
+      const long own = t % a.copies * (2L * a.nm * a.nm * a.nm);
+      a.m3f += own;
+      a.m3r += own;
+   }
    constexpr int D = 4;                                      // K is a multiple of 32 = 8 D
    __shared__ double2 wins[4 * 768];
    const int lane = threadIdx.x & 63;
@@ -1623,6 +1615,33 @@ __device__ __forceinline__ void kahan_add(double &s, double &c, double v)
    const double t = s + y;
    c = (t - s) - y;
    s = t;
+}
+
+// Sum of nc doubles v(0 .. nc-1), compensated; the plain sum where it is no longer finite
+// (the correction of an infinity would be NaN).  W loads go out together: on the device
+// 192 of them one after the other took 35 us.
+template <class Get>
+__device__ __forceinline__ double sum_all(int nc, Get v)
+{
+   constexpr int W = 16;
+   double s = v(0), c = 0.0, plain = s, q[W];
+   for (int k = 1; k < nc; k += W) {
+#pragma unroll
+      for (int j = 0; j < W; ++j) q[j] = k + j < nc ? v(k + j) : 0.0;
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+         kahan_add(s, c, q[j]);
+         plain += q[j];
+      }
+   }
+   return plain - plain == 0.0 ? s : plain;
+}
+
+// p[i] = sum of the nc copies p[c * n + i], n doubles each
+__global__ void k_sum_copies(double *p, long n, int nc)
+{
+   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+   if (i < n) p[i] = sum_all(nc, [&](int c) { return p[c * n + i]; });
 }
 
 __global__ void k_sum_lists(const double *__restrict__ vals, const long *__restrict__ off,

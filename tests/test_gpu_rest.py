@@ -1,11 +1,10 @@
-"""The atomic sums of the FP64 third moments keep the errors of their additions: the
-moments equal the fixed-order compensated sums of the same contributions, whatever the
-order of the atomics, for all wave tiles, both ways the errors come back (with the
-results, or joined on the device) and in batches.
+"""The atomic sums of the FP64 third moments lose next to nothing to the order of their
+additions: the moments equal the fixed-order compensated sums of the same contributions,
+for all wave tiles, with few copies of the moments and many, and in batches.
 
-Tolerance 4 * 2^-53 of the largest entry: the compensated sum of n contributions is off
-by 2 * 2^-53 of the result plus n 2^-106 of their absolute sum, the two-sums by the same,
-with one rounding at the end."""
+Tolerance 4 * 2^-53 of the largest entry: a copy takes about four additions, so that its
+sum is off by at most four roundings of 2^-53 of its largest partial sum, and the copies'
+own sum and the fixed-order one are compensated."""
 import numpy as np
 import pytest
 
