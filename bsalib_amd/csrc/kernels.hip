@@ -926,32 +926,31 @@ __device__ __forceinline__ long xcd_lid()
 
 // Tiles of the FP64 G kernel: a wave takes 16 BR table rows x 16 BC table columns
 // (r = BR / BC, 1 or 2).  G is symmetric: row tile R goes with the column tiles c from r R
-// on, the first r of them diagonal.  The waves of a mode are numbered row by row; a
-// workgroup takes four that follow one another, as a rule neighbours of one row, and none
-// of them idles (with four column tiles and a row tile per workgroup, those below the
-// diagonal and beyond the last column did, on the same SIMDs throughout: 270 rows, 30
-// modes, 700 nodes 394 us where 64 x 64 tiles take 297).
+// on, the first r of them diagonal.  The waves of a mode are numbered by groups of r
+// columns, rows R <= g of group g one after the other; a workgroup takes four that follow
+// one another and none of them idles (with four column tiles and a row tile per workgroup,
+// those below the diagonal and beyond the last column did, on the same SIMDs throughout:
+// 270 rows, 30 modes, 700 nodes 394 us where 64 x 64 tiles take 297).  Numbered by rows
+// instead, 14 nodes, 28 modes, 81 frequencies take 589 us where this takes 561, and 166,
+// 13, 374 1514 / 1493, but 22, 13, 176 255 / 261.
 // Counts fit 32 bits: a plan's grid has at most 2^24 tile pairs of 64.
-__host__ __device__ inline unsigned f64_row(unsigned R, unsigned nc, unsigned r)
-{
-   return R * nc - r * (R * (R - 1) / 2);
-}
+__host__ __device__ inline unsigned f64_group(unsigned g, unsigned r) { return r * (g * (g + 1) / 2); }
 
 __host__ __device__ inline void f64_tile(unsigned i, unsigned nc, unsigned r, int &R, int &c)
 {
-   const float b = (float)nc + 0.5f * r, d = b * b - 2.0f * r * (float)i;
-   unsigned q = (unsigned)((b - sqrtf(d > 0.0f ? d : 0.0f)) / r);      // the loops make it exact
-   while (q > 0 && f64_row(q, nc, r) > i) --q;
-   while (i - f64_row(q, nc, r) >= nc - r * q) ++q;
-   R = (int)q;
-   c = (int)(r * q + i - f64_row(q, nc, r));
+   unsigned g = (unsigned)((sqrtf(8.0f * (float)i / r + 1.0f) - 1.0f) * 0.5f);   // the loops make it exact
+   while (g > 0 && f64_group(g, r) > i) --g;
+   while (f64_group(g + 1, r) <= i) ++g;
+   const unsigned o = i - f64_group(g, r), n = nc - r * g < r ? nc - r * g : r;
+   R = (int)(o / n);
+   c = (int)(r * g + o % n);
 }
 
 // waves of a mode, workgroups of a mode
 __host__ __device__ inline unsigned f64_waves(long rows, int BR, int BC)
 {
-   const unsigned nc = (unsigned)((rows + 16 * BC - 1) / (16 * BC)), r = BR / BC;
-   return f64_row((nc + r - 1) / r, nc, r);
+   const unsigned nc = (unsigned)((rows + 16 * BC - 1) / (16 * BC)), r = BR / BC, g = nc / r;
+   return f64_group(g, r) + nc % r * (g + 1);
 }
 
 __host__ __device__ inline long f64_tiles(long rows, int BR, int BC)
