@@ -1365,7 +1365,7 @@ int msh_integrate_jobs(const std::vector<MshJob *> &jobs)
 }
 
 // The accumulators of a run, zero: copies of m3f then m3r, and behind them `ntile` slots
-// of m3r.  msh_acc_sum replaces them by their sum.
+// of m3r.  msh_acc_sum leaves the sum of the copies in the first.
 int msh_acc(bsahip_mesher *m, size_t ntile, double **acc, double **slots)
 {
    const size_t n = 2 * (size_t)m->nc * MSH_COPIES, all = n + ntile * m->nc;
@@ -1374,14 +1374,11 @@ int msh_acc(bsahip_mesher *m, size_t ntile, double **acc, double **slots)
    return fill(*acc, all, 0.0);
 }
 
-int msh_acc_sum(bsahip_mesher *m, double **acc)
+int msh_acc_sum(bsahip_mesher *m, double *acc)
 {
    const long n = 2L * m->nc;
-   double *sum;
-   CHK(m->B.get("m_sum", (size_t)n, &sum));
-   k_sum_fixed<<<(unsigned)((n + 255) / 256), 256, 0, g.s>>>(*acc, MSH_COPIES, n, n, sum);
+   k_sum_copies<<<(unsigned)((n + 63) / 64), 64, 0, g.s>>>(acc, n, MSH_COPIES);
    HIPC(hipGetLastError());
-   *acc = sum;
    return 0;
 }
 
@@ -1699,7 +1696,7 @@ int bsahip_mesher_run_tiles(bsahip_mesher *m, const int32_t *levels, double *til
       },
       evals_post, [&](bool) { return msh_integrate_jobs({&job}); }));
    const long brm = job.brm;
-   CHK(msh_acc_sum(m, &acc));
+   CHK(msh_acc_sum(m, acc));
    if (tile_m3mr)
       HIPC(hipMemcpyAsync(tile_m3mr, slots, nt * nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
    if (m3mf) HIPC(hipMemcpyAsync(m3mf, acc, nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
@@ -1778,7 +1775,7 @@ int bsahip_mesher_run_batch(int32_t n, bsahip_mesher *const *ms, const int32_t *
    if (!diag.empty()) CHK(msh_integrate_jobs(diag));
    for (int i = 0; i < n; ++i) {
       const size_t nm3 = (size_t)ms[i]->nc;
-      CHK(msh_acc_sum(ms[i], &acc[i]));
+      CHK(msh_acc_sum(ms[i], acc[i]));
       if (m3mf && m3mf[i])
          HIPC(hipMemcpyAsync(m3mf[i], acc[i], nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
       if (m3mr && m3mr[i])

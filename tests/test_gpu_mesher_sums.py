@@ -91,3 +91,20 @@ def test_force_moments(gpu_lib, nn, seed):
         for r in runs:
             assert np.abs(r["m3mf"] - want).max() <= TOL * np.abs(want).max(), (level, points)
     M.close()
+
+
+def test_beyond_the_largest_number(gpu_lib):
+    """A moment that exceeds the largest double is infinite, not NaN, on the Mesher's copies
+    as on those of the FP64 contraction; the values it is made of are finite."""
+    p = synth.tower(nn=14, nm=1, comps=(1,), natf=np.array([0.2]), xi=np.array([0.01]),
+                    nfreqs=257, df=0.25, seed=0, u10=30.0)
+    p.turb_scales = 0.05 * p.turb_scales                   # a wide peak at the origin
+    cfg = dict(bkg_base_rfmnt=12, tile_cells=16)
+    run = {"plan": lambda: abi.classic_run(p), "mesher": lambda: abi.Mesher(p, **cfg).run(levels=1)}
+    base = {k: r()["m3mf"][0] for k, r in run.items()}
+    peak = abi.bfm_points(p, np.zeros(1), np.zeros(1), with_brm=False)[0][0, 0]
+    s = (1e308 / min(base.values())) ** (1 / 3)
+    assert 0 < peak * s ** 3 < 2e307
+    p.wfc = 4 ** (1 / 3) * s * p.wfc
+    for k, r in run.items():
+        assert np.isposinf(r()["m3mf"][0]), k
