@@ -1696,11 +1696,13 @@ int bsahip_mesher_run_tiles(bsahip_mesher *m, const int32_t *levels, double *til
       },
       evals_post, [&](bool) { return msh_integrate_jobs({&job}); }));
    const long brm = job.brm;
-   CHK(msh_acc_sum(m, acc));
+   if (m3mf || (m3mr && !tile_m3mr)) CHK(msh_acc_sum(m, acc));
+   Pull pl;
+   CHK(pl.add(m3mf, acc, nm3 * sizeof(double)));
+   if (!tile_m3mr) CHK(pl.add(m3mr, acc + nm3, nm3 * sizeof(double)));
    if (tile_m3mr)
       HIPC(hipMemcpyAsync(tile_m3mr, slots, nt * nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
-   if (m3mf) HIPC(hipMemcpyAsync(m3mf, acc, nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
-   HIPC(hipStreamSynchronize(g.s));
+   CHK(pl.finish());
    if (tile_m3mr)
       // a mirror image has the slot of its first tile, integrated for both
       for (size_t k = 0; k < nt; ++k) {
@@ -1708,16 +1710,12 @@ int bsahip_mesher_run_tiles(bsahip_mesher *m, const int32_t *levels, double *til
          if (j >= 0 && j < (long)k)
             std::copy(tile_m3mr + j * nm3, tile_m3mr + (j + 1) * nm3, tile_m3mr + k * nm3);
       }
-   if (m3mr) {
-      if (tile_m3mr) {
-         // tile by tile, so that each pass reads one contiguous slot
-         std::fill(m3mr, m3mr + nm3, 0.0);
-         for (size_t k = 0; k < nt; ++k) {
-            const double *c = tile_m3mr + k * nm3;
-            for (size_t q = 0; q < nm3; ++q) m3mr[q] += c[q];
-         }
-      } else {
-         HIPC(hipMemcpy(m3mr, acc + nm3, nm3 * sizeof(double), hipMemcpyDeviceToHost));
+   if (m3mr && tile_m3mr) {
+      // tile by tile, so that each pass reads one contiguous slot
+      std::fill(m3mr, m3mr + nm3, 0.0);
+      for (size_t k = 0; k < nt; ++k) {
+         const double *c = tile_m3mr + k * nm3;
+         for (size_t q = 0; q < nm3; ++q) m3mr[q] += c[q];
       }
    }
    if (counts) {
@@ -1773,15 +1771,14 @@ int bsahip_mesher_run_batch(int32_t n, bsahip_mesher *const *ms, const int32_t *
    for (MshJob &J : jobs) (J.M->diag ? diag : full).push_back(&J);
    if (!full.empty()) CHK(msh_integrate_jobs(full));
    if (!diag.empty()) CHK(msh_integrate_jobs(diag));
+   Pull pl;
    for (int i = 0; i < n; ++i) {
       const size_t nm3 = (size_t)ms[i]->nc;
       CHK(msh_acc_sum(ms[i], acc[i]));
-      if (m3mf && m3mf[i])
-         HIPC(hipMemcpyAsync(m3mf[i], acc[i], nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
-      if (m3mr && m3mr[i])
-         HIPC(hipMemcpyAsync(m3mr[i], acc[i] + nm3, nm3 * sizeof(double), hipMemcpyDeviceToHost, g.s));
+      if (m3mf) CHK(pl.add(m3mf[i], acc[i], nm3 * sizeof(double)));
+      if (m3mr) CHK(pl.add(m3mr[i], acc[i] + nm3, nm3 * sizeof(double)));
    }
-   HIPC(hipStreamSynchronize(g.s));
+   CHK(pl.finish());
    if (counts)
       for (int i = 0; i < n; ++i) {
          counts[3 * i] = ms[i]->evals_lv0;
@@ -1805,14 +1802,14 @@ int msh_adapt(bsahip_mesher *m, double tol, int32_t *levels, int64_t *evals, dou
    if (!m || !levels || !(tol > 0.0)) return fail(BSAHIP_EINVAL, "need a Mesher, levels and tol > 0");
    const bool want = m3mf_out || m3mr_out || counts_out;
    const size_t nt = m->tiles.size(), nm3 = (size_t)m->nc;
-   std::vector<double> prev(nt * nm3), cur(nt * nm3), m3f(nm3), m3r(nm3);
+   std::vector<double> prev(nt * nm3), cur(nt * nm3), m3r(nm3);
    std::vector<int32_t> lev(nt, 1), lr(nt);
    std::vector<char> up(nt);
    int64_t cnt[3] = {0, 0, 0};
    // level 1 (the resident level-0 samples), then level 2 on every tile
-   CHK(bsahip_mesher_run_tiles(m, lev.data(), prev.data(), m3f.data(), m3r.data(), nullptr));
+   CHK(bsahip_mesher_run_tiles(m, lev.data(), prev.data(), nullptr, m3r.data(), nullptr));
    std::fill(lev.begin(), lev.end(), 2);
-   CHK(bsahip_mesher_run_tiles(m, lev.data(), cur.data(), m3f.data(), m3r.data(), cnt));
+   CHK(bsahip_mesher_run_tiles(m, lev.data(), cur.data(), nullptr, m3r.data(), cnt));
    double M = 0.0;
    for (size_t q = 0; q < nm3; ++q) M = std::max(M, std::fabs(m3r[q]));
    const double budget = 0.5 * tol * M;
@@ -1865,7 +1862,7 @@ int msh_adapt(bsahip_mesher *m, double tol, int32_t *levels, int64_t *evals, dou
          for (size_t q = 0; q < nm3; ++q) E[q] -= 0.75 * delta[t * nm3 + q];
       }
       if (!any) break;
-      CHK(bsahip_mesher_run_tiles(m, lr.data(), cur.data(), m3f.data(), m3r.data(), cnt));
+      CHK(bsahip_mesher_run_tiles(m, lr.data(), cur.data(), nullptr, m3r.data(), cnt));
       for (size_t t = 0; t < nt; ++t)
          if (up[t]) {
             set_delta(t);
@@ -1882,7 +1879,14 @@ int msh_adapt(bsahip_mesher *m, double tol, int32_t *levels, int64_t *evals, dou
    if (evals) *evals = n;
    // with outputs, the last run was at the final levels: level 2 everywhere,
    // or a refinement round whose kept tiles ran at their own levels
-   if (m3mf_out) std::copy(m3f.begin(), m3f.end(), m3mf_out);
+   if (m3mf_out) {
+      double *acc;
+      CHK(m->B.get("m_acc", 2 * nm3 * MSH_COPIES, &acc));     // as that run left it
+      CHK(msh_acc_sum(m, acc));
+      Pull pl;
+      CHK(pl.add(m3mf_out, acc, nm3 * sizeof(double)));
+      CHK(pl.finish());
+   }
    if (m3mr_out) std::copy(m3r.begin(), m3r.end(), m3mr_out);
    if (counts_out) std::copy(cnt, cnt + 3, counts_out);
    return 0;
