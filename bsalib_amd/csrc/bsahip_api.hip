@@ -823,14 +823,17 @@ void host_pair(long t, int &R, int &Q)
 // FP64 wave tile (blocks of 16 rows x columns) for nm modes x and nm (diagonal model: one)
 // runs of `per` table rows: the larger tiles load and scale less per MFMA, the smaller ones
 // give more waves.  Measured in us at (rows, nm, K), tiles 1x1 / 2x2 / 4x2: full model
-// (193, 1, 608) 27 / 40 / 62, (195, 3, 32) 22 / 23 / 33, (771, 3, 608) 137 / 69 / 81,
-// (780, 12, 608) 260 / 144 / 170, (3084, 12, 608) 3195 / 1537 / 1432, (2910, 30, 608)
-// 7254 / 3418 / 3264; diagonal model, no accumulators shared between modes, (257, 4, 608)
-// 33 / 39 / -, (65, 60, 128) 11 / 14 / -, (257, 20, 3008) 297 / 243 / -.  `least` is the
-// count of waves from which 2x2 is the faster.  A wave sums for each pair of modes it
-// meets, one after the other: tiles that would meet more than some four keep to 2x2, (270,
-// 30, 608) 156 / 157 / 241, (990, 30, 608) 918 / 518 / 539, (900, 100, 32)
-// 2388 / 2068 / 2538.
+// (193, 1, 608) 27 / 39 / 61, (195, 3, 32) 16 / 21 / 31, (390, 5, 608) 44 / 51 / -,
+// (516, 4, 2016) 165 / 115 / -, (771, 3, 608) 72 / 50 / 76, (780, 12, 608) 239 / 135 / 161,
+// (3084, 12, 608) 3146 / 1481 / 1391, (2910, 30, 608) 7131 / 3394 / 3189; diagonal model
+// (257, 4, 608) 33 / 39 / -, (65, 60, 128) 11 / 14 / -, (257, 20, 3008) 297 / 243 / -.
+// `least` is the count of waves from which 2x2 is taken.  In both models 1x1 is the faster
+// while all its waves run at once, up to some 400 to 512 of 2x2; the full model takes 2x2
+// from 32 on all the same, since it is the batches' tile: a structure's moments are then
+// sums of the same contributions in a batch as alone.  A wave sums for each pair of modes
+// it meets, one after the other: tiles that would meet more than some four keep to 2x2,
+// (270, 30, 608) 148 / 153 / 235, (990, 30, 608) 924 / 476 / 503, (900, 100, 32)
+// 2431 / 2090 / 2548.
 constexpr long F64_LARGE = 48;
 
 void f64_shape(long rows, long per, int nm, double least, int &br, int &bc)

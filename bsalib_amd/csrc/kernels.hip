@@ -743,7 +743,7 @@ __device__ __forceinline__ void epi_halve(double (&v)[9], int lane)
 // y == z, off the tile diagonal, the second six are those of the first again, with x == y ==
 // z two of them are left.  An atomic to one address takes some 40 ns however many waves
 // wait, and the entries of one mode are the ones that most waves share: 300 nodes, 1 mode,
-// 193 frequencies 42 -> 27 us.
+// 193 frequencies 42 -> 27 us (with one copy of the moments).
 // ONE: a structure of one mode.
 __host__ __device__ inline int epi_count(bool f64, int x, int y, int z, bool diag)
 {
@@ -967,8 +967,8 @@ __host__ __device__ inline long f64_tiles(long rows, int BR, int BC)
 // (BR multiplies per 4 BR BC MFMAs) and the epilogue.  Staged through LDS with two
 // barriers per chunk of 32 K rows it took 254 ms at 1000 nodes, 30 modes, 513
 // frequencies (61 TFLOP/s where bare MFMA reaches 76.9) and 2690 / 262 us at 333, 17,
-// 193 / 40, 20, 65; now 232.7 ms, of which the epilogue 24, and 2415 / 200 us, of which
-// 520 / 139.
+// 193 / 40, 20, 65; now 231.7 ms, of which the epilogue 24, and 2395 / 192 us, of which
+// 497 / 130.
 // The blocks near the origin and the resonances hold most of a moment, and with hundreds
 // of small additions after them the order alone costs ten roundings and more; waves that
 // add to one address wait for each other, too (some 40 ns each).  The workgroups of a mode
@@ -1055,9 +1055,9 @@ __device__ __forceinline__ void gsym_f64_wave(const GsymArgs &args, int x, long 
 
 // Two waves per SIMD (registers; LDS allows three).  The bound of 4 for the tiles up to
 // 2x2 makes the compiler keep the accumulators in AGPRs, without copies: with 2 it takes
-// 100 us where 4 takes 95 at 151 nodes, 9 modes, 101 frequencies, 68 / 66 at 60, 8, 129,
-// 33 / 28 at 300, 1, 193, and a call of the diagonal model 248 / 244 at 500, 20, 257.
-// A bound of 3 spills: 20 to 35 % slower.
+// 96 us where 4 takes 93 at 151 nodes, 9 modes, 101 frequencies, 67 / 64 at 60, 8, 129,
+// 32 / 27 at 300, 1, 193, and a call of the diagonal model 248 / 242 at 500, 20, 257.
+// A bound of 3 spills: 153, 105, 32 and 245.
 constexpr int f64_bound(int blocks) { return blocks > 4 ? 2 : 4; }
 
 template <int BR, int BC>
